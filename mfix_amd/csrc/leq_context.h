@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/mfix_leq.h"
+#include "leq_line.h"
 #include "leq_phases.h"
 
 namespace mfix {
@@ -47,7 +48,7 @@ constexpr int kSizeClasses = 12;  // 8K, 32K, ..., 4^11 * 8K cells
 constexpr int kMaxRPasses = 4;    // 'R' characters of a 4-character LINE sweep string
 
 // Launch shape of the streaming kernels: threads per block, cells per
-// thread, and threads (= lines) per block of the line-solve kernels.
+// thread, and lines per block of the line-solve kernels (0: by their own rule).
 struct Shape {
     int bs = 0, cpt = 0, lines_per_block = 0;
 };
@@ -56,30 +57,33 @@ int size_class(int64_t n3);
 void launch_resid_finish(const DGrid &g, int kind, int debug, double norm, double *partials, int64_t nblk,
                          mfix_leq_resid *d_out, hipStream_t s);
 int default_block_size(int64_t n3, bool fp32);
-int default_lines_per_block(int64_t n3);
 double mixed_delta(int64_t n3);
 
 using Sweep = std::array<char, 4>;
+// Batched red-black passes of a LINE sweep string, -1 when it needs the
+// one-by-one sweep (I/K wavefronts, A).
+int rb_passes(const Sweep &sw, bool do_k);
 
 // Block maps of one launch sequence over the systems `ids` of a table:
 // stream kernels (smap), finish kernels (fmap), reliable updates (umap,
-// update_blocks() entries per system), batched red-black line
-// phases (lmap[lines-per-block variant][pass]); LINE systems whose sweep string is not made of R/S
-// passes are swept one by one (line_seq).
+// update_blocks() entries per system), batched red-black line phases
+// (lmap[line kernel][pass]); LINE systems whose sweep string is not made of
+// R/S passes are swept one by one (line_seq).
 struct MapSet {
     std::vector<int> ids;
-    std::vector<int2> smap, fmap, umap, lmap[kLineLpbVariants][kMaxRPasses];
+    std::vector<int2> smap, fmap, umap, lmap[kLineKernels][kMaxRPasses];
     // FP32 tables: red-black passes of the several-lanes-per-line kernel,
     // one map per kernel variant (line length class) and pass
     std::vector<int2> pmap[kPcrVariants][kMaxRPasses];
     int nlpass = 0;
+    int whole_lds = 0;            // LDS bytes of a k_line_whole launch (the largest of its systems)
     std::vector<int> line_seq;
     double cells = 0.0;           // sum of N3 over ids (timing bytes)
     double k1_bytes = 0.0;        // algorithmic bytes of one first-stencil launch over all ids
     int n_line = 0, n_fused = 0;  // LINE systems / DIAG+NONE systems among ids
     DevBuf dev;
     int *d_ids = nullptr;
-    int2 *d_smap = nullptr, *d_fmap = nullptr, *d_umap = nullptr, *d_lmap[kLineLpbVariants][kMaxRPasses] = {};
+    int2 *d_smap = nullptr, *d_fmap = nullptr, *d_umap = nullptr, *d_lmap[kLineKernels][kMaxRPasses] = {};
     int2 *d_pmap[kPcrVariants][kMaxRPasses] = {};
     uint64_t version = 0;         // bumped whenever the device copy changes
 };

@@ -56,6 +56,7 @@ struct SolverState {
     int nonunit_diag;       // some unit-scaled A0 differs from -1 (DIAG must read the A0 plane)
     int k1_launches;        // launches of the first stencil pass that worked on this system (timing)
     int line_launches;      // colour-phase launches that worked on this system (timing)
+    int line_general;       // LINE: some line needs DGTSV itself (row interchange, zero pivot, range): k_line_factor
     double l2[4 * kFinishBlocks];  // level-2 sums of the finish launches
 };
 
@@ -546,14 +547,13 @@ __host__ __device__ inline bool color_line(int nu, int nv, int vw, int param, in
         const int u0 = (param + 1) & 1;
         const int cnt = (nu - u0 + 1) / 2;
         if (cnt <= 0) return false;
-        v = (int)(t / cnt);
+        v = (int)((uint32_t)t / (uint32_t)cnt);  // (fewer than 2^31 lines)
         if (v >= nv) return false;
-        u = u0 + 2 * (int)(t % cnt);
+        u = u0 + 2 * ((int)t - v * cnt);
         return true;
     }
-    const int64_t m = t / nu;
-    const int r = (int)(t - m * nu);
-    v = (int)(2 * m);
+    const int m = (int)((uint32_t)t / (uint32_t)nu), r = (int)t - m * nu;
+    v = 2 * m;
     const int u0 = (param + v) & 1;
     const int cnt0 = (nu - u0 + 1) / 2;
     if (r < cnt0) {

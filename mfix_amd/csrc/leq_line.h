@@ -1,0 +1,623 @@
+// Red-black J-line phases of the LINE preconditioner (LEQ_MSOLVE,
+// model/leqsol_mod.f:286-598; LEQ_IKSWEEP :851-921; DGTSV
+// model/DGTSV.f:107-246), whole lines in LDS.
+//
+// A block of 256 threads takes S.lpb lines of one colour and holds their
+// rows in LDS: all threads load them (consecutive lanes take consecutive rows
+// of a line, every load of a thread issued before its first use) and form the
+// right-hand side, one lane per line runs the tridiagonal solve in LDS, and
+// all threads store the solution.  One memory round trip and four barriers a
+// block; blocks of a CU overlap each other's loads and chains.
+//
+// What bounds a phase is the serial chain of a line where few blocks share a
+// CU, and where many do the time a line holds its LDS (chain, load and store)
+// against the bytes.  The chain is shortened by factoring once per solve: the
+// multipliers and the eliminated diagonal of DGTSV depend on A_M alone, which
+// does not change during a solve, so k_line_factor runs the elimination of
+// every line at set-up (DGTSV's operations in its order) and the phases read
+// its results in the places of DL and A0.  A phase's chain is then b_i -=
+// fact_i b_{i-1} forward (a product and a difference) and x_i = (b_i - u_i
+// x_{i+1})/d_i back, the division done with the refined reciprocal of d_i
+// (Newton-Raphson, then Markstein's quotient correction: q = n r, q += (n - q
+// d) r): five dependent operations where a division alone takes about ten.
+// Blocks with a row interchange carry it through both passes.  Every value is
+// the one DGTSV's own operations give, bit for bit (but for the sign of a
+// zero), as long as no operand leaves the range in which the correction is
+// exact; a system with a pivot outside it or zero (SolverState::line_general)
+// runs DGTSV itself in LDS, and so does a block whose solution holds a value
+// outside the range.
+//
+// Measured (events of the dispatches, LINE solve, colour phase; before, one
+// DGTSV lane per line over 16-row tiles with the finished rows in global
+// scratch): 64^3 28.4 -> 10.2 us, 128^3 56.2 -> 29.0 us, 158^3 70.9 -> 50.5
+// us, 256^3 409 -> 234 us.
+#pragma once
+#include "leq_phases.h"
+
+namespace mfix {
+
+constexpr int kWholeThreads = 256;
+// Rows a thread loads at most (their diagonals stay in its registers through
+// the forward pass); longer lines take k_line_color_sys.
+constexpr int kWholeElems = 6, kWholeRows = kWholeThreads * kWholeElems;
+// LDS of one block's lines: four blocks fit on a CU.
+constexpr int kWholeLdsTarget = 160 * 1024 / 4 - 2048;
+constexpr int kWholeLines = 64;  // one lane of the solving wave per line
+
+// A line holds whole_rows rows (its own and up to three identity rows, so that
+// the chains take four rows a step) and lines sit an odd number of 16-byte
+// units apart: the solving lanes (one line each, the same two rows) and the
+// loading lanes (one line, consecutive rows) both spread over the banks.
+__host__ __device__ constexpr int whole_rows(int n) { return (n + 3) & ~3; }
+__host__ __device__ constexpr int whole_stride(int n) { return whole_rows(n) + 2; }
+__host__ inline bool whole_fits(int n) { return n <= kWholeRows; }
+// Elements kept free before the first array and behind the last, for the
+// chains' reads past a line's ends.
+constexpr int kWholeFront = 16, kWholeTail = 16;
+// LDS elements of a block of lpb lines: four arrays.
+__host__ __device__ constexpr int whole_elems(int n, int lpb) {
+    return kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
+}
+
+// Lines per block for lines of n rows, `lines` of them in a colour: as many
+// as the LDS target and the rows per thread hold, but few enough that a colour
+// makes 512 blocks (two per CU; below that CUs idle while others run a second
+// block), at least one.  pin: mfix_leq_set_line_block's value, 0 = none.
+__host__ inline int whole_lpb(int n, int64_t lines, size_t elem, int pin) {
+    const int64_t rows = kWholeRows / n;
+    int64_t lpb = (kWholeLdsTarget / (int64_t)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    const int64_t spread = (lines + 511) / 512;
+    if (spread < lpb) lpb = spread;
+    if (pin > 0) lpb = pin;
+    if (lpb > rows) lpb = rows;
+    if (lpb > kWholeLines) lpb = kWholeLines;
+    return lpb < 1 ? 1 : (int)lpb;
+}
+
+// The ranges in which the corrected quotient is the correctly rounded one: no
+// intermediate of it is subnormal or overflows (the remainder's last place is
+// at least 2^-106 of the numerator, |x d| >= 2^-960).
+__device__ __forceinline__ bool factor_in_range(double d) {
+    const double m = fabs(d);
+    return m >= 0x1p-60 && m <= 0x1p60;  // (NaN: false)
+}
+__device__ __forceinline__ bool solution_in_range(double x) {
+    const double m = fabs(x);
+    return x == 0.0 || (m >= 0x1p-900 && m <= 0x1p900);
+}
+
+// 1/d to the last place but for ties: two Newton-Raphson steps on the
+// hardware's estimate.
+__device__ __forceinline__ double refined_rcp(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+// n/d from r = refined_rcp(d).
+__device__ __forceinline__ double corrected_quotient(double n, double d, double r) {
+    const double q = n * r;
+    return __builtin_fma(__builtin_fma(-q, d, n), r, q);
+}
+
+// Start cell and I/K neighbour offsets of the block's lines, constant along a
+// J-line (set_increments.f:72-112); the lines past the colour's last are
+// missing from the end.
+struct WholeLines {
+    uint32_t c0[kWholeLines], im[kWholeLines], ip[kWholeLines], km[kWholeLines], kp[kWholeLines];
+    int n;
+};
+__device__ __forceinline__ void whole_lines(const DGrid &g, int lpb, int64_t first, int param, WholeLines &w) {
+    const int l = threadIdx.x;
+    if (l < 64) {
+        int u = 0, v = 0;
+        const bool ok = l < lpb && color_line(g.ni, g.nk, g.do_k ? 1 : 0, param, first + l, u, v);
+        const uint32_t c1 = (uint32_t)g.c1, c2 = (uint32_t)g.c2;
+        if (ok) {
+            w.c0[l] = (uint32_t)u * c1 + (uint32_t)v * c2;
+            w.im[l] = (uint32_t)(nb_minus(u, g.ni, g.cyc_x) - u) * c1;
+            w.ip[l] = (uint32_t)(nb_plus(u, g.ni, g.cyc_x) - u) * c1;
+            w.km[l] = g.do_k ? (uint32_t)(nb_minus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
+            w.kp[l] = g.do_k ? (uint32_t)(nb_plus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
+        }
+        const uint64_t have = __ballot(ok);
+        if (l == 0) w.n = __popcll(have);
+    }
+    __syncthreads();
+}
+
+// A multiplier of an interchanged row is stored times 2^600: DGTSV's
+// multipliers are at most 1 in size, so the factor marks the row and comes off
+// exactly.
+constexpr double kSwapUp = 0x1p600, kSwapDown = 0x1p-600;
+__device__ __forceinline__ bool swapped(double f) { return fabs(f) > 2.0; }
+
+// DGTSV's elimination of every line of the listed FP64 systems, both colours
+// (blockIdx.y = colour), in cell order: the multipliers (row 0: 0) to S.lf and
+// the eliminated diagonal to S.ld, and, for a block of lines with a row
+// interchange, the eliminated first and second super-diagonals to S.lu and
+// S.lu2 (else they are A_M's upper coupling and 0).
+static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<double> *__restrict__ sys,
+                                                                      const int2 *__restrict__ map) {
+    extern __shared__ __align__(16) char whole_lds[];
+    __shared__ WholeLines w;
+    const int2 e = map[blockIdx.x];
+    if (e.x < 0) return;
+    const Sys<double> &S = sys[e.x];
+    auto *__restrict__ st = to_global(S.st);
+    if (st->done) return;
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n);
+    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, (int)blockIdx.y, w);
+    const int nl = w.n, tot = nl * n;
+    double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ D = F + S.lpb * ls,
+                         *__restrict__ U = D + S.lpb * ls, *__restrict__ V = U + S.lpb * ls;
+    const int64_t n3 = g.n3;
+    const gptr<const double> a = to_global(S.a);
+    for (int e0 = threadIdx.x; e0 < tot; e0 += 2 * kWholeThreads) {
+        double dl[2], d[2], du[2];
+        int o[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int x = e0 + k * kWholeThreads < tot ? e0 + k * kWholeThreads : e0;
+            const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n;
+            const uint32_t c = w.c0[l] + (uint32_t)q;
+            o[k] = l * ls + q;
+            dl[k] = q > 0 ? a[1 * n3 + c] : 0.0;
+            d[k] = a[3 * n3 + c];
+            du[k] = q < n - 1 ? a[5 * n3 + c] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            F[o[k]] = dl[k];
+            D[o[k]] = d[k];
+            U[o[k]] = du[k];
+        }
+    }
+    __syncthreads();
+    int any = 0;
+    if ((int)threadIdx.x < nl) {
+        const int o = threadIdx.x * ls;
+        double d = D[o], u = U[o];
+        bool ok = true;
+        double dl1 = F[o + 1], d1 = D[o + 1], u1 = U[o + 1];  // (a line has at least three rows)
+        for (int i = 0; i < n - 1; ++i) {
+            const int nx = i + 2 < n ? i + 2 : n - 1;  // the next row is read ahead of this one's division
+            const double dl2 = F[o + nx], d2 = D[o + nx], u2 = U[o + nx];
+            double fd = d, fu = u, fv = 0.0, f, dn, un = u1;
+            if (fabs(d) >= fabs(dl1)) {
+                f = dl1 / d;  // (DGTSV.f:111-122)
+                dn = d1 - f * u;
+            } else {
+                // interchange rows i and i+1 (DGTSV.f:123-136, :148-158)
+                const double fact = d / dl1;
+                fd = dl1;
+                fu = d1;
+                dn = u - fact * d1;
+                if (i < n - 2) {
+                    fv = u1;
+                    un = -fact * u1;
+                }
+                f = fact * kSwapUp;
+                ok = ok && swapped(f);
+                any = 1;
+            }
+            ok = ok && factor_in_range(fd);
+            F[o + i + 1] = f;
+            D[o + i] = fd;
+            U[o + i] = fu;
+            V[o + i] = fv;
+            d = dn;
+            u = un;
+            dl1 = dl2;
+            d1 = d2;
+            u1 = u2;
+        }
+        D[o + n - 1] = d;
+        U[o + n - 1] = 0.0;
+        V[o + n - 1] = 0.0;
+        ok = ok && factor_in_range(d);
+        if (!ok) atomicOr((int *)&st->line_general, 1);
+    }
+    any = __syncthreads_or(any);
+    const gptr<double> lf = to_global(S.lf), ld = to_global(S.ld), lu = to_global(S.lu), lu2 = to_global(S.lu2);
+    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+        const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
+        const uint32_t c = w.c0[l] + (uint32_t)q;
+        lf[c] = F[at];
+        ld[c] = D[at];
+        if (any) {
+            lu[c] = U[at];
+            lu2[c] = V[at];
+        }
+    }
+}
+
+// The two passes of one line on its factored rows, in the lane that solves it,
+// over whole_rows(n) rows.  A pass is bound by its LDS instructions (each
+// costs what all 64 lanes of it would, 10-25 cycles) more than by the
+// arithmetic (a dependent FP64 operation takes about five): two rows move per
+// instruction, read one register set ahead of the chain at fixed offsets from
+// running pointers, and the scheduler keeps the order written here.  The last
+// reads run past the line's end (forward) or before its first row (back),
+// inside the block's LDS, and are not used.  Measured alone: 35 and 61 cycles
+// a row.
+typedef double pair2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void whole_forward(const double *__restrict__ pf, double *__restrict__ pb, int rows) {
+    constexpr int R = 8;
+    struct Rows {
+        pair2 f[R / 2], b[R / 2];
+    } s0, s1;
+    auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            w.f[k] = *(const pair2 *)&pf[at + 2 * k];
+            w.b[k] = *(const pair2 *)&pb[at + 2 * k];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    double b = 0.0;  // (row 0's multiplier is 0)
+    auto run = [&](const Rows &w, int at, int cnt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < cnt / 2; ++k) {
+            pair2 o;
+            b = w.b[k].x - w.f[k].x * b;
+            o.x = b;
+            b = w.b[k].y - w.f[k].y * b;
+            o.y = b;
+            *(pair2 *)&pb[at + 2 * k] = o;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(s0, 0);
+    for (; rows >= 2 * R; rows -= 2 * R, pf += 2 * R, pb += 2 * R) {
+        get(s1, R);
+        run(s0, 0, R);
+        get(s0, 2 * R);
+        run(s1, R, R);
+    }
+    if (rows >= R) {
+        get(s1, R);
+        run(s0, 0, R);
+        if (rows > R) run(s1, R, R / 2);
+    } else if (rows > 0) {
+        run(s0, 0, R / 2);
+    }
+}
+
+__device__ __forceinline__ void whole_back(double *__restrict__ pb, const double *__restrict__ pu,
+                                           const double *__restrict__ pd, const double *__restrict__ pr, int rows) {
+    constexpr int R = 4;
+    struct Rows {
+        pair2 b[R / 2], u[R / 2], d[R / 2], r[R / 2];
+    } s0, s1;
+    pb += rows - 2;
+    pu += rows - 2;
+    pd += rows - 2;
+    pr += rows - 2;
+    double x = 0.0;  // (the last row's upper coupling is 0)
+    auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            w.b[k] = *(const pair2 *)&pb[-at - 2 * k];
+            w.u[k] = *(const pair2 *)&pu[-at - 2 * k];
+            w.d[k] = *(const pair2 *)&pd[-at - 2 * k];
+            w.r[k] = *(const pair2 *)&pr[-at - 2 * k];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto run = [&](const Rows &w, int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            pair2 o;
+            x = corrected_quotient(w.b[k].y - w.u[k].y * x, w.d[k].y, w.r[k].y);
+            o.y = x;
+            x = corrected_quotient(w.b[k].x - w.u[k].x * x, w.d[k].x, w.r[k].x);
+            o.x = x;
+            *(pair2 *)&pb[-at - 2 * k] = o;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(s0, 0);
+    for (; rows >= 2 * R; rows -= 2 * R, pb -= 2 * R, pu -= 2 * R, pd -= 2 * R, pr -= 2 * R) {
+        get(s1, R);
+        run(s0, 0);
+        get(s0, 2 * R);
+        run(s1, R);
+    }
+    if (rows > 0) run(s0, 0);
+}
+
+// The same two passes where some line of the block interchanges rows: the
+// right-hand sides trade places with them, and the second super-diagonal (in
+// V, the reciprocals' place: they are formed in the chain here) comes in.
+__device__ __forceinline__ void whole_forward_swap(const double *__restrict__ pf, double *__restrict__ pb, int n) {
+    constexpr int R = 4;
+    double f[R], r[R];
+    auto get = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int q = q0 + k < n ? q0 + k : n - 1;
+            f[k] = pf[q];
+            r[k] = pb[q];
+        }
+    };
+    double b = pb[0];
+    get(1);
+    for (int q0 = 1; q0 < n; q0 += R) {
+        double cf[R], cr[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            cf[k] = f[k];
+            cr[k] = r[k];
+        }
+        get(q0 + R);
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (q0 + k < n) {
+                const bool s = swapped(cf[k]);
+                const double fact = s ? cf[k] * kSwapDown : cf[k];
+                const double top = s ? cr[k] : b;  // row q-1's after the interchange
+                b = (s ? b : cr[k]) - fact * top;
+                pb[q0 + k - 1] = top;
+            }
+    }
+    pb[n - 1] = b;
+}
+
+__device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const double *__restrict__ pu,
+                                                const double *__restrict__ pv, const double *__restrict__ pd, int n) {
+    constexpr int R = 4;
+    double b[R], u[R], v[R], d[R];
+    auto get = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int q = q0 - k > 0 ? q0 - k : 0;
+            b[k] = pb[q];
+            u[k] = pu[q];
+            v[k] = pv[q];
+            d[k] = pd[q];
+        }
+    };
+    double x1 = 0.0, x2 = 0.0;
+    get(n - 1);
+    for (int q0 = n - 1; q0 >= 0; q0 -= R) {
+        double cb[R], cu[R], cv[R], cd[R], cr[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            cb[k] = b[k];
+            cu[k] = u[k];
+            cv[k] = v[k];
+            cd[k] = d[k];
+            cr[k] = refined_rcp(d[k]);
+        }
+        get(q0 - R);
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (q0 - k >= 0) {
+                const double x = corrected_quotient(cb[k] - cu[k] * x1 - cv[k] * x2, cd[k], cr[k]);
+                x2 = x1;
+                x1 = x;
+                pb[q0 - k] = x;
+            }
+    }
+}
+
+// DGTSV.f:107-163, :233-246 of one line in place: row i's diagonal, first and
+// second super-diagonal and right-hand side stay in slot i of D, U, F, B
+// (DL(i) was consumed one step before).  Returns INFO.
+template <typename T>
+__device__ __forceinline__ int whole_dgtsv(T *__restrict__ F, T *__restrict__ B, T *__restrict__ U,
+                                           T *__restrict__ D, int n) {
+    T d0 = D[0], u0 = U[0], b0 = B[0];
+    int info = 0;
+    for (int i = 0; i < n - 1; ++i) {
+        const T dl1 = F[i + 1], d1 = D[i + 1], u1 = U[i + 1], b1 = B[i + 1];
+        const bool keep = fabs((double)d0) >= fabs((double)dl1);  // no interchange
+        if (keep && d0 == (T)0 && !info) info = i + 1;
+        const T fact = (keep ? dl1 : d0) / (keep ? d0 : dl1);
+        const T pm = keep ? u0 : d1;  // row i's DU after the interchange
+        const T pb = keep ? b0 : b1;  // row i's B after the interchange
+        const bool sh = !keep && i < n - 2;
+        D[i] = keep ? d0 : dl1;
+        U[i] = pm;
+        F[i] = sh ? u1 : (T)0;
+        B[i] = pb;
+        d0 = (keep ? d1 : u0) - fact * pm;
+        u0 = sh ? -fact * u1 : u1;
+        b0 = (keep ? b1 : b0) - fact * pb;
+    }
+    if (!info && d0 == (T)0) info = n;  // DGTSV.f:160-163
+    T x1 = b0 / d0, x2 = (T)0;
+    B[n - 1] = x1;
+    for (int q = n - 2; q >= 0; --q) {  // (row n-2 has F = 0 and x2 = 0)
+        const T x = (B[q] - U[q] * x1 - F[q] * x2) / D[q];
+        x2 = x1;
+        x1 = x;
+        B[q] = x;
+    }
+    return info;
+}
+
+// Row inputs of one element of a colour phase: B minus the I/K neighbour terms
+// in LEQ_IKSWEEP's order (leqsol_mod.f:891-902), the coupling to the row
+// above, and two planes' values at the row (the multiplier and the eliminated
+// diagonal, or DL and A0).
+template <typename T>
+struct WholeArrays {
+    gptr<const T> im, ip, km, kp, jp, bm, f, d;
+    gptr<T> var;
+};
+template <typename T>
+struct WholeRow {
+    T b, im, ip, km, kp, vim, vip, vkm, vkp, f, d, u;
+    __device__ __forceinline__ void load(const WholeArrays<T> &A, const WholeLines &w, int l, uint32_t c) {
+        b = A.bm[c];
+        im = A.im[c];
+        ip = A.ip[c];
+        vim = A.var[c + w.im[l]];
+        vip = A.var[c + w.ip[l]];
+        km = A.km[c];  // (in 2-D the K offsets are 0: in bounds, not used)
+        kp = A.kp[c];
+        vkm = A.var[c + w.km[l]];
+        vkp = A.var[c + w.kp[l]];
+        f = A.f[c];
+        d = A.d[c];
+        u = A.jp[c];
+    }
+    __device__ __forceinline__ T rhs(int do_k) const {
+        const T two = b - im * vim - ip * vip;
+        return do_k ? two - km * vkm - kp * vkp : two;
+    }
+};
+
+// One colour phase: block e takes lines [e.y*S.lpb, +S.lpb) of colour
+// `param` (color_line).  which = 0 preconditions P into Phat, 1 S into Shat.
+// FP32 tables (lines longer than the k_line_pcr_sys variants hold) always run
+// DGTSV in LDS.
+template <typename T>
+__global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *__restrict__ sys,
+                                                              const int2 *__restrict__ map, int param, int which) {
+    extern __shared__ __align__(16) char whole_lds[];
+    __shared__ WholeLines w;
+    __shared__ int linfo[kWholeLines];  // DGTSV INFO per line
+    const int2 e = map[blockIdx.x];
+    if (e.x < 0) return;
+    const Sys<T> &S = sys[e.x];
+    auto *__restrict__ st = to_global(S.st);
+    if (st->done || (which == 1 && st->s_exit)) return;
+    if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n), do_k = g.do_k;
+    const int rows = whole_rows(n);
+    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, param, w);
+    const int nl = w.n, tot = nl * n;
+    // right-hand side (then the solution), upper coupling, and: multipliers
+    // (then the eliminated diagonal) and its reciprocals, or DL (then the
+    // second super-diagonal) and A0
+    T *__restrict__ F = (T *)whole_lds + kWholeFront, *__restrict__ B = F + S.lpb * ls, *__restrict__ U = B + S.lpb * ls,
+                    *__restrict__ D = U + S.lpb * ls;
+    const int64_t n3 = g.n3;
+    const gptr<const T> a = to_global(S.a);
+    WholeArrays<T> A;
+    A.km = a;
+    A.im = a + 2 * n3;
+    A.ip = a + 4 * n3;
+    A.jp = a + 5 * n3;
+    A.kp = a + 6 * n3;
+    A.bm = to_global((const T *)(which == 0 ? S.p : S.s));
+    A.var = to_global(which == 0 ? S.phat : S.shat);
+    // (a line's rows are consecutive elements: element x is row x % n of line x / n)
+    auto line_of = [&](int x) { return (int)div_by((uint32_t)x, g.mnj, g.snj); };
+    if constexpr (sizeof(T) == sizeof(double)) {
+        if (!st->line_general) {
+            A.f = to_global((const T *)S.lf);
+            A.d = to_global((const T *)S.ld);
+            constexpr int K = 3;  // rows in flight per thread
+            T td[kWholeElems];    // the diagonals wait for the multipliers' place
+            int o[kWholeElems], any = 0;
+#pragma unroll
+            for (int k0 = 0; k0 < kWholeElems; k0 += K) {
+                if (k0 * kWholeThreads >= tot) break;
+                WholeRow<T> r[K];
+                bool last[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
+                    const int x = x0 < tot ? x0 : tot - 1;  // (past the end: the last row again)
+                    const int l = line_of(x), q = x - l * n;
+                    o[k0 + k] = l * ls + q;
+                    r[k].load(A, w, l, w.c0[l] + (uint32_t)q);
+                    last[k] = q == n - 1;
+                }
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    F[o[k0 + k]] = r[k].f;  // (0 on the first row)
+                    any |= swapped(r[k].f);
+                    B[o[k0 + k]] = r[k].rhs(do_k);
+                    U[o[k0 + k]] = last[k] ? (T)0 : r[k].u;
+                    D[o[k0 + k]] = (T)refined_rcp(r[k].d);
+                    td[k0 + k] = r[k].d;
+                }
+            }
+            for (int x = threadIdx.x; x < 4 * nl; x += kWholeThreads) {
+                const int q = n + (x & 3), at = (x >> 2) * ls + q;
+                if (q < rows) {  // identity rows
+                    F[at] = B[at] = U[at] = 0.0;
+                    D[at] = 1.0;
+                }
+            }
+            const bool swaps = __syncthreads_or(any);
+            if (swaps) {
+                const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
+                for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+                    const int l = line_of(x), q = x - l * n;
+                    const uint32_t c = w.c0[l] + (uint32_t)q;
+                    U[l * ls + q] = lu[c];
+                    D[l * ls + q] = lu2[c];
+                }
+            }
+            // the solving wave: another one in each of the blocks that share a
+            // CU (every 256th), so that they do not share a SIMD
+            const int solver = (int)threadIdx.x - 64 * ((blockIdx.x >> 8) & 3);
+            const bool mine = solver >= 0 && solver < nl;
+            const int ol = solver * ls;
+            if (mine) {
+                if (swaps) whole_forward_swap(F + ol, B + ol, n);
+                else whole_forward(F + ol, B + ol, rows);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < kWholeElems; ++k)
+                if (k / K * K * kWholeThreads < tot) F[o[k]] = td[k];
+            for (int x = threadIdx.x; x < 4 * nl; x += kWholeThreads) {
+                const int q = n + (x & 3);
+                if (q < rows) F[(x >> 2) * ls + q] = 1.0;
+            }
+            __syncthreads();
+            if (mine) {
+                if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, n);
+                else whole_back(B + ol, U + ol, F + ol, D + ol, rows);
+            }
+            __syncthreads();
+            int bad = 0;
+            for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+                const int l = line_of(x);
+                bad |= !solution_in_range((double)B[l * ls + (x - l * n)]);
+            }
+            if (!__syncthreads_or(bad)) {
+                for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+                    const int l = line_of(x), q = x - l * n;
+                    A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+                }
+                return;
+            }
+        }
+    }
+    // DGTSV itself
+    A.f = a + n3;
+    A.d = a + (int64_t)DiagPlane<T>::value * n3;
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+        const int l = line_of(x), q = x - l * n, at = l * ls + q;
+        WholeRow<T> r;
+        r.load(A, w, l, w.c0[l] + (uint32_t)q);
+        F[at] = q > 0 ? r.f : (T)0;
+        B[at] = r.rhs(do_k);
+        U[at] = q < n - 1 ? r.u : (T)0;
+        D[at] = r.d;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) {
+        const int ol = threadIdx.x * ls;
+        linfo[threadIdx.x] = whole_dgtsv(F + ol, B + ol, U + ol, D + ol, n);
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+        const int l = line_of(x), q = x - l * n;
+        // a line whose elimination hit a zero pivot keeps its values (leqsol_mod.f:910-914)
+        if (!linfo[l]) A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+    }
+}
+
+}  // namespace mfix

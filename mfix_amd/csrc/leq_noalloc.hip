@@ -48,7 +48,7 @@ size_t map_bytes(const DGrid &g, const Part &P) {
     b += up256(e * kFinishBlocks);                                   // fmap
     b += up256(e * (size_t)update_blocks(P.nblk));                   // umap
     b += kMaxRPasses * up256(e * (size_t)((lines + 15) / 16 + kNumXcd));  // lmap of the variant in use
-    b += (kLineLpbVariants - 1) * kMaxRPasses * 256;                 // the other variants' empty maps
+    b += 2 * kMaxRPasses * 256;                                      // room kept for the other kernels' maps
     b += kPcrVariants * kMaxRPasses * 256;                           // empty FP32 maps
     return b;
 }
@@ -89,9 +89,19 @@ static int solve_fp64_noalloc(char *base, const SysDesc &d, const Shape &sh, mfi
     G.bs = sh.bs;
     G.mixed = false;
     sys_carve<double>(G.sys[0], d, P, base + o_ws);
+    // the red-black kernels use n3 elements of each of the four scratch
+    // planes; their block maps (one entry per few lines) go behind those, the
+    // others' stay in the map region
+    char *map = base + o_map;
+    size_t map_cap = maps;
+    if (d.pc == PC_LINE && rb_passes(d.sweep, d.g.do_k != 0) >= 0 && whole_fits(d.g.nj)) {
+        const size_t used = up256(4 * (size_t)d.g.n3 * sizeof(double));
+        map = (char *)G.sys[0].line_scratch + used;
+        map_cap = (size_t)line_scratch_elems(d.g) * sizeof(double) - used;
+    }
     int rc;
     if ((rc = upload_table<double>(G, s, base + o_tab, up256(sizeof(Sys<double>))))) return rc;
-    if ((rc = build_maps<double>(G, std::vector<int>{0}, G.iter, s, base + o_map, maps))) return rc;
+    if ((rc = build_maps<double>(G, std::vector<int>{0}, G.iter, s, map, map_cap))) return rc;
     enqueue_setup<double>(G, G.iter, s);
     rc = run_group<double>(G, d.itmax, s, false, (int *)(base + o_cnt));
     SolverState *h = C.host_state;

@@ -35,6 +35,13 @@ inline void launch_timed(hipEvent_t e0, hipEvent_t e1, void (*kernel)(Args...), 
     if (e0) hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, static_cast<Args>(args)...);
     else hipLaunchKernelGGL(kernel, grid, block, 0, s, static_cast<Args>(args)...);
 }
+// The same with dynamic LDS.
+template <typename... Args, typename... P>
+inline void launch_timed_lds(hipEvent_t e0, hipEvent_t e1, void (*kernel)(Args...), dim3 grid, dim3 block, int lds,
+                             hipStream_t s, P... args) {
+    if (e0) hipExtLaunchKernelGGL(kernel, grid, block, lds, s, e0, e1, 0, static_cast<Args>(args)...);
+    else hipLaunchKernelGGL(kernel, grid, block, lds, s, static_cast<Args>(args)...);
+}
 
 // Work the set-up pass does on a row before it scales it
 // (mfix_leq_resid_relax_bicgs_dev): the CALC_RESID row of the equation as
@@ -67,6 +74,8 @@ struct Sys {
     T *x, *r, *rt, *p, *s, *t, *v, *phat, *shat;  // x: VAR (FP64 solve only)
     double *y;             // mixed: FP64 correction accumulator since the last reliable update
     T *line_scratch;       // 4 planes of DGTSV scratch (LINE)
+    T *lf, *ld, *lu, *lu2; // LINE, FP64: every line's elimination (k_line_factor), the four planes of line_scratch
+    int lpb;               // LINE: lines per block of k_line_whole
     SolverState *st;
     double *partials;      // kMaxPartials * P.nblk
     double *a64, *b64, *xa, *xb, *r64;
@@ -791,7 +800,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_finish_sys(const Sys<T> *__res
 template <typename T, int LPB>
 __global__ void __launch_bounds__(320) k_line_color_sys(const Sys<T> *__restrict__ sys, const int2 *__restrict__ map,
                                                         int param, int which) {
-    static_assert(LPB == 64 || LPB == 32 || LPB == 16, "lines per block");
+    static_assert(LPB == 64, "lines per block");
     constexpr int RL = 1024 / LPB; // rows per run a loader instruction reads of each line
     constexpr int LPI = 64 / RL;   // lines per load instruction
     constexpr int K = 4;           // tile elements per loader lane
@@ -1069,11 +1078,12 @@ __global__ void __launch_bounds__(320) k_line_color_sys(const Sys<T> *__restrict
 
 constexpr int kLineBlock = 320;  // threads of k_line_color_sys: one solving wave, four loaders
 
-// Lines-per-block variants of k_line_color_sys (a launch shape picks one per
-// grid size).
-constexpr int kLineLpbVariants = 3;
-__host__ __device__ constexpr int line_lpb_of(int var) { return var == 0 ? 64 : var == 1 ? 32 : 16; }
-__host__ __device__ inline int line_lpb_variant(int lpb) { return lpb >= 64 ? 0 : lpb >= 32 ? 1 : 2; }
+constexpr int kLongLpb = 64;     // its lines per block
+
+// Red-black line kernels with one lane per line: k_line_whole (whole lines in
+// LDS) and, for lines that do not fit there, k_line_color_sys.
+enum LineKernel : int { LINE_WHOLE = 0, LINE_LONG = 1 };
+constexpr int kLineKernels = 2;
 
 // Red-black line phase along J for the FP32 inner solve of the mixed path:
 // several lanes per line.  The FP64 kernel above must repeat DGTSV's

@@ -180,7 +180,6 @@ Shape Context::shape_for(int64_t n3, bool fp32) const {
     const int cls = size_class(n3);
     Shape s = tuned[fp32 ? 1 : 0][cls];
     if (!s.bs) s = Shape{default_block_size(n3, fp32), 1, 0};
-    if (!s.lines_per_block) s.lines_per_block = default_lines_per_block(n3);
     return s;
 }
 
@@ -191,14 +190,6 @@ Shape Context::shape_for(int64_t n3, bool fp32) const {
 // 1024-cell blocks sums 33.5K / 16.8K partials in two levels; the single-block
 // finish over 16.8K partials ran 474.6-474.9).
 int default_block_size(int64_t n3, bool fp32) { return fp32 && n3 > (int64_t(1) << 23) ? 512 : 256; }
-
-// Lines per block of the red-black line kernel when none was tuned: 64.
-// A colour phase is bound by the chain of dependent memory round trips of
-// one line (tile loads forward, scratch reads back), which fewer lines per
-// block do not shorten: measured at 128^3 (8,450 lines per colour) 73 / 120 /
-// 168 us per phase at 64 / 32 / 16 lines per block, although 64 leaves half
-// the CUs idle; at 256^3 476 / 575 / 937 us.
-int default_lines_per_block(int64_t) { return 64; }
 
 // Reliable-update trigger of mixed solves that set none (opts->inner_tol):
 // the recursive FP32 residual fell by 1e-4 since the last FP64 update on
@@ -347,21 +338,39 @@ int launch_msolve_line(const DGrid &g, const Shape &sh, const char *cmethod, con
 // R passes or characters that do nothing here (S; J; K and A in 2-D),
 // through the red-black kernels the solver uses: z = r (SETGUESS,
 // :341-357), then per R pass the (i+k)-odd colour and the even one.  FP64:
-// k_line_color_sys (DGTSV per line, the reference's bits); FP32 (A in the
-// inner solve's difference layout, A0 in plane 7): k_line_pcr_sys where the
-// line fits one of its variants.  A one-system table carries the arrays; its
-// state is blank, so the kernels never return early.  Returns 1, launching
-// nothing, for a sweep string with I/K/A passes (the caller runs
-// k_line_phase instead).
+// k_line_whole after k_line_factor, or k_line_color_sys for long lines (DGTSV
+// per line, the reference's bits); FP32 (A in the inner solve's difference
+// layout, A0 in plane 7): k_line_pcr_sys where the line fits one of its
+// variants.  A one-system table carries the arrays; its state is blank, so
+// the kernels never return early.  Returns 1, launching nothing, for a sweep
+// string with I/K/A passes (the caller runs k_line_phase instead).
 template <typename T>
-static void launch_line_color(int lv, dim3 gs, hipStream_t s, const Sys<T> *tab, const int2 *mp, int param,
-                              int which, std::pair<hipEvent_t, hipEvent_t> ev = {nullptr, nullptr}) {
-    const dim3 lb(kLineBlock);
-    switch (lv) {
-    case 0: launch_timed(ev.first, ev.second, k_line_color_sys<T, 64>, gs, lb, s, tab, mp, param, which); break;
-    case 1: launch_timed(ev.first, ev.second, k_line_color_sys<T, 32>, gs, lb, s, tab, mp, param, which); break;
-    default: launch_timed(ev.first, ev.second, k_line_color_sys<T, 16>, gs, lb, s, tab, mp, param, which); break;
-    }
+static void launch_line_color(int kernel, dim3 gs, int lds, hipStream_t s, const Sys<T> *tab, const int2 *mp,
+                              int param, int which, std::pair<hipEvent_t, hipEvent_t> ev = {nullptr, nullptr}) {
+    if (kernel == LINE_WHOLE)
+        launch_timed_lds(ev.first, ev.second, k_line_whole<T>, gs, dim3(kWholeThreads), lds, s, tab, mp, param, which);
+    else
+        launch_timed(ev.first, ev.second, k_line_color_sys<T, kLongLpb>, gs, dim3(kLineBlock), s, tab, mp, param,
+                     which);
+}
+static void launch_line_factor(dim3 gs, int lds, hipStream_t s, const Sys<double> *tab, const int2 *mp) {
+    hipLaunchKernelGGL(k_line_factor, dim3(gs.x, 2), dim3(kWholeThreads), lds, s, tab, mp);
+}
+
+// The one-lane-per-line kernel for lines of n rows, its lines per block and
+// the blocks a colour takes.
+static int line_kernel(int n) { return whole_fits(n) ? LINE_WHOLE : LINE_LONG; }
+static int64_t colour_lines(const LineGeom &L) { return ((int64_t)L.nu * L.nv + 1) / 2; }
+template <typename T>
+static int lines_of_block(const DGrid &g) {
+    const LineGeom L = line_geom(g, AX_J);
+    if (line_kernel(L.n) == LINE_LONG) return kLongLpb;
+    return whole_lpb(L.n, colour_lines(L), sizeof(T),
+                     ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block);
+}
+template <typename T>
+static int whole_lds_bytes(const Sys<T> &S) {
+    return (int)sizeof(T) * whole_elems(S.g.nj, S.lpb);
 }
 
 template <typename T>
@@ -378,11 +387,10 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     }
     Context &C = ctx();
     const LineGeom L = line_geom(g, AX_J);
-    const int64_t lines = ((int64_t)L.nu * L.nv + 1) / 2;
     const int var = sizeof(T) == sizeof(float) ? line_pcr_variant(L.n) : -1;
-    const int lv = line_lpb_variant(C.shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block);
-    const int lpb = var >= 0 ? line_pcr_lpb(var) : line_lpb_of(lv);
-    const int64_t lb = (lines + lpb - 1) / lpb;
+    const int lk = line_kernel(L.n);
+    const int lpb = var >= 0 ? line_pcr_lpb(var) : lines_of_block<T>(g);
+    const int64_t lb = (colour_lines(L) + lpb - 1) / lpb;
     const size_t o_st = align256(sizeof(Sys<T>));
     const size_t o_map = o_st + align256(sizeof(SolverState));
     int rc;
@@ -395,6 +403,11 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     S.p = const_cast<T *>(r);
     S.phat = z;
     S.line_scratch = scratch;
+    S.lf = scratch;
+    S.ld = scratch + g.n3;
+    S.lu = scratch + 2 * g.n3;
+    S.lu2 = scratch + 3 * g.n3;
+    S.lpb = lpb;
     S.st = (SolverState *)(base + o_st);
     std::vector<int2> map;
     push_slab_map(map, 0, lb);
@@ -407,15 +420,17 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     const Sys<T> *tab = (const Sys<T> *)base;
     const int2 *mp = (const int2 *)(base + o_map);
     const dim3 gs((unsigned)map.size());
+    if constexpr (sizeof(T) == sizeof(double))
+        if (np > 0 && lk == LINE_WHOLE) launch_line_factor(gs, whole_lds_bytes(S), s, tab, mp);
     for (int q = 0; q < np; ++q)
         for (int param : {1, 0}) {
             const auto ev = pf.take(0.5 * (double)g.n3 * 13.0 * sizeof(T));
             if constexpr (sizeof(T) == sizeof(float)) {
                 const Sys<float> *tf = (const Sys<float> *)tab;
                 if (var >= 0) launch_line_pcr(var, gs, s, tf, mp, param, 0, ev.first, ev.second);
-                else launch_line_color<float>(lv, gs, s, tf, mp, param, 0, ev);
+                else launch_line_color<float>(lk, gs, whole_lds_bytes(S), s, tf, mp, param, 0, ev);
             } else {
-                launch_line_color<T>(lv, gs, s, tab, mp, param, 0, ev);
+                launch_line_color<T>(lk, gs, whole_lds_bytes(S), s, tab, mp, param, 0, ev);
             }
         }
     // the table must outlive the launches before it is rewritten
@@ -500,7 +515,13 @@ void sys_carve(Sys<T> &S, const SysDesc &d, const Part &P, char *base) {
     if (d.pc == PC_LINE) {
         S.phat = (T *)take(n3 * sizeof(T));
         S.shat = (T *)take(n3 * sizeof(T));
+        // (line_scratch_elems is more than 4 n3: the factored lines take four planes)
         S.line_scratch = (T *)take((size_t)line_scratch_elems(d.g) * sizeof(T));
+        S.lf = S.line_scratch;
+        S.ld = S.line_scratch + n3;
+        S.lu = S.line_scratch + 2 * n3;
+        S.lu2 = S.line_scratch + 3 * n3;
+        S.lpb = lines_of_block<T>(d.g);
     }
     if (mixed) {
         S.a = (const T *)take(8 * n3 * sizeof(float));
@@ -528,7 +549,7 @@ template void sys_carve<float>(Sys<float> &, const SysDesc &, const Part &, char
 // character is R (a pass) or a character that does nothing in this
 // dimension (S, and J; K and A too in 2-D).  Returns the number of passes,
 // or -1 when the system needs the one-by-one sweep (I/K wavefronts, A).
-static int rb_passes(const Sweep &sw, bool do_k) {
+int rb_passes(const Sweep &sw, bool do_k) {
     int n = 0;
     for (char ch : sw) {
         if (ch == 'R' || ch == 'r') ++n;
@@ -540,9 +561,9 @@ static int rb_passes(const Sweep &sw, bool do_k) {
 
 template <typename T>
 int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStream_t s, char *ext, size_t ext_cap) {
-    std::vector<int2> smap, fmap, umap, lmap[kLineLpbVariants][kMaxRPasses], pmap[kPcrVariants][kMaxRPasses];
+    std::vector<int2> smap, fmap, umap, lmap[kLineKernels][kMaxRPasses], pmap[kPcrVariants][kMaxRPasses];
     std::vector<int> seq;
-    int nlpass = 0, n_line = 0, n_fused = 0;
+    int nlpass = 0, n_line = 0, n_fused = 0, lds = 0;
     double cells = 0.0, k1 = 0.0;
     const double sa = sizeof(T), sv = sizeof(T);
     for (int id : ids) {
@@ -567,33 +588,33 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
                 seq.push_back(id);
             } else {
                 const LineGeom L = line_geom(S.g, AX_J);
-                const int64_t lines = ((int64_t)L.nu * L.nv + 1) / 2;
                 // FP32 (the mixed path's inner solve): several lanes per line
                 // where the line fits a variant; FP64: DGTSV lane per line
                 const int var = sizeof(T) == sizeof(float) ? line_pcr_variant(L.n) : -1;
-                const int lv = line_lpb_variant(ctx().shape_for(S.g.n3, sizeof(T) == sizeof(float)).lines_per_block);
-                const int lpb = var >= 0 ? line_pcr_lpb(var) : line_lpb_of(lv);
-                const int64_t lb = (lines + lpb - 1) / lpb;
+                const int lk = line_kernel(L.n);
+                const int lpb = var >= 0 ? line_pcr_lpb(var) : S.lpb;
+                const int64_t lb = (colour_lines(L) + lpb - 1) / lpb;
+                if (var < 0 && lk == LINE_WHOLE) lds = std::max(lds, whole_lds_bytes(S));
                 // the same XCD slab order as the stream kernels: XCD x takes a
                 // contiguous run of line blocks, so the I/K neighbour lines its
                 // blocks read (the other colour's, about two blocks away along
                 // K) come through one L2
                 for (int q = 0; q < np; ++q) {
                     if (var >= 0) push_slab_map(pmap[var][q], id, lb);
-                    else push_slab_map(lmap[lv][q], id, lb);
+                    else push_slab_map(lmap[lk][q], id, lb);
                 }
                 nlpass = std::max(nlpass, np);
             }
         }
     }
     bool same = M.ids == ids && M.smap.size() == smap.size() && M.fmap.size() == fmap.size() &&
-                M.nlpass == nlpass && M.line_seq == seq && M.dev.ptr;
+                M.nlpass == nlpass && M.whole_lds == lds && M.line_seq == seq && M.dev.ptr;
     if (same) same = !std::memcmp(M.smap.data(), smap.data(), smap.size() * sizeof(int2)) &&
                      !std::memcmp(M.fmap.data(), fmap.data(), fmap.size() * sizeof(int2)) &&
                      M.umap.size() == umap.size() &&
                      !std::memcmp(M.umap.data(), umap.data(), umap.size() * sizeof(int2));
     for (int q = 0; q < kMaxRPasses && same; ++q) {
-        for (int v = 0; v < kLineLpbVariants && same; ++v)
+        for (int v = 0; v < kLineKernels && same; ++v)
             same = M.lmap[v][q].size() == lmap[v][q].size() &&
                    !std::memcmp(M.lmap[v][q].data(), lmap[v][q].data(), lmap[v][q].size() * sizeof(int2));
         for (int v = 0; v < kPcrVariants && same; ++v)
@@ -610,12 +631,13 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
     M.fmap.swap(fmap);
     M.umap.swap(umap);
     for (int q = 0; q < kMaxRPasses; ++q) {
-        for (int v = 0; v < kLineLpbVariants; ++v) M.lmap[v][q].swap(lmap[v][q]);
+        for (int v = 0; v < kLineKernels; ++v) M.lmap[v][q].swap(lmap[v][q]);
         for (int v = 0; v < kPcrVariants; ++v) M.pmap[v][q].swap(pmap[v][q]);
     }
     M.nlpass = nlpass;
+    M.whole_lds = lds;
     M.line_seq.swap(seq);
-    // one device block: ids | smap | fmap | umap | lmap[variant][pass] | pmap[variant][pass]
+    // one device block: ids | smap | fmap | umap | lmap[kernel][pass] | pmap[variant][pass]
     std::vector<char> blob;
     auto put = [&](const void *p, size_t bytes) {
         const size_t off = blob.size();
@@ -627,8 +649,8 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
     const size_t o_s = put(M.smap.data(), M.smap.size() * sizeof(int2));
     const size_t o_f = put(M.fmap.data(), M.fmap.size() * sizeof(int2));
     const size_t o_u = put(M.umap.data(), M.umap.size() * sizeof(int2));
-    size_t o_l[kLineLpbVariants][kMaxRPasses], o_p[kPcrVariants][kMaxRPasses];
-    for (int v = 0; v < kLineLpbVariants; ++v)
+    size_t o_l[kLineKernels][kMaxRPasses], o_p[kPcrVariants][kMaxRPasses];
+    for (int v = 0; v < kLineKernels; ++v)
         for (int q = 0; q < kMaxRPasses; ++q) o_l[v][q] = put(M.lmap[v][q].data(), M.lmap[v][q].size() * sizeof(int2));
     for (int v = 0; v < kPcrVariants; ++v)
         for (int q = 0; q < kMaxRPasses; ++q) o_p[v][q] = put(M.pmap[v][q].data(), M.pmap[v][q].size() * sizeof(int2));
@@ -647,7 +669,7 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
     M.d_smap = (int2 *)(base + o_s);
     M.d_fmap = (int2 *)(base + o_f);
     M.d_umap = (int2 *)(base + o_u);
-    for (int v = 0; v < kLineLpbVariants; ++v)
+    for (int v = 0; v < kLineKernels; ++v)
         for (int q = 0; q < kMaxRPasses; ++q) M.d_lmap[v][q] = (int2 *)(base + o_l[v][q]);
     for (int v = 0; v < kPcrVariants; ++v)
         for (int q = 0; q < kMaxRPasses; ++q) M.d_pmap[v][q] = (int2 *)(base + o_p[v][q]);
@@ -698,6 +720,10 @@ static void setup_bs(Group<T> &G, const MapSet &M, hipStream_t s) {
     if (G.mixed) hipLaunchKernelGGL((k_prepare_a32<BS>), gs, blk, 0, s, (const Sys<float> *)G.d_sys, M.d_smap);
     hipLaunchKernelGGL((k_shadow<BS, T>), gs, blk, 0, s, G.d_sys, M.d_smap);
     finish<T, FIN_SHADOW, 1>(G, M, s);
+    if constexpr (sizeof(T) == sizeof(double))
+        if (!M.lmap[LINE_WHOLE][0].empty())
+            launch_line_factor(dim3((unsigned)M.lmap[LINE_WHOLE][0].size()), M.whole_lds, s, G.d_sys,
+                               M.d_lmap[LINE_WHOLE][0]);
 }
 
 template <typename T>
@@ -718,11 +744,11 @@ static void line_sweeps(const Group<T> &G, const MapSet &M, int which, hipStream
         for (int param : {1, 0}) {
             // one timed launch per colour and kernel family; the bytes are
             // those of every LINE system of the table (a single solve: its own)
-            for (int v = 0; v < kLineLpbVariants; ++v) {
+            for (int v = 0; v < kLineKernels; ++v) {
                 if (M.lmap[v][q].empty()) continue;
                 const auto ev = pf.take(0.5 * M.cells * 13.0 * sizeof(T));
-                launch_line_color<T>(v, dim3((unsigned)M.lmap[v][q].size()), s, G.d_sys, M.d_lmap[v][q], param, which,
-                                     ev);
+                launch_line_color<T>(v, dim3((unsigned)M.lmap[v][q].size()), M.whole_lds, s, G.d_sys, M.d_lmap[v][q],
+                                     param, which, ev);
             }
             if constexpr (sizeof(T) == sizeof(float)) {
                 const Sys<float> *tab = (const Sys<float> *)G.d_sys;
@@ -807,17 +833,17 @@ static void enqueue_count(const Group<T> &G, const MapSet &M, int *d_out, int *d
 }
 
 // Line-kernel launch of a LINE system: 1 + its variant index among the
-// red-black kernels (the FP32 several-lanes-per-line variants, or the FP64
-// lines-per-block variants), 0 for other systems and one-by-one sweeps.
+// red-black kernels (LineKernel, then the FP32 several-lanes-per-line
+// variants), 0 for other systems and one-by-one sweeps.
 template <typename T>
 static int line_launch_of(const Group<T> &G, int id) {
     const Sys<T> &S = G.sys[id];
     if (S.pc != PC_LINE || rb_passes(G.sweep[id], S.g.do_k != 0) < 0) return 0;
     if (sizeof(T) == sizeof(float)) {
         const int var = line_pcr_variant(line_geom(S.g, AX_J).n);
-        if (var >= 0) return 1 + kLineLpbVariants + var;
+        if (var >= 0) return 1 + kLineKernels + var;
     }
-    return 1 + line_lpb_variant(ctx().shape_for(S.g.n3, sizeof(T) == sizeof(float)).lines_per_block);
+    return 1 + line_kernel(S.g.nj);
 }
 
 // Drop finished systems from a table's block maps once the running systems
@@ -836,7 +862,7 @@ static int compact(Group<T> &G, const int *d_flags, int running, hipStream_t s) 
     if (e != hipSuccess) return hip_fail(e, "running flags");
     std::vector<int> keep;
     double cells = 0.0;
-    constexpr int kLaunches = 1 + kLineLpbVariants + kPcrVariants;
+    constexpr int kLaunches = 1 + kLineKernels + kPcrVariants;
     bool mapped[kLaunches] = {}, running_in[kLaunches] = {};
     for (size_t q = 0; q < flags.size(); ++q) {
         const int l = line_launch_of(G, M.ids[q]);
@@ -1412,9 +1438,8 @@ int autotune(int imax, int jmax, int kmax, int mixed, Shape *best_out) {
     const int bss[] = {db0, db0 == 256 ? 512 : 256, 1024};
     const int bi = pick(PC_DIAG, dp, dbp, 3, [&](int c) { slot = Shape{bss[c], 1, 0}; });
     Shape best = Shape{bss[bi], 1, 0};
-    // lines per block of the red-black line kernel: the size default first
-    const int d = default_lines_per_block(n3);
-    const int lpbs[] = {d, d == 64 ? 32 : 64, d == 16 ? 32 : 16};
+    // lines per block of the red-black line kernel: its own rule first
+    const int lpbs[] = {0, 32, 16};
     if (!rc) {
         const int li = pick(PC_LINE, dm, dbm, 3, [&](int c) { slot = Shape{best.bs, 1, lpbs[c]}; });
         best.lines_per_block = lpbs[li];
@@ -1422,7 +1447,10 @@ int autotune(int imax, int jmax, int kmax, int mixed, Shape *best_out) {
     slot = rc ? saved : best;
     for (double *q : {da, db, dx, dp, dm, dbp, dbm}) (void)hipFree(q);
     if (rc) return rc;
-    if (best_out) *best_out = best;
+    if (best_out) {
+        *best_out = best;
+        if (!best.lines_per_block) best_out->lines_per_block = lines_of_block<double>(g);
+    }
     return 0;
 }
 
