@@ -122,7 +122,7 @@ int mfix_leq_bicgs_dev(const char *cmethod, double tol, const char *pc,
 /* mfix_leq_bicgs_dev without any allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under
  * stream capture, tight serving loops, harnesses that forbid it).  The
- * workspace, system table, block maps and poll words live in a fixed
+ * workspace, system table and block maps live in a fixed
  * device array of MFIX_LEQ_NOALLOC_BYTES per GPU (held until the process
  * ends; its address is taken when the library initialises on that GPU).
  * Same arguments, results and bits as mfix_leq_bicgs_dev; no graph replays

@@ -43,6 +43,7 @@ struct Prof {
 };
 constexpr int kNumProf = 2;
 constexpr int kHostStates = 1024; // pinned state mirrors (max systems read back at once)
+constexpr int kPollInts = 2 + kHostStates;  // a poll's answer: running systems, its number, running flags
 constexpr int kMaxPartials = 4;   // partial-sum arrays any reduction kernel writes (NV <= 4)
 constexpr int kSizeClasses = 12;  // 8K, 32K, ..., 4^11 * 8K cells
 constexpr int kMaxRPasses = 4;    // 'R' characters of a 4-character LINE sweep string
@@ -88,6 +89,14 @@ struct MapSet {
     uint64_t version = 0;         // bumped whenever the device copy changes
 };
 
+// A captured chunk of iterations and what it was captured for.
+struct ChunkGraph {
+    hipGraphExec_t exec = nullptr;
+    int iters = 0;
+    uint64_t version = 0;
+    const void *sys = nullptr;
+};
+
 // A table of systems of one storage type and its device copy.
 template <typename T>
 struct Group {
@@ -98,11 +107,7 @@ struct Group {
     DevBuf dev;
     Sys<T> *d_sys = nullptr;
     MapSet iter;                  // systems being iterated
-    // captured chunk of iterations (replayed until every system is done)
-    hipGraphExec_t exec = nullptr;
-    int exec_iters = 0;
-    uint64_t exec_version = 0;
-    const void *exec_sys = nullptr;
+    ChunkGraph chunks[2];         // captured chunks of iterations, the first ones' length and the later ones'
     void drop_graph();
 };
 
@@ -120,7 +125,8 @@ struct Context {
     DevBuf bws;                    // batch workspace
     DevBuf partials, state, misc, tmp;
     SolverState *host_state = nullptr;  // pinned mirrors of device states
-    int *host_count = nullptr;          // pinned running-system count
+    int *host_count = nullptr;          // pinned: kPollInts of the FP64 table, then of the FP32 table
+    int poll = 0;                       // number of the last poll issued
     Group<double> g64;             // single-solve tables
     Group<float> g32;
     Group<double> b64;             // batch tables
@@ -187,11 +193,8 @@ template <typename T>
 void enqueue_setup(Group<T> &G, const MapSet &M, hipStream_t s);
 template <typename T>
 void enqueue_iterations(Group<T> &G, const MapSet &M, int n, hipStream_t s);
-// d_count (kCountBytes of device memory; NULL: the context's own buffer)
-// receives the running-system count and flags polled between chunks.
-constexpr size_t kCountBytes = 256 + 2 * sizeof(int) * kHostStates;
 template <typename T>
-int run_group(Group<T> &G, int max_iters, hipStream_t s, bool graphs, int *d_count = nullptr);
+int run_group(Group<T> &G, int max_iters, hipStream_t s, bool graphs);
 template <typename T>
 int read_states(const Group<T> &G, const std::vector<int> &ids, SolverState *h, hipStream_t s);
 

@@ -1,6 +1,6 @@
 // LEQ_BICGS on device arrays without any allocation: mfix_leq_bicgs_dev's
 // FP64 solve with its workspace (Krylov vectors, line-solve scratch, partial
-// sums, solver state), its one-row system table, block maps and poll words
+// sums, solver state), its one-row system table and block maps
 // carved from a fixed device array of kNoAllocBytes instead of the library's
 // grow-only buffers.  For callers that cannot allocate device memory (code
 // under stream capture, tight serving loops, harnesses that forbid it).
@@ -14,7 +14,7 @@
 // GPU (different streams or threads) race and must be serialised by the
 // caller.  Nothing carried over from the previous call is read before it is
 // rewritten: the solver state is reset by the set-up kernel, and every
-// partial sum and poll word is written before it is read.
+// partial sum is written before it is read.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -29,6 +29,8 @@ namespace {
 
 constexpr size_t kNoAllocBytes = MFIX_LEQ_NOALLOC_BYTES;
 constexpr int kMaxDevices = 64;
+// Kept free behind the table, so that the largest system that fits stays what it was.
+constexpr size_t kReserve = 8448;
 
 static __device__ __align__(256) char scratch[kNoAllocBytes];
 
@@ -72,8 +74,7 @@ static int solve_fp64_noalloc(char *base, const SysDesc &d, const Shape &sh, mfi
     Context &C = ctx();
     const Part P = make_part(d.g.n3, sh.bs, sh.cpt);
     const size_t o_tab = 0;
-    const size_t o_cnt = o_tab + up256(sizeof(Sys<double>));
-    const size_t o_map = o_cnt + up256(kCountBytes);
+    const size_t o_map = o_tab + up256(sizeof(Sys<double>)) + kReserve;
     const size_t maps = map_bytes(d.g, P);
     const size_t o_ws = o_map + maps;
     const size_t need = o_ws + sys_bytes(d.g, P, d.pc, false);
@@ -103,7 +104,7 @@ static int solve_fp64_noalloc(char *base, const SysDesc &d, const Shape &sh, mfi
     if ((rc = upload_table<double>(G, s, base + o_tab, up256(sizeof(Sys<double>))))) return rc;
     if ((rc = build_maps<double>(G, std::vector<int>{0}, G.iter, s, map, map_cap))) return rc;
     enqueue_setup<double>(G, G.iter, s);
-    rc = run_group<double>(G, d.itmax, s, false, (int *)(base + o_cnt));
+    rc = run_group<double>(G, d.itmax, s, false);
     SolverState *h = C.host_state;
     if (rc || (rc = read_states<double>(G, std::vector<int>{0}, h, s))) return rc;
     const hipError_t e = hipGetLastError();

@@ -96,11 +96,17 @@ struct Sys {
 // Fresh solver state of the listed systems (the whole struct is rewritten,
 // so nothing of a previous solve carries over).
 template <typename T>
-__global__ void k_init_states(const Sys<T> *__restrict__ sys, const int *__restrict__ ids, int nids) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(64) k_init_states(const Sys<T> *__restrict__ sys, const int *__restrict__ ids, int nids) {
+    const int q = blockIdx.x;
     if (q >= nids) return;
     const Sys<T> &S = sys[ids[q]];
-    SolverState s = {};
+    // a wave clears the struct (a thread alone, copying a local one, took 44 us: it went through scratch)
+    static_assert(sizeof(SolverState) % 8 == 0, "cleared in 8-byte words");
+    const gptr<double> words = to_global((double *)S.st);
+    for (int k = threadIdx.x; k < (int)(sizeof(SolverState) / 8); k += 64) words[k] = 0.0;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    SolverState &s = *S.st;
     s.tol = S.tol;
     s.itmax = S.itmax;
     s.i = 1;
@@ -113,7 +119,6 @@ __global__ void k_init_states(const Sys<T> *__restrict__ sys, const int *__restr
     s.restart_always = S.mixed && S.g.n3 >= (int64_t(1) << 18);
     s.nonunit_diag = !S.mixed || !S.unit_diag;  // the FP64 solver always divides, like the reference
     s.true_rnorm = -1.0;
-    *S.st = s;
 }
 
 // Unit scaling (leq_bicgs.f:194-233) fused with R = B - A*Var (:283-287) and
@@ -1386,21 +1391,26 @@ inline void launch_line_pcr(int var, dim3 grid, hipStream_t s, const Sys<float> 
     }
 }
 
-// Number of the listed systems still running, and a running flag per
-// listed system.
+// Number of the listed systems still running and the poll's number, and
+// a running flag per listed system, to pinned host memory that the host
+// watches (no copy, no stream synchronisation): out = {count, poll, flags}.
 template <typename T>
 __global__ void k_count_running(const Sys<T> *__restrict__ sys, const int *__restrict__ ids, int nids, int *out,
-                                int *flags) {
+                                int poll) {
     __shared__ int cnt;
     if (threadIdx.x == 0) cnt = 0;
     __syncthreads();
     for (int q = threadIdx.x; q < nids; q += blockDim.x) {
         const int run = !sys[ids[q]].st->done;
-        flags[q] = run;
+        __hip_atomic_store(&out[2 + q], run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (run) atomicAdd(&cnt, 1);
     }
+    __threadfence_system();  // the flags before the poll's number
     __syncthreads();
-    if (threadIdx.x == 0) *out = cnt;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&out[0], cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&out[1], poll, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ---- LEQ_MATVEC / LEQ_MSOLVE1 / dot / copy as standalone kernels ----------
@@ -1463,14 +1473,15 @@ __global__ void __launch_bounds__(kFinishBlock) k_finish(SolverState *st, const 
         fin_apply<F, NV>(st, tot, out);
 }
 
-// Blank state for the standalone dot/scale entries.
-static __global__ void k_init_state(SolverState *st) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        SolverState s = {};
-        s.icheck = 1;
-        s.itmax = 1;
-        s.true_rnorm = -1.0;
-        *st = s;
+// Blank state for the standalone dot/scale entries (one wave).
+static __global__ void __launch_bounds__(64) k_init_state(SolverState *st) {
+    const gptr<double> words = to_global((double *)st);
+    for (int k = threadIdx.x; k < (int)(sizeof(SolverState) / 8); k += 64) words[k] = 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        st->icheck = 1;
+        st->itmax = 1;
+        st->true_rnorm = -1.0;
     }
 }
 

@@ -2,8 +2,8 @@
 // workspaces, launch shapes (picked per grid size by the autotuner), system
 // tables and their block maps, the launch sequence of LEQ_BICGS0
 // (model/leq_bicgs.f:107-509) over a table, the driver that polls the
-// running-system count between chunks of iterations (replaying a captured
-// HIP graph per chunk), and the single and batched solve entries built on
+// running-system count between chunks of iterations (replaying captured
+// HIP graphs), and the single and batched solve entries built on
 // it.  The mixed-precision inner solve (FP32 recurrence, FP64 reliable
 // updates) runs the same sequence on a float table.
 #include <hip/hip_runtime.h>
@@ -86,9 +86,10 @@ void DevBuf::release() {
 
 template <typename T>
 void Group<T>::drop_graph() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    exec = nullptr;
-    exec_iters = 0;
+    for (ChunkGraph &k : chunks) {
+        if (k.exec) (void)hipGraphExecDestroy(k.exec);
+        k = ChunkGraph{};
+    }
 }
 template struct Group<double>;
 template struct Group<float>;
@@ -109,8 +110,10 @@ int Context::init(int dev) {
     if (e != hipSuccess) return hip_fail(e, "hipStreamCreate");
     e = hipHostMalloc((void **)&host_state, sizeof(SolverState) * kHostStates, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
-    e = hipHostMalloc((void **)&host_count, sizeof(int) * 4, hipHostMallocDefault);
+    e = hipHostMalloc((void **)&host_count, sizeof(int) * 2 * kPollInts, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
+    std::memset(host_count, 0, sizeof(int) * 2 * kPollInts);
+    poll = 0;
     if (const char *v = std::getenv("MFIX_LEQ_GRAPHS")) use_graphs = std::atoi(v);
     initialised = true;
     return 0;
@@ -415,7 +418,7 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     if (e == hipSuccess) e = hipMemcpyAsync(base + o_map, map.data(), sizeof(int2) * map.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(z, r, sizeof(T) * (size_t)g.n3, hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) return hip_fail(e, "line table upload");
-    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(1), 0, s, S.st);
+    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(64), 0, s, S.st);
     Prof &pf = C.prof[1];
     const Sys<T> *tab = (const Sys<T> *)base;
     const int2 *mp = (const int2 *)(base + o_map);
@@ -713,7 +716,7 @@ template <int BS, typename T>
 static void setup_bs(Group<T> &G, const MapSet &M, hipStream_t s) {
     const dim3 gs((unsigned)M.smap.size()), blk(BS);
     const int nids = (int)M.ids.size();
-    hipLaunchKernelGGL(k_init_states<T>, dim3((unsigned)((nids + 255) / 256)), dim3(256), 0, s, G.d_sys, M.d_ids,
+    hipLaunchKernelGGL(k_init_states<T>, dim3((unsigned)nids), dim3(64), 0, s, G.d_sys, M.d_ids,
                        nids);
     hipLaunchKernelGGL((k_setup_residual<BS, T>), gs, blk, 0, s, G.d_sys, M.d_smap);
     finish<T, FIN_SETUP, 1>(G, M, s);
@@ -827,9 +830,22 @@ template void enqueue_iterations<double>(Group<double> &, const MapSet &, int, h
 template void enqueue_iterations<float>(Group<float> &, const MapSet &, int, hipStream_t);
 
 template <typename T>
-static void enqueue_count(const Group<T> &G, const MapSet &M, int *d_out, int *d_flags, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_running<T>, dim3(1), dim3(256), 0, s, G.d_sys, M.d_ids, (int)M.ids.size(), d_out,
-                       d_flags);
+static void enqueue_count(const Group<T> &G, const MapSet &M, int *h_out, int poll, hipStream_t s) {
+    hipLaunchKernelGGL(k_count_running<T>, dim3(1), dim3(256), 0, s, G.d_sys, M.d_ids, (int)M.ids.size(), h_out, poll);
+}
+
+// Waits until both counts (either may be null) are of poll `poll` or a later
+// one.  The stream is asked now and then, so a failed launch ends the wait.
+static int wait_poll(const int *a, const int *b, int poll, hipStream_t s) {
+    auto there = [&](const int *p) { return !p || __atomic_load_n(p + 1, __ATOMIC_ACQUIRE) - poll >= 0; };
+    for (int spins = 1; !(there(a) && there(b)); ++spins) {
+        if (spins % 4096) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return hip_fail(e, "running count");
+        if (!(there(a) && there(b))) return hip_fail(hipErrorUnknown, "running count");
+    }
+    return 0;
 }
 
 // Line-kernel launch of a LINE system: 1 + its variant index among the
@@ -853,21 +869,17 @@ static int line_launch_of(const Group<T> &G, int id) {
 // dispatch a launch of idle blocks 8 times per iteration): later launches
 // stop dispatching their blocks (a handful of rebuilds per batch).
 template <typename T>
-static int compact(Group<T> &G, const int *d_flags, int running, hipStream_t s) {
+static int compact(Group<T> &G, const int *flags, int running, hipStream_t s) {
     MapSet &M = G.iter;
     if (running >= (int)M.ids.size() || running == 0) return 0;
-    std::vector<int> flags(M.ids.size());
-    hipError_t e = hipMemcpyAsync(flags.data(), d_flags, sizeof(int) * flags.size(), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return hip_fail(e, "running flags");
     std::vector<int> keep;
     double cells = 0.0;
     constexpr int kLaunches = 1 + kLineKernels + kPcrVariants;
     bool mapped[kLaunches] = {}, running_in[kLaunches] = {};
-    for (size_t q = 0; q < flags.size(); ++q) {
+    for (size_t q = 0; q < M.ids.size(); ++q) {
         const int l = line_launch_of(G, M.ids[q]);
         mapped[l] = true;
-        if (flags[q]) {
+        if (__atomic_load_n(flags + q, __ATOMIC_RELAXED)) {
             keep.push_back(M.ids[q]);
             cells += (double)G.sys[M.ids[q]].g.n3;
             running_in[l] = true;
@@ -880,14 +892,6 @@ static int compact(Group<T> &G, const int *d_flags, int running, hipStream_t s) 
 }
 
 // Chunk of iterations of both tables, captured once and replayed.
-struct ChunkGraph {
-    hipGraphExec_t exec = nullptr;
-    int iters = 0;
-    uint64_t v64 = 0, v32 = 0;
-    const void *s64 = nullptr, *s32 = nullptr;
-    const void *m64 = nullptr, *m32 = nullptr;
-};
-
 static int capture_chunk(Group<double> *G64, Group<float> *G32, int iters, hipStream_t s, hipGraphExec_t *out) {
     hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
@@ -904,85 +908,97 @@ static int capture_chunk(Group<double> *G64, Group<float> *G32, int iters, hipSt
     return 0;
 }
 
-// Drive both tables (either may be null) until every system is done.  The
-// running count is polled after each chunk; chunks grow 4, 8, ... 64
-// iterations (direct launches) or are a captured graph of 16, never more
-// than ITMAX.  Launches after a system is done return at once, so
-// overshooting is harmless, but each still dispatches its blocks.
-static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs,
-                      int *d_count = nullptr) {
+// Drive both tables (either may be null) until every system is done.  After
+// each chunk of iterations (direct launches, or replays of a captured graph)
+// a kernel writes the running-system count to pinned host memory; the host
+// issues the next chunk before it waits for the previous chunk's count, so
+// the device never idles for it and at most one chunk runs after the last
+// system is done.  Its launches return at once, but each still dispatches its
+// blocks: an idle LINE iteration costs about 35 us at 128^3 (16 launches)
+// where a working one takes 360 us and such solves take 1-20 iterations, so
+// LINE tables start with chunks of one iteration, the others (whose
+// iterations are 5-9 short launches, hundreds a solve) with four.  Chunks of
+// a fixed 16 iterations, each polled with a copy, ran a 128^3 LINE momentum
+// solve of four iterations in 2,101 us; now 1,695.  No chunk runs past ITMAX.
+static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
     Context &C = ctx();
     int rc;
-    if (!d_count) {
-        if ((rc = C.misc.ensure(kCountBytes))) return rc;
-        d_count = (int *)C.misc.ptr;
-    }
-    int *d_cnt = d_count;
-    int *d_flags64 = (int *)((char *)d_count + 256);
-    int *d_flags32 = d_flags64 + kHostStates;
+    int *h64 = C.host_count, *h32 = C.host_count + kPollInts;
     if (G64 && G64->iter.ids.empty()) G64 = nullptr;
     if (G32 && G32->iter.ids.empty()) G32 = nullptr;
     if (!G64 && !G32) return 0;
     if (C.prof[0].on || C.prof[1].on) graphs = false;
     // one-by-one LINE sweeps bake their arrays into the launches: no replay
     if ((G64 && !G64->iter.line_seq.empty()) || (G32 && !G32->iter.line_seq.empty())) graphs = false;
-    // graph owner: the float table's slot when present, else the double one
-    hipGraphExec_t *exec = G32 ? &G32->exec : &G64->exec;
-    int *exec_iters = G32 ? &G32->exec_iters : &G64->exec_iters;
-    uint64_t *exec_version = G32 ? &G32->exec_version : &G64->exec_version;
-    const void **exec_sys = G32 ? &G32->exec_sys : &G64->exec_sys;
-    const void *sys_key = G32 ? (const void *)G32->d_sys : (const void *)G64->d_sys;
-    // no chunk runs past ITMAX: with MFIX's LEQ_IT of 5-20 a fixed 16 would
-    // dispatch every block of up to 11 idle iterations per solve
-    const int cap = std::max(1, std::min(max_iters, 64));
-    const int kGraphIters = std::min(16, cap);
-    int64_t issued = 0;
-    int chunk = std::min(4, cap);
-    for (;;) {
-        if (G64) enqueue_count<double>(*G64, G64->iter, d_cnt + 0, d_flags64, s);
-        if (G32) enqueue_count<float>(*G32, G32->iter, d_cnt + 1, d_flags32, s);
-        hipError_t e = hipMemcpyAsync(C.host_count, d_cnt, 2 * sizeof(int), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return hip_fail(e, "running count");
-        const int running = (G64 ? C.host_count[0] : 0) + (G32 ? C.host_count[1] : 0);
-        if (running == 0) return 0;
-        if (issued > 4 * ((int64_t)max_iters + 8)) return hip_fail(hipErrorUnknown, "solver did not terminate");
-        if (G64 && (rc = compact<double>(*G64, d_flags64, C.host_count[0], s))) return rc;
-        if (G32 && (rc = compact<float>(*G32, d_flags32, C.host_count[1], s))) return rc;
-        if (G64 && G64->iter.ids.empty()) G64 = nullptr;
-        if (G32 && G32->iter.ids.empty()) G32 = nullptr;
-        const uint64_t version = (G64 ? G64->iter.version * 1000003ull : 0) ^ (G32 ? G32->iter.version : 0) ^
-                                 ((G64 ? 1ull : 0) << 62) ^ ((G32 ? 1ull : 0) << 63);
-        if (graphs) {
-            if (!*exec || *exec_iters != kGraphIters || *exec_version != version || *exec_sys != sys_key) {
-                if (*exec) (void)hipGraphExecDestroy(*exec);
-                *exec = nullptr;
-                if ((rc = capture_chunk(G64, G32, kGraphIters, s, exec))) return rc;
-                *exec_iters = kGraphIters;
-                *exec_version = version;
-                *exec_sys = sys_key;
-            }
-            e = hipGraphLaunch(*exec, s);
-            if (e != hipSuccess) return hip_fail(e, "hipGraphLaunch");
-            issued += kGraphIters;
-        } else {
-            for (int q = 0; q < chunk; ++q) {
+    const bool line = (G64 && G64->iter.n_line) || (G32 && G32->iter.n_line);
+    const int first = line ? 1 : 4, most = line ? 4 : 16;
+    auto count = [&](int poll) {
+        if (G64) enqueue_count<double>(*G64, G64->iter, h64, poll, s);
+        if (G32) enqueue_count<float>(*G32, G32->iter, h32, poll, s);
+    };
+    // `iters` iterations, by a replay of the captured chunk of that length
+    // where there is one (kept in the float table's slots when present)
+    auto issue = [&](int iters) -> int {
+        if (!graphs || (iters != first && iters != most)) {
+            for (int q = 0; q < iters; ++q) {
                 if (G64) enqueue_iterations<double>(*G64, G64->iter, 1, s);
                 if (G32) enqueue_iterations<float>(*G32, G32->iter, 1, s);
             }
-            issued += chunk;
-            chunk = std::min(chunk * 2, cap);
+            return 0;
         }
+        ChunkGraph &K = (G32 ? G32->chunks : G64->chunks)[iters == most ? 1 : 0];
+        const void *sys_key = G32 ? (const void *)G32->d_sys : (const void *)G64->d_sys;
+        const uint64_t version = (G64 ? G64->iter.version * 1000003ull : 0) ^ (G32 ? G32->iter.version : 0) ^
+                                 ((G64 ? 1ull : 0) << 62) ^ ((G32 ? 1ull : 0) << 63);
+        if (!K.exec || K.iters != iters || K.version != version || K.sys != sys_key) {
+            if (K.exec) (void)hipGraphExecDestroy(K.exec);
+            K.exec = nullptr;
+            int e;
+            if ((e = capture_chunk(G64, G32, iters, s, &K.exec))) return e;
+            K.iters = iters;
+            K.version = version;
+            K.sys = sys_key;
+        }
+        const hipError_t e = hipGraphLaunch(K.exec, s);
+        return e == hipSuccess ? 0 : hip_fail(e, "hipGraphLaunch");
+    };
+    int64_t issued = 0;
+    count(++C.poll);
+    for (int done_chunks = 0;; ++done_chunks) {
+        const int poll = C.poll;
+        // the next chunk, while the device works towards poll `poll`; every
+        // system is done after ITMAX iterations
+        if (issued < max_iters) {
+            int chunk = done_chunks < 8 ? first : most;
+            if (chunk > max_iters - issued) chunk = (int)(max_iters - issued);
+            if ((rc = issue(chunk))) return rc;
+            issued += chunk;
+            count(++C.poll);
+        }
+        if ((rc = wait_poll(G64 ? h64 : nullptr, G32 ? h32 : nullptr, poll, s))) return rc;
+        const int run64 = G64 ? __atomic_load_n(h64, __ATOMIC_RELAXED) : 0;
+        const int run32 = G32 ? __atomic_load_n(h32, __ATOMIC_RELAXED) : 0;
+        if (run64 + run32 == 0) return 0;
+        if (poll == C.poll) return hip_fail(hipErrorUnknown, "solver did not terminate");
+        const uint64_t v64 = G64 ? G64->iter.version : 0, v32 = G32 ? G32->iter.version : 0;
+        if (G64 && (rc = compact<double>(*G64, h64 + 2, run64, s))) return rc;
+        if (G32 && (rc = compact<float>(*G32, h32 + 2, run32, s))) return rc;
+        const bool rebuilt = (G64 && G64->iter.version != v64) || (G32 && G32->iter.version != v32);
+        if (G64 && !run64) G64 = nullptr;
+        if (G32 && !run32) G32 = nullptr;
+        // flags are in the order of the maps' systems: polls issued before a
+        // rebuild are not looked at (they ran before its upload)
+        if (rebuilt) count(++C.poll);
     }
 }
 
 template <typename T>
-int run_group(Group<T> &G, int max_iters, hipStream_t s, bool graphs, int *d_count) {
-    if constexpr (sizeof(T) == sizeof(double)) return run_tables(&G, nullptr, max_iters, s, graphs, d_count);
-    else return run_tables(nullptr, &G, max_iters, s, graphs, d_count);
+int run_group(Group<T> &G, int max_iters, hipStream_t s, bool graphs) {
+    if constexpr (sizeof(T) == sizeof(double)) return run_tables(&G, nullptr, max_iters, s, graphs);
+    else return run_tables(nullptr, &G, max_iters, s, graphs);
 }
-template int run_group<double>(Group<double> &, int, hipStream_t, bool, int *);
-template int run_group<float>(Group<float> &, int, hipStream_t, bool, int *);
+template int run_group<double>(Group<double> &, int, hipStream_t, bool);
+template int run_group<float>(Group<float> &, int, hipStream_t, bool);
 
 template <typename T>
 int read_states(const Group<T> &G, const std::vector<int> &ids, SolverState *h, hipStream_t s) {
@@ -1289,7 +1305,7 @@ int run_matvec32(const DGrid &g, const float *a, const float *x, float *y, hipSt
     hipError_t e = hipMemcpyAsync(base, &S, sizeof(S), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(base + o_map, map.data(), sizeof(int2) * map.size(), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return hip_fail(e, "matvec table upload");
-    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(1), 0, s, S.st);
+    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(64), 0, s, S.st);
     const Sys<float> *tab = (const Sys<float> *)base;
     const int2 *mp = (const int2 *)(base + o_map);
     MFIX_DISPATCH_BS(sh.bs, BS,
@@ -1314,7 +1330,7 @@ int run_dot(const DGrid &g, const double *x, const double *y, double *d_out, hip
     if ((rc = C.partials.ensure(sizeof(double) * P.nblk * kMaxPartials + 64))) return rc;
     if ((rc = C.state.ensure(sizeof(SolverState)))) return rc;
     SolverState *st = (SolverState *)C.state.ptr;
-    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(1), 0, s, st);
+    hipLaunchKernelGGL(k_init_state, dim3(1), dim3(64), 0, s, st);
     MFIX_DISPATCH_BS(sh.bs, BS,
                      hipLaunchKernelGGL((k_dot<BS, double>), grid_of(P), dim3(BS), 0, s, g, P, x, y, g.dot_all ? 0 : 1,
                                         (double *)C.partials.ptr));
@@ -1344,7 +1360,7 @@ int run_scale(const DGrid &g, double *a, double *b, int *zero_row, hipStream_t s
     sys_carve<double>(G.sys[0], d, P, (char *)C.ws.ptr);
     if ((rc = upload_table<double>(G, s)) || (rc = build_maps<double>(G, std::vector<int>{0}, G.iter, s))) return rc;
     const int nids = 1;
-    hipLaunchKernelGGL(k_init_states<double>, dim3(1), dim3(256), 0, s, G.d_sys, G.iter.d_ids, nids);
+    hipLaunchKernelGGL(k_init_states<double>, dim3(1), dim3(64), 0, s, G.d_sys, G.iter.d_ids, nids);
     MFIX_DISPATCH_BS(sh.bs, BS,
                      hipLaunchKernelGGL((k_setup_residual<BS, double>), dim3((unsigned)G.iter.smap.size()), dim3(BS),
                                         0, s, G.d_sys, G.iter.d_smap));
