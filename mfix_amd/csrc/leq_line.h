@@ -131,109 +131,9 @@ __device__ __forceinline__ void whole_lines(const DGrid &g, int lpb, int64_t fir
 constexpr double kSwapUp = 0x1p600, kSwapDown = 0x1p-600;
 __device__ __forceinline__ bool swapped(double f) { return fabs(f) > 2.0; }
 
-// DGTSV's elimination of every line of the listed FP64 systems, both colours
-// (blockIdx.y = colour), in cell order: the multipliers (row 0: 0) to S.lf and
-// the eliminated diagonal to S.ld, and, for a block of lines with a row
-// interchange, the eliminated first and second super-diagonals to S.lu and
-// S.lu2 (else they are A_M's upper coupling and 0).
-static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<double> *__restrict__ sys,
-                                                                      const int2 *__restrict__ map) {
-    extern __shared__ __align__(16) char whole_lds[];
-    __shared__ WholeLines w;
-    const int2 e = map[blockIdx.x];
-    if (e.x < 0) return;
-    const Sys<double> &S = sys[e.x];
-    auto *__restrict__ st = to_global(S.st);
-    if (st->done) return;
-    const DGrid &g = S.g;
-    const int n = g.nj, ls = whole_stride(n);
-    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, (int)blockIdx.y, w);
-    const int nl = w.n, tot = nl * n;
-    double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ D = F + S.lpb * ls,
-                         *__restrict__ U = D + S.lpb * ls, *__restrict__ V = U + S.lpb * ls;
-    const int64_t n3 = g.n3;
-    const gptr<const double> a = to_global(S.a);
-    for (int e0 = threadIdx.x; e0 < tot; e0 += 2 * kWholeThreads) {
-        double dl[2], d[2], du[2];
-        int o[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int x = e0 + k * kWholeThreads < tot ? e0 + k * kWholeThreads : e0;
-            const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n;
-            const uint32_t c = w.c0[l] + (uint32_t)q;
-            o[k] = l * ls + q;
-            dl[k] = q > 0 ? a[1 * n3 + c] : 0.0;
-            d[k] = a[3 * n3 + c];
-            du[k] = q < n - 1 ? a[5 * n3 + c] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            F[o[k]] = dl[k];
-            D[o[k]] = d[k];
-            U[o[k]] = du[k];
-        }
-    }
-    __syncthreads();
-    int any = 0;
-    if ((int)threadIdx.x < nl) {
-        const int o = threadIdx.x * ls;
-        double d = D[o], u = U[o];
-        bool ok = true;
-        double dl1 = F[o + 1], d1 = D[o + 1], u1 = U[o + 1];  // (a line has at least three rows)
-        for (int i = 0; i < n - 1; ++i) {
-            const int nx = i + 2 < n ? i + 2 : n - 1;  // the next row is read ahead of this one's division
-            const double dl2 = F[o + nx], d2 = D[o + nx], u2 = U[o + nx];
-            double fd = d, fu = u, fv = 0.0, f, dn, un = u1;
-            if (fabs(d) >= fabs(dl1)) {
-                f = dl1 / d;  // (DGTSV.f:111-122)
-                dn = d1 - f * u;
-            } else {
-                // interchange rows i and i+1 (DGTSV.f:123-136, :148-158)
-                const double fact = d / dl1;
-                fd = dl1;
-                fu = d1;
-                dn = u - fact * d1;
-                if (i < n - 2) {
-                    fv = u1;
-                    un = -fact * u1;
-                }
-                f = fact * kSwapUp;
-                ok = ok && swapped(f);
-                any = 1;
-            }
-            ok = ok && factor_in_range(fd);
-            F[o + i + 1] = f;
-            D[o + i] = fd;
-            U[o + i] = fu;
-            V[o + i] = fv;
-            d = dn;
-            u = un;
-            dl1 = dl2;
-            d1 = d2;
-            u1 = u2;
-        }
-        D[o + n - 1] = d;
-        U[o + n - 1] = 0.0;
-        V[o + n - 1] = 0.0;
-        ok = ok && factor_in_range(d);
-        if (!ok) atomicOr((int *)&st->line_general, 1);
-    }
-    any = __syncthreads_or(any);
-    const gptr<double> lf = to_global(S.lf), ld = to_global(S.ld), lu = to_global(S.lu), lu2 = to_global(S.lu2);
-    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
-        const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
-        const uint32_t c = w.c0[l] + (uint32_t)q;
-        lf[c] = F[at];
-        ld[c] = D[at];
-        if (any) {
-            lu[c] = U[at];
-            lu2[c] = V[at];
-        }
-    }
-}
-
-// The two passes of one line on its factored rows, in the lane that solves it,
-// over whole_rows(n) rows.  A pass is bound by its LDS instructions (each
+// The elimination of one line without row interchanges and the two passes on
+// its factored rows, in the lane that solves the line, over whole_rows(n)
+// rows.  A pass is bound by its LDS instructions (each
 // costs what all 64 lanes of it would, 10-25 cycles) more than by the
 // arithmetic (a dependent FP64 operation takes about five): two rows move per
 // instruction, read one register set ahead of the chain at fixed offsets from
@@ -242,6 +142,52 @@ static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<
 // inside the block's LDS, and are not used.  Measured alone: 35 and 61 cycles
 // a row.
 typedef double pair2 __attribute__((ext_vector_type(2)));
+
+// (the divisions by the running diagonal are the chain: rows in and out are
+// the last of it).  Whether the multipliers and the diagonal are DGTSV's is for
+// the caller to look at: |F| <= 1 (no interchange) and both in range.
+__device__ __forceinline__ void whole_eliminate(double *__restrict__ pf, double *__restrict__ pd,
+                                                const double *__restrict__ pu, int rows) {
+    constexpr int R = 4;
+    struct Rows {
+        pair2 f[R / 2], d[R / 2], u[R / 2];
+    } s0, s1;
+    auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            w.f[k] = *(const pair2 *)&pf[at + 2 * k];
+            w.d[k] = *(const pair2 *)&pd[at + 2 * k];
+            w.u[k] = *(const pair2 *)&pu[at + 2 * k];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    double d = 1.0, u = 0.0;  // (row 0's lower coupling is 0)
+    auto one = [&](double &f, double &dr, double ur) __attribute__((always_inline)) {
+        f = corrected_quotient(f, d, refined_rcp(d));
+        d = dr - f * u;
+        dr = d;
+        u = ur;
+    };
+    auto run = [&](Rows &w, int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            double f0 = w.f[k].x, f1 = w.f[k].y, d0 = w.d[k].x, d1 = w.d[k].y;
+            one(f0, d0, w.u[k].x);
+            one(f1, d1, w.u[k].y);
+            *(pair2 *)&pf[at + 2 * k] = pair2{f0, f1};
+            *(pair2 *)&pd[at + 2 * k] = pair2{d0, d1};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(s0, 0);
+    for (; rows >= 2 * R; rows -= 2 * R, pf += 2 * R, pd += 2 * R, pu += 2 * R) {
+        get(s1, R);
+        run(s0, 0);
+        get(s0, 2 * R);
+        run(s1, R);
+    }
+    if (rows > 0) run(s0, 0);
+}
 
 __device__ __forceinline__ void whole_forward(const double *__restrict__ pf, double *__restrict__ pb, int rows) {
     constexpr int R = 8;
@@ -331,75 +277,229 @@ __device__ __forceinline__ void whole_back(double *__restrict__ pb, const double
 // The same two passes where some line of the block interchanges rows: the
 // right-hand sides trade places with them, and the second super-diagonal (in
 // V, the reciprocals' place: they are formed in the chain here) comes in.
-__device__ __forceinline__ void whole_forward_swap(const double *__restrict__ pf, double *__restrict__ pb, int n) {
+__device__ __forceinline__ void whole_forward_swap(const double *__restrict__ pf, double *__restrict__ pb, int rows) {
     constexpr int R = 4;
-    double f[R], r[R];
-    auto get = [&](int q0) __attribute__((always_inline)) {
+    struct Rows {
+        pair2 f[R / 2], b[R / 2];
+    } s0, s1;
+    auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int q = q0 + k < n ? q0 + k : n - 1;
-            f[k] = pf[q];
-            r[k] = pb[q];
+        for (int k = 0; k < R / 2; ++k) {
+            w.f[k] = *(const pair2 *)&pf[at + 2 * k];
+            w.b[k] = *(const pair2 *)&pb[at + 2 * k];
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    double b = pb[0];
-    get(1);
-    for (int q0 = 1; q0 < n; q0 += R) {
-        double cf[R], cr[R];
+    double b = 0.0;
+    // row q's multiplier and right-hand side; returns row q-1's after the interchange
+    auto one = [&](double f, double r) __attribute__((always_inline)) {
+        const bool s = swapped(f);
+        const double fact = s ? f * kSwapDown : f;
+        const double top = s ? r : b;
+        b = (s ? b : r) - fact * top;
+        return top;
+    };
+    auto run = [&](const Rows &w, int at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-            cf[k] = f[k];
-            cr[k] = r[k];
+        for (int k = 0; k < R / 2; ++k) {  // (row 0 writes in front of the line, an element that is not used)
+            pb[at + 2 * k - 1] = one(w.f[k].x, w.b[k].x);
+            pb[at + 2 * k] = one(w.f[k].y, w.b[k].y);
         }
-        get(q0 + R);
-#pragma unroll
-        for (int k = 0; k < R; ++k)
-            if (q0 + k < n) {
-                const bool s = swapped(cf[k]);
-                const double fact = s ? cf[k] * kSwapDown : cf[k];
-                const double top = s ? cr[k] : b;  // row q-1's after the interchange
-                b = (s ? b : cr[k]) - fact * top;
-                pb[q0 + k - 1] = top;
-            }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(s0, 0);
+    for (; rows >= 2 * R; rows -= 2 * R, pf += 2 * R, pb += 2 * R) {
+        get(s1, R);
+        run(s0, 0);
+        get(s0, 2 * R);
+        run(s1, R);
     }
-    pb[n - 1] = b;
+    if (rows > 0) {
+        run(s0, 0);
+        pb += R;
+    }
+    pb[-1] = b;
 }
 
 __device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const double *__restrict__ pu,
-                                                const double *__restrict__ pv, const double *__restrict__ pd, int n) {
+                                                const double *__restrict__ pv, const double *__restrict__ pd, int rows) {
     constexpr int R = 4;
-    double b[R], u[R], v[R], d[R];
-    auto get = [&](int q0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int q = q0 - k > 0 ? q0 - k : 0;
-            b[k] = pb[q];
-            u[k] = pu[q];
-            v[k] = pv[q];
-            d[k] = pd[q];
-        }
-    };
+    struct Rows {
+        pair2 b[R / 2], u[R / 2], v[R / 2], d[R / 2];
+    } s0, s1;
+    pb += rows - 2;
+    pu += rows - 2;
+    pv += rows - 2;
+    pd += rows - 2;
     double x1 = 0.0, x2 = 0.0;
-    get(n - 1);
-    for (int q0 = n - 1; q0 >= 0; q0 -= R) {
-        double cb[R], cu[R], cv[R], cd[R], cr[R];
+    auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-            cb[k] = b[k];
-            cu[k] = u[k];
-            cv[k] = v[k];
-            cd[k] = d[k];
-            cr[k] = refined_rcp(d[k]);
+        for (int k = 0; k < R / 2; ++k) {
+            w.b[k] = *(const pair2 *)&pb[-at - 2 * k];
+            w.u[k] = *(const pair2 *)&pu[-at - 2 * k];
+            w.v[k] = *(const pair2 *)&pv[-at - 2 * k];
+            w.d[k] = *(const pair2 *)&pd[-at - 2 * k];
         }
-        get(q0 - R);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto one = [&](double b, double u, double v, double d) __attribute__((always_inline)) {
+        const double x = corrected_quotient(b - u * x1 - v * x2, d, refined_rcp(d));
+        x2 = x1;
+        x1 = x;
+        return x;
+    };
+    auto run = [&](const Rows &w, int at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < R; ++k)
-            if (q0 - k >= 0) {
-                const double x = corrected_quotient(cb[k] - cu[k] * x1 - cv[k] * x2, cd[k], cr[k]);
-                x2 = x1;
-                x1 = x;
-                pb[q0 - k] = x;
+        for (int k = 0; k < R / 2; ++k) {
+            pair2 o;
+            o.y = one(w.b[k].y, w.u[k].y, w.v[k].y, w.d[k].y);
+            o.x = one(w.b[k].x, w.u[k].x, w.v[k].x, w.d[k].x);
+            *(pair2 *)&pb[-at - 2 * k] = o;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(s0, 0);
+    for (; rows >= 2 * R; rows -= 2 * R, pb -= 2 * R, pu -= 2 * R, pv -= 2 * R, pd -= 2 * R) {
+        get(s1, R);
+        run(s0, 0);
+        get(s0, 2 * R);
+        run(s1, R);
+    }
+    if (rows > 0) run(s0, 0);
+}
+
+// DGTSV's elimination of every line of the listed FP64 systems, both colours
+// (blockIdx.y = colour), in cell order: the multipliers (row 0: 0) to S.lf and
+// the eliminated diagonal to S.ld, and, for a block of lines with a row
+// interchange, the eliminated first and second super-diagonals to S.lu and
+// S.lu2 (else they are A_M's upper coupling and 0).
+static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<double> *__restrict__ sys,
+                                                                      const int2 *__restrict__ map) {
+    extern __shared__ __align__(16) char whole_lds[];
+    __shared__ WholeLines w;
+    const int2 e = map[blockIdx.x];
+    if (e.x < 0) return;
+    const Sys<double> &S = sys[e.x];
+    auto *__restrict__ st = to_global(S.st);
+    if (st->done) return;
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n);
+    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, (int)blockIdx.y, w);
+    const int nl = w.n, tot = nl * n;
+    double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ D = F + S.lpb * ls,
+                         *__restrict__ U = D + S.lpb * ls, *__restrict__ V = U + S.lpb * ls;
+    const int64_t n3 = g.n3;
+    const gptr<const double> a = to_global(S.a);
+    auto load = [&]() {
+#pragma unroll
+        for (int k0 = 0; k0 < kWholeElems; k0 += 3) {
+            if (k0 * kWholeThreads >= tot) break;
+            double dl[3], d[3], du[3];
+            int o[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
+                const int x = x0 < tot ? x0 : tot - 1;  // (past the end: the last row again)
+                const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n;
+                const uint32_t c = w.c0[l] + (uint32_t)q;
+                o[k] = l * ls + q;
+                dl[k] = q > 0 ? a[1 * n3 + c] : 0.0;
+                d[k] = a[3 * n3 + c];
+                du[k] = q < n - 1 ? a[5 * n3 + c] : 0.0;
             }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                F[o[k]] = dl[k];
+                D[o[k]] = d[k];
+                U[o[k]] = du[k];
+            }
+        }
+        for (int x = threadIdx.x; x < 4 * nl; x += kWholeThreads) {
+            const int q = n + (x & 3), at = (x >> 2) * ls + q;
+            if (q < whole_rows(n)) {  // identity rows
+                F[at] = U[at] = 0.0;
+                D[at] = 1.0;
+            }
+        }
+        __syncthreads();
+    };
+    const gptr<double> lf = to_global(S.lf), ld = to_global(S.ld), lu = to_global(S.lu), lu2 = to_global(S.lu2);
+    // without interchanges first; all threads look at the result
+    load();
+    if ((int)threadIdx.x < nl) {
+        const int o = threadIdx.x * ls;
+        whole_eliminate(F + o, D + o, U + o, whole_rows(n));
+    }
+    __syncthreads();
+    int bad = 0;
+    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+        const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), at = l * ls + x - l * n;
+        bad |= !(fabs(F[at]) <= 1.0 && solution_in_range(F[at]) && factor_in_range(D[at]));
+    }
+    if (!__syncthreads_or(bad)) {
+        for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+            const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
+            const uint32_t c = w.c0[l] + (uint32_t)q;
+            lf[c] = F[at];
+            ld[c] = D[at];
+        }
+        return;
+    }
+    load();
+    int any = 0;
+    if ((int)threadIdx.x < nl) {
+        const int o = threadIdx.x * ls;
+        double d = D[o], u = U[o];
+        bool ok = true;
+        double dl1 = F[o + 1], d1 = D[o + 1], u1 = U[o + 1];  // (a line has at least three rows)
+        for (int i = 0; i < n - 1; ++i) {
+            const int nx = i + 2 < n ? i + 2 : n - 1;  // the next row is read ahead of this one's division
+            const double dl2 = F[o + nx], d2 = D[o + nx], u2 = U[o + nx];
+            double fd = d, fu = u, fv = 0.0, f, dn, un = u1;
+            if (fabs(d) >= fabs(dl1)) {
+                f = dl1 / d;  // (DGTSV.f:111-122)
+                dn = d1 - f * u;
+            } else {
+                // interchange rows i and i+1 (DGTSV.f:123-136, :148-158)
+                const double fact = d / dl1;
+                fd = dl1;
+                fu = d1;
+                dn = u - fact * d1;
+                if (i < n - 2) {
+                    fv = u1;
+                    un = -fact * u1;
+                }
+                f = fact * kSwapUp;
+                ok = ok && swapped(f);
+                any = 1;
+            }
+            ok = ok && factor_in_range(fd);
+            F[o + i + 1] = f;
+            D[o + i] = fd;
+            U[o + i] = fu;
+            V[o + i] = fv;
+            d = dn;
+            u = un;
+            dl1 = dl2;
+            d1 = d2;
+            u1 = u2;
+        }
+        D[o + n - 1] = d;
+        U[o + n - 1] = 0.0;
+        V[o + n - 1] = 0.0;
+        ok = ok && factor_in_range(d);
+        if (!ok) atomicOr((int *)&st->line_general, 1);
+    }
+    any = __syncthreads_or(any);
+    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+        const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
+        const uint32_t c = w.c0[l] + (uint32_t)q;
+        lf[c] = F[at];
+        ld[c] = D[at];
+        if (any) {
+            lu[c] = U[at];
+            lu2[c] = V[at];
+        }
     }
 }
 
@@ -563,7 +663,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             const bool mine = solver >= 0 && solver < nl;
             const int ol = solver * ls;
             if (mine) {
-                if (swaps) whole_forward_swap(F + ol, B + ol, n);
+                if (swaps) whole_forward_swap(F + ol, B + ol, rows);
                 else whole_forward(F + ol, B + ol, rows);
             }
             __syncthreads();
@@ -576,7 +676,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             }
             __syncthreads();
             if (mine) {
-                if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, n);
+                if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
                 else whole_back(B + ol, U + ol, F + ol, D + ol, rows);
             }
             __syncthreads();
