@@ -13,6 +13,7 @@
 #include "../../include/mfix_leq.h"
 #include "leq_line.h"
 #include "leq_phases.h"
+#include "leq_resident.h"
 
 namespace mfix {
 

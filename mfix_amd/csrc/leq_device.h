@@ -435,18 +435,52 @@ __device__ __forceinline__ int64_t march_cell(const DGrid &g, int64_t L, int bs,
     return m < g.c2 ? (int64_t)k * g.c2 + m : -1;
 }
 
-// ---- deterministic reductions (fixed tree, wave64 shuffles) ----------------
+// ---- deterministic reductions (fixed tree over a wave's 64 lanes) ------------
+
+// Lane l's value of lane l + N of its row of 16 (row shift; past the row's end: 0).
+template <int N>
+__device__ __forceinline__ double row_down(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x100 | N, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x100 | N, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// The upper half of the wave in its lower half (32), or the odd rows of 16 in
+// the even ones (16).
+template <int N>
+__device__ __forceinline__ double half_down(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t a = (uint32_t)u, b = (uint32_t)(u >> 32);
+    if constexpr (N == 32) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        return __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+    } else {
+        const auto lo = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        return __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+    }
+}
+// Sum over the wave in lane 0 (the other lanes hold partial sums): lanes l and
+// l + 32 first, then l and l + 16, down to 1, the order of a __shfl_down tree,
+// by lane permutes of the vector unit instead of the LDS pipe (a level takes
+// about 20 cycles where a shuffle of two halves takes about 130).
+__device__ __forceinline__ double wave_sum(double s) {
+    s += half_down<32>(s);
+    s += half_down<16>(s);
+    s += row_down<8>(s);
+    s += row_down<4>(s);
+    s += row_down<2>(s);
+    s += row_down<1>(s);
+    return s;
+}
+
 // block_sum leaves the block totals in thread 0; lds holds NV * (BS/64).
 template <int BS, int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double *lds) {
     constexpr int NW = BS / 64;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = v[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        v[q] = s;
-    }
+    for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) {
 #pragma unroll
@@ -498,12 +532,7 @@ __device__ __forceinline__ void block_partial_last(double (&v)[NV], PD partials,
                                                    double *lds, unsigned *cnt) {
     constexpr int NW = BS / 64;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = v[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        v[q] = s;
-    }
+    for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);
     if ((threadIdx.x & 63) != 0) return;
     if (NW == 1) {
 #pragma unroll

@@ -1038,6 +1038,30 @@ static Sweep make_sweep(const char *cmethod) {
     return sw;
 }
 
+// Whether a system can run as one resident launch (k_resident): FP64, DIAG or
+// NONE, 256-cell blocks, at most as many as the device holds at once (two per
+// CU, 131,072 cells).  Up to there an iteration takes half the launches' time
+// (48^3, 488 blocks: 15.4 against 30.3 us); with four blocks of 128 VGPRs per
+// CU, part of the neighbours' values in scratch, the advantage is gone (50^3
+// 28.4 against 28.9 us, 62^3 35.9 against 34).
+static bool resident_fits(const Sys<double> &S, int bs) {
+    return S.pc != PC_LINE && bs == kResidentBlock && S.P.chunk == kResidentBlock && S.P.nblk <= kResidentBlocks;
+}
+
+// False when the device does not take the launch (nothing ran then).
+static bool launch_resident(Group<double> &G, hipStream_t s) {
+    const int64_t nblk = G.sys[0].P.nblk;
+    const Sys<double> *tab = G.d_sys;
+    hipLaunchKernelGGL(k_resident_slots, dim3((unsigned)((resident_slots(nblk) + 255) / 256)), dim3(256), 0, s, tab);
+    void *args[] = {(void *)&tab};
+    const void *f = G.sys[0].pc == PC_DIAG ? (const void *)k_resident<OP_DIAG> : (const void *)k_resident<OP_PLAIN>;
+    if (hipLaunchCooperativeKernel(f, dim3((unsigned)nblk), dim3(kResidentBlock), args, 0, s) ==
+        hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 template <typename T>
 static int solve_one(Group<T> &G, const SysDesc &d, const Shape &sh, mfix_leq_stats *stats, hipStream_t s) {
     Context &C = ctx();
@@ -1070,7 +1094,10 @@ static int solve_one(Group<T> &G, const SysDesc &d, const Shape &sh, mfix_leq_st
     if (resid) launch_resid_finish(d.g, d.pro.resid_kind, d.resid_debug, d.resid_norm, G.sys[0].pro.rpart, P.nblk,
                                    d_rout, s);
     const bool graphs = C.use_graphs && d.g.n3 <= ((int64_t)1 << 22);
-    rc = run_group<T>(G, d.itmax, s, graphs);
+    bool whole = false;
+    if constexpr (sizeof(T) == sizeof(double))
+        if (graphs && !C.prof[0].on && resident_fits(G.sys[0], G.bs)) whole = launch_resident(G, s);
+    if (!whole) rc = run_group<T>(G, d.itmax, s, graphs);
     (void)hipEventRecord(e1, s);
     (void)hipEventSynchronize(e1);
     float ms = 0.f;
@@ -1101,6 +1128,7 @@ static int solve_one(Group<T> &G, const SysDesc &d, const Shape &sh, mfix_leq_st
     fill_stats(*h, stats);
     if (stats) stats->device_ms = ms;
     if (h->msolve_fatal) return MFIX_LEQ_EDGTSV;
+    if (h->resident_gone) return hip_fail(hipErrorLaunchTimeOut, "resident solve");
     return 0;
 }
 
