@@ -171,6 +171,7 @@ struct SysDesc {
     double *x, *a, *b;            // VAR, A_M, B_M (FP64, device)
     const double *noise;
     uint64_t seed;
+    double line_lds = 0.0;        // LINE, FP64: LDS of a colour's lines of all systems of the launch (0: this one's)
     Prologue pro;                 // residual / under-relaxation in the set-up pass
     mfix_leq_resid *resid_out = nullptr;  // host: the residual's result (pro.resid_kind >= 0)
     int resid_debug = 0;

@@ -32,6 +32,8 @@
 // scratch): 64^3 28.4 -> 10.2 us, 128^3 56.2 -> 29.0 us, 158^3 70.9 -> 50.5
 // us, 256^3 409 -> 234 us.
 #pragma once
+#include <cmath>
+
 #include "leq_phases.h"
 
 namespace mfix {
@@ -59,15 +61,22 @@ __host__ __device__ constexpr int whole_elems(int n, int lpb) {
     return kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
 }
 
-// Lines per block for lines of n rows, `lines` of them in a colour: as many
-// as the LDS target and the rows per thread hold, but few enough that a colour
-// makes 512 blocks (two per CU; below that CUs idle while others run a second
-// block), at least one.  pin: mfix_leq_set_line_block's value, 0 = none.
-__host__ inline int whole_lpb(int n, int64_t lines, size_t elem, int pin) {
+// Lines per block.  `table` is the LDS that all lines of one colour of every
+// system of the launch take together.  Where it fits the device in one round
+// (four blocks per CU), blocks are sized for two per CU: fewer would leave CUs
+// with one more block than others, more only share them (64^3 10.2 us a phase
+// with five lines a block, 13.2 with three).  Else the blocks' shares are even
+// over the fewest rounds that hold it: a round more costs a whole load, chain
+// and store (nine 64^3 systems 45 us a phase with five lines a block, four
+// rounds, 34 us with ten, two rounds).  pin: mfix_leq_set_line_block's value, 0
+// = none.
+__host__ inline int whole_lpb(int n, double table, size_t elem, int pin) {
+    const double line = 4.0 * whole_stride(n) * (double)elem;
     const int64_t rows = kWholeRows / n;
-    int64_t lpb = (kWholeLdsTarget / (int64_t)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
-    const int64_t spread = (lines + 511) / 512;
-    if (spread < lpb) lpb = spread;
+    const double rounds = std::ceil(table / (4.0 * kNumCus * kWholeLdsTarget));
+    int64_t lpb = (int64_t)std::ceil(table / ((rounds > 1.0 ? 4.0 * rounds : 2.0) * kNumCus) / line);
+    const int64_t most = (kWholeLdsTarget / (int64_t)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    if (lpb > most) lpb = most;
     if (pin > 0) lpb = pin;
     if (lpb > rows) lpb = rows;
     if (lpb > kWholeLines) lpb = kWholeLines;

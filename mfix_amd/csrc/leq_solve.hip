@@ -364,11 +364,18 @@ static void launch_line_factor(dim3 gs, int lds, hipStream_t s, const Sys<double
 // the blocks a colour takes.
 static int line_kernel(int n) { return whole_fits(n) ? LINE_WHOLE : LINE_LONG; }
 static int64_t colour_lines(const LineGeom &L) { return ((int64_t)L.nu * L.nv + 1) / 2; }
+// LDS of a colour of the grid's lines (k_line_whole).
 template <typename T>
-static int lines_of_block(const DGrid &g) {
+static double colour_lds(const DGrid &g) {
+    const LineGeom L = line_geom(g, AX_J);
+    return line_kernel(L.n) == LINE_LONG ? 0.0 : (double)colour_lines(L) * 4.0 * whole_stride(L.n) * sizeof(T);
+}
+// table: that of every system of the launch (0: this grid's alone)
+template <typename T>
+static int lines_of_block(const DGrid &g, double table = 0.0) {
     const LineGeom L = line_geom(g, AX_J);
     if (line_kernel(L.n) == LINE_LONG) return kLongLpb;
-    return whole_lpb(L.n, colour_lines(L), sizeof(T),
+    return whole_lpb(L.n, table > 0.0 ? table : colour_lds<T>(g), sizeof(T),
                      ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block);
 }
 template <typename T>
@@ -524,7 +531,7 @@ void sys_carve(Sys<T> &S, const SysDesc &d, const Part &P, char *base) {
         S.ld = S.line_scratch + n3;
         S.lu = S.line_scratch + 2 * n3;
         S.lu2 = S.line_scratch + 3 * n3;
-        S.lpb = lines_of_block<T>(d.g);
+        S.lpb = lines_of_block<T>(d.g, d.line_lds);
     }
     if (mixed) {
         S.a = (const T *)take(8 * n3 * sizeof(float));
@@ -1197,6 +1204,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<Part> parts((size_t)nsys);
     std::vector<size_t> offs((size_t)nsys);
     size_t total = 0;
+    double line_lds = 0.0;
     const int bs = 256;
     for (int q = 0; q < nsys; ++q) {
         const mfix_leq_batch_item &it = items[q];
@@ -1220,6 +1228,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
         descs[q].seed = it.noise_seed;
         const Shape sh = C.shape_for(g.n3, it.mixed != 0);
         parts[q] = make_part(g.n3, bs, sh.bs == bs ? sh.cpt : 1);
+        if (pc == PC_LINE && !it.mixed) line_lds += colour_lds<double>(g);
         offs[q] = total;
         total += sys_bytes(g, parts[q], pc, it.mixed != 0);
     }
@@ -1236,6 +1245,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<std::pair<int, int>> where((size_t)nsys);  // (precision, row)
     std::vector<int> ids64, ids32;
     for (int q = 0; q < nsys; ++q) {
+        descs[q].line_lds = items[q].mixed ? 0.0 : line_lds;
         char *base = (char *)C.bws.ptr + offs[q];
         if (items[q].mixed) {
             G32.sys.emplace_back();
