@@ -331,22 +331,6 @@ __device__ __forceinline__ bool resid_row_vals(const DGrid &g, int kind, double 
     return true;
 }
 
-// resid_row_vals with the row, B and VAR loaded here (PP reads only B).
-template <typename PA, typename PV, typename PF>
-__device__ __forceinline__ bool resid_row(const DGrid &g, int kind, double tol, const double *ep_s, double dil_ep_s,
-                                          PA a, PA b, PV var, PF flag, int64_t c, double &num1, double &den1) {
-    if (c >= g.n3 || !is_interior(g, c) || !fluid_at(flag[c])) return false;
-    double ar[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double vc = 0.0;
-    if (kind != RESID_PP) {
-        const int64_t n3 = g.n3;
-#pragma unroll
-        for (int p = 0; p < 7; ++p) ar[p] = a[p * n3 + c];
-        vc = var[c];
-    }
-    return resid_row_vals(g, kind, tol, ep_s, dil_ep_s, ar, b[c], vc, var, flag, c, num1, den1);
-}
-
 // The larger residual candidate (value, 0-based cell); equal values keep
 // the first cell, as the reference's scan with a strict '>' does.
 __device__ __forceinline__ void resid_better(double &v, double &i, double ov, double oi) {
