@@ -73,12 +73,14 @@ int rb_passes(const Sweep &sw, bool do_k);
 // R/S passes are swept one by one (line_seq).
 struct MapSet {
     std::vector<int> ids;
+    std::vector<int> streams[kMaxRPasses];  // lmap[LINE_STREAM][pass]: each system's entries, a launch each
     std::vector<int2> smap, fmap, umap, lmap[kLineKernels][kMaxRPasses];
     // FP32 tables: red-black passes of the several-lanes-per-line kernel,
     // one map per kernel variant (line length class) and pass
     std::vector<int2> pmap[kPcrVariants][kMaxRPasses];
     int nlpass = 0;
     int whole_lds = 0;            // LDS bytes of a k_line_whole launch (the largest of its systems)
+    int stream_lds = 0;           // of a k_line_stream launch
     std::vector<int> line_seq;
     double cells = 0.0;           // sum of N3 over ids (timing bytes)
     double k1_bytes = 0.0;        // algorithmic bytes of one first-stencil launch over all ids

@@ -46,6 +46,12 @@ constexpr int kWholeElems = 6, kWholeRows = kWholeThreads * kWholeElems;
 constexpr int kWholeLdsTarget = 160 * 1024 / 4 - 2048;
 constexpr int kWholeLines = 64;  // one lane of the solving wave per line
 
+// k_line_stream: two blocks per CU, one wave of each solving, the other
+// threads holding rows.
+constexpr int kStreamThreads = 512, kStreamLoaders = kStreamThreads - 64, kStreamElems = 5,
+              kStreamRows = kStreamLoaders * kStreamElems, kStreamBlocks = 2 * kNumCus,
+              kStreamLdsTarget = 160 * 1024 / 2 - 3072;
+
 // A line holds whole_rows rows (its own and up to three identity rows, so that
 // the chains take four rows a step) and lines sit an odd number of 16-byte
 // units apart: the solving lanes (one line each, the same two rows) and the
@@ -72,15 +78,39 @@ __host__ __device__ constexpr int whole_elems(int n, int lpb) {
 // = none.
 __host__ inline int whole_lpb(int n, double table, size_t elem, int pin) {
     const double line = 4.0 * whole_stride(n) * (double)elem;
-    const int64_t rows = kWholeRows / n;
     const double rounds = std::ceil(table / (4.0 * kNumCus * kWholeLdsTarget));
     int64_t lpb = (int64_t)std::ceil(table / ((rounds > 1.0 ? 4.0 * rounds : 2.0) * kNumCus) / line);
     const int64_t most = (kWholeLdsTarget / (int64_t)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    const int64_t rows = kWholeRows / n;
     if (lpb > most) lpb = most;
     if (pin > 0) lpb = pin;
     if (lpb > rows) lpb = rows;
     if (lpb > kWholeLines) lpb = kWholeLines;
     return lpb < 1 ? 1 : (int)lpb;
+}
+
+// Whether the lines of a system, `lds` bytes a colour in all, stream: they
+// take more than one round of k_line_whole's blocks.
+__host__ inline bool line_streams(int n, double lds, int64_t cells) {
+    return lds > 4.0 * kNumCus * kWholeLdsTarget && n <= kWholeRows && cells < (1ll << 29);
+}
+// Entries of a colour of `lines` lines then: the fewest a block, of lines that
+// it holds.
+__host__ inline int64_t stream_entries(int n, int64_t lines) {
+    int64_t most = (kStreamLdsTarget / 8 - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    if (most > kStreamRows / n) most = kStreamRows / n;
+    if (most > kWholeLines) most = kWholeLines;
+    return (lines + kStreamBlocks * most - 1) / (kStreamBlocks * most) * kStreamBlocks;
+}
+// Lines of entry j of a colour: [first(j), first(j + 1)), where first(j) = j
+// step / 2^32.  step = lines / entries, rounded up, shares them evenly (the last
+// entry's end is the last line: entries < 2^32); a whole number of lines is exact.
+__host__ inline uint64_t entry_step(int64_t lines, int64_t entries) {
+    const unsigned __int128 l = (unsigned __int128)lines << 32;
+    return (uint64_t)((l + (uint64_t)entries - 1) / (uint64_t)entries);
+}
+__host__ __device__ __forceinline__ int64_t entry_first(uint64_t step, int j) {
+    return (int64_t)(((unsigned __int128)step * (uint64_t)j) >> 32);
 }
 
 // The ranges in which the corrected quotient is the correctly rounded one: no
@@ -115,11 +145,13 @@ struct WholeLines {
     uint32_t c0[kWholeLines], im[kWholeLines], ip[kWholeLines], km[kWholeLines], kp[kWholeLines];
     int n;
 };
-__device__ __forceinline__ void whole_lines(const DGrid &g, int lpb, int64_t first, int param, WholeLines &w) {
+__device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j, int param, WholeLines &w) {
     const int l = threadIdx.x;
     if (l < 64) {
         int u = 0, v = 0;
-        const bool ok = l < lpb && color_line(g.ni, g.nk, g.do_k ? 1 : 0, param, first + l, u, v);
+        const int64_t first = entry_first(step, j);
+        const bool ok = l < entry_first(step, j + 1) - first &&
+                        color_line(g.ni, g.nk, g.do_k ? 1 : 0, param, first + l, u, v);
         const uint32_t c1 = (uint32_t)g.c1, c2 = (uint32_t)g.c2;
         if (ok) {
             w.c0[l] = (uint32_t)u * c1 + (uint32_t)v * c2;
@@ -393,21 +425,19 @@ static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<
     if (st->done) return;
     const DGrid &g = S.g;
     const int n = g.nj, ls = whole_stride(n);
-    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, (int)blockIdx.y, w);
+    whole_lines(g, S.lstep, e.y, (int)blockIdx.y, w);
     const int nl = w.n, tot = nl * n;
     double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ D = F + S.lpb * ls,
                          *__restrict__ U = D + S.lpb * ls, *__restrict__ V = U + S.lpb * ls;
     const int64_t n3 = g.n3;
     const gptr<const double> a = to_global(S.a);
     auto load = [&]() {
-#pragma unroll
-        for (int k0 = 0; k0 < kWholeElems; k0 += 3) {
-            if (k0 * kWholeThreads >= tot) break;
+        for (int xs = threadIdx.x; xs < tot; xs += 3 * kWholeThreads) {
             double dl[3], d[3], du[3];
             int o[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
+                const int x0 = xs + k * kWholeThreads;
                 const int x = x0 < tot ? x0 : tot - 1;  // (past the end: the last row again)
                 const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n;
                 const uint32_t c = w.c0[l] + (uint32_t)q;
@@ -503,7 +533,7 @@ static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<
     for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
         const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
         const uint32_t c = w.c0[l] + (uint32_t)q;
-        lf[c] = F[at];
+        lf[c] = any && x == 0 ? kSwapUp : F[at];  // (the block's mark: a first row has no multiplier)
         ld[c] = D[at];
         if (any) {
             lu[c] = U[at];
@@ -580,6 +610,55 @@ struct WholeRow {
     }
 };
 
+// DGTSV itself on the block's lines.
+template <typename T>
+__device__ __forceinline__ WholeArrays<T> whole_arrays(const Sys<T> &S, int which) {
+    const gptr<const T> a = to_global(S.a);
+    const int64_t n3 = S.g.n3;
+    WholeArrays<T> A;
+    A.km = a;
+    A.im = a + 2 * n3;
+    A.ip = a + 4 * n3;
+    A.jp = a + 5 * n3;
+    A.kp = a + 6 * n3;
+    A.bm = to_global((const T *)(which == 0 ? S.p : S.s));
+    A.var = to_global(which == 0 ? S.phat : S.shat);
+    A.f = a + n3;
+    A.d = a + (int64_t)DiagPlane<T>::value * n3;
+    return A;
+}
+template <typename T, int NT>
+__device__ void whole_general(const Sys<T> &S, const WholeLines &w, int *linfo, int which) {
+    extern __shared__ __align__(16) char whole_lds[];
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n), nl = w.n, tot = nl * n, do_k = g.do_k;
+    T *__restrict__ F = (T *)whole_lds + kWholeFront, *__restrict__ B = F + S.lpb * ls, *__restrict__ U = B + S.lpb * ls,
+                    *__restrict__ D = U + S.lpb * ls;
+    const WholeArrays<T> A = whole_arrays(S, which);
+    auto line_of = [&](int x) { return (int)div_by((uint32_t)x, g.mnj, g.snj); };
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += NT) {
+        const int l = line_of(x), q = x - l * n, at = l * ls + q;
+        WholeRow<T> r;
+        r.load(A, w, l, w.c0[l] + (uint32_t)q);
+        F[at] = q > 0 ? r.f : (T)0;
+        B[at] = r.rhs(do_k);
+        U[at] = q < n - 1 ? r.u : (T)0;
+        D[at] = r.d;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) {
+        const int ol = threadIdx.x * ls;
+        linfo[threadIdx.x] = whole_dgtsv(F + ol, B + ol, U + ol, D + ol, n);
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += NT) {
+        const int l = line_of(x), q = x - l * n;
+        // a line whose elimination hit a zero pivot keeps its values (leqsol_mod.f:910-914)
+        if (!linfo[l]) A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+    }
+}
+
 // One colour phase: block e takes lines [e.y*S.lpb, +S.lpb) of colour
 // `param` (color_line).  which = 0 preconditions P into Phat, 1 S into Shat.
 // FP32 tables (lines longer than the k_line_pcr_sys variants hold) always run
@@ -599,23 +678,14 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
     const DGrid &g = S.g;
     const int n = g.nj, ls = whole_stride(n), do_k = g.do_k;
     const int rows = whole_rows(n);
-    whole_lines(g, S.lpb, (int64_t)e.y * S.lpb, param, w);
+    whole_lines(g, S.lstep, e.y, param, w);
     const int nl = w.n, tot = nl * n;
     // right-hand side (then the solution), upper coupling, and: multipliers
     // (then the eliminated diagonal) and its reciprocals, or DL (then the
     // second super-diagonal) and A0
     T *__restrict__ F = (T *)whole_lds + kWholeFront, *__restrict__ B = F + S.lpb * ls, *__restrict__ U = B + S.lpb * ls,
                     *__restrict__ D = U + S.lpb * ls;
-    const int64_t n3 = g.n3;
-    const gptr<const T> a = to_global(S.a);
-    WholeArrays<T> A;
-    A.km = a;
-    A.im = a + 2 * n3;
-    A.ip = a + 4 * n3;
-    A.jp = a + 5 * n3;
-    A.kp = a + 6 * n3;
-    A.bm = to_global((const T *)(which == 0 ? S.p : S.s));
-    A.var = to_global(which == 0 ? S.phat : S.shat);
+    WholeArrays<T> A = whole_arrays(S, which);
     // (a line's rows are consecutive elements: element x is row x % n of line x / n)
     auto line_of = [&](int x) { return (int)div_by((uint32_t)x, g.mnj, g.snj); };
     if constexpr (sizeof(T) == sizeof(double)) {
@@ -629,7 +699,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             for (int k0 = 0; k0 < kWholeElems; k0 += K) {
                 if (k0 * kWholeThreads >= tot) break;
                 WholeRow<T> r[K];
-                bool last[K];
+                bool first[K], last[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
@@ -637,11 +707,12 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
                     const int l = line_of(x), q = x - l * n;
                     o[k0 + k] = l * ls + q;
                     r[k].load(A, w, l, w.c0[l] + (uint32_t)q);
+                    first[k] = q == 0;
                     last[k] = q == n - 1;
                 }
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    F[o[k0 + k]] = r[k].f;  // (0 on the first row)
+                    F[o[k0 + k]] = first[k] ? (T)0 : r[k].f;
                     any |= swapped(r[k].f);
                     B[o[k0 + k]] = r[k].rhs(do_k);
                     U[o[k0 + k]] = last[k] ? (T)0 : r[k].u;
@@ -703,29 +774,270 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             }
         }
     }
-    // DGTSV itself
-    A.f = a + n3;
-    A.d = a + (int64_t)DiagPlane<T>::value * n3;
-    __syncthreads();
-    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
-        const int l = line_of(x), q = x - l * n, at = l * ls + q;
-        WholeRow<T> r;
-        r.load(A, w, l, w.c0[l] + (uint32_t)q);
-        F[at] = q > 0 ? r.f : (T)0;
-        B[at] = r.rhs(do_k);
-        U[at] = q < n - 1 ? r.u : (T)0;
-        D[at] = r.d;
+    whole_general<T, kWholeThreads>(S, w, linfo, which);
+}
+
+// The same phase of a system of more than one round of blocks, its lines
+// streamed through kStreamBlocks blocks: block b takes the map entries b,
+// b + gridDim.x, ...  One wave solves; the others read the next entry's rows
+// into registers meanwhile (right-hand side, multiplier, upper coupling,
+// diagonal, and the second super-diagonal where rows were interchanged).
+// What bounded k_line_whole there was not the bytes: an LDS instruction costs a
+// CU about 11 cycles whatever its active lanes, so four solving waves a CU of
+// four lines each took twice as long over their chains as one does alone, and
+// a block's loads, chain and store came one after the other.  With two solving
+// waves of eight lines the chains fit beside the loads, and a phase moves what
+// it moves (a fifth more than the arrays: the other colour's values twice) at
+// 4.2 of the 5.1 TB/s of a copy: 256^3 233 -> 201 us, 170^3 71 -> 59 us,
+// 150x201x180 76 -> 69 us.  Non-temporal loads of the arrays read once: 195 us
+// at 256^3, but 48 for 42 us at 200x100x200, whose arrays the last-level cache
+// holds.
+// Start cell and I/K neighbour offsets of line `lane` of a block, in every wave.
+struct StreamLines {
+    uint32_t c0, im, ip, km, kp;
+    int n;
+    __device__ __forceinline__ void set(const DGrid &g, uint64_t step, int j, int param, int lane) {
+        int u = 0, v = 0;
+        const int64_t first = entry_first(step, j);
+        const bool ok = lane < entry_first(step, j + 1) - first &&
+                        color_line(g.ni, g.nk, g.do_k ? 1 : 0, param, first + lane, u, v);
+        const uint32_t c1 = (uint32_t)g.c1, c2 = (uint32_t)g.c2;
+        c0 = ok ? (uint32_t)u * c1 + (uint32_t)v * c2 : 0u;
+        im = (uint32_t)(nb_minus(u, g.ni, g.cyc_x) - u) * c1;
+        ip = (uint32_t)(nb_plus(u, g.ni, g.cyc_x) - u) * c1;
+        km = g.do_k ? (uint32_t)(nb_minus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
+        kp = g.do_k ? (uint32_t)(nb_plus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
+        n = __popcll(__ballot(ok));
     }
+    static __device__ __forceinline__ uint32_t of(uint32_t v, int l) { return (uint32_t)__shfl((int)v, l, 64); }
+};
+
+static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const Sys<double> *__restrict__ sys,
+                                                                         const int2 *__restrict__ map, int nmap,
+                                                                         int param, int which) {
+    extern __shared__ __align__(16) char whole_lds[];
+    __shared__ WholeLines w;
+    __shared__ int linfo[kWholeLines];
+    __shared__ int redo;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // another solving wave in each of the blocks that share a CU (every 256th)
+    const int solver = (blockIdx.x >> 8) & 1;
+    const int lt = (wave < solver ? wave : wave - 1) * 64 + lane;
+    const int step = (int)gridDim.x;
+    int it = blockIdx.x;
+    int2 e = map[it];
+    if (e.x < 0) return;
+    const int id = e.x;
+    const Sys<double> &S = sys[id];
+    auto *__restrict__ st = to_global(S.st);
+    if (st->done || (which == 1 && st->s_exit)) return;
+    if (threadIdx.x == 0) redo = st->line_general;
     __syncthreads();
-    if ((int)threadIdx.x < nl) {
-        const int ol = threadIdx.x * ls;
-        linfo[threadIdx.x] = whole_dgtsv(F + ol, B + ol, U + ol, D + ol, n);
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n), do_k = g.do_k, rows = whole_rows(n), lpb = S.lpb;
+    double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ B = F + lpb * ls,
+                         *__restrict__ U = B + lpb * ls, *__restrict__ D = U + lpb * ls;
+    if (!redo) {
+        WholeArrays<double> A = whole_arrays(S, which);
+        A.f = to_global((const double *)S.lf);
+        A.d = to_global((const double *)S.ld);
+        const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
+        // rows lt + k kStreamLoaders of the block's: row q of line l
+        double b[kStreamElems], f[kStreamElems], u[kStreamElems], v[kStreamElems], d[kStreamElems];
+        int lq[kStreamElems];
+#pragma unroll
+        for (int k = 0; k < kStreamElems; ++k) {
+            const int x0 = lt + k * kStreamLoaders, x = x0 < lpb * n ? x0 : lpb * n - 1;
+            const int l = (int)div_by((uint32_t)x, g.mnj, g.snj);
+            lq[k] = l << 16 | (x - l * n);
+        }
+        StreamLines L;
+        int tot = 0;
+        // (opaque: what is formed from lq is formed again in each step and
+        // not held in registers over the loop)
+        auto fresh = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k) asm volatile("" : "+v"(lq[k]));
+        };
+        auto at = [&](int k) __attribute__((always_inline)) { return (lq[k] >> 16) * ls + (lq[k] & 0xffff); };
+        auto here = [&](int k) __attribute__((always_inline)) { return lt + k * kStreamLoaders < tot; };
+        // byte offset of its cell (a row past the entry's last: a row of
+        // line 0, not used)
+        auto cell = [&](int k) __attribute__((always_inline)) {
+            const int l = lq[k] >> 16;
+            return 8u * (StreamLines::of(L.c0, l < L.n ? l : 0) + (uint32_t)(lq[k] & 0xffff));
+        };
+        auto ld = [](gptr<const double> p, uint32_t o) __attribute__((always_inline)) {
+            return *(gptr<const double>)((gptr<const char>)p + o);
+        };
+        auto rhs2 = [&](int k0) __attribute__((always_inline)) {
+            if (k0 * kStreamLoaders >= L.n * n) return;
+            double bb[2], m[2][4], y[2][4];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (k0 + k >= kStreamElems) break;
+                const int l0 = lq[k0 + k] >> 16, l = l0 < L.n ? l0 : 0;
+                const uint32_t c = cell(k0 + k);
+                bb[k] = ld(A.bm, c);
+                m[k][0] = ld(A.im, c);
+                m[k][1] = ld(A.ip, c);
+                m[k][2] = ld(A.km, c);  // (in 2-D the K offsets are 0: in bounds, not used)
+                m[k][3] = ld(A.kp, c);
+                y[k][0] = ld(A.var, c + 8u * StreamLines::of(L.im, l));
+                y[k][1] = ld(A.var, c + 8u * StreamLines::of(L.ip, l));
+                y[k][2] = ld(A.var, c + 8u * StreamLines::of(L.km, l));
+                y[k][3] = ld(A.var, c + 8u * StreamLines::of(L.kp, l));
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (k0 + k >= kStreamElems) break;
+                const double two = bb[k] - m[k][0] * y[k][0] - m[k][1] * y[k][1];
+                b[k0 + k] = do_k ? two - m[k][2] * y[k][2] - m[k][3] * y[k][3] : two;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto factors = [&](int sw) __attribute__((always_inline)) {
+            const gptr<const double> up = sw ? lu : A.jp;
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k) {
+                if (k * kStreamLoaders >= L.n * n) break;
+                const uint32_t c = cell(k);
+                f[k] = ld(A.f, c);
+                d[k] = ld(A.d, c);
+                u[k] = ld(up, c);
+                if (sw) v[k] = ld(lu2, c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto mark = [&]() __attribute__((always_inline)) { return ld(A.f, 8u * StreamLines::of(L.c0, 0)); };  // (in every wave alike)
+        auto marked = [](double f) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)swapped(f)); };
+        // (both loops below take the same entries and meet at the same four
+        // barriers an entry; apart, the solving wave's chains and the others'
+        // rows do not share registers)
+        auto next = [&]() __attribute__((always_inline)) {
+            return it + step < nmap ? map[it + step] : make_int2(-1, 0);
+        };
+        int2 en = next();
+        L.set(g, S.lstep, e.y, param, lane);
+        double mk = mark();
+        if (wave == solver) {
+            for (;;) {
+                if (e.y == 0 && lane == 0) st->line_launches += 1;  // (timing: working launches)
+                const bool more = en.x == id, mine = lane < L.n;
+                const int swp = marked(mk), ol = lane * ls;
+                if (more) L.set(g, S.lstep, en.y, param, lane);
+                it += step;
+                e = en;
+                if (more) en = next();
+                if (more) mk = mark();
+                __syncthreads();  // the rows are there
+                if (mine) {
+                    if (swp) whole_forward_swap(F + ol, B + ol, rows);
+                    else whole_forward(F + ol, B + ol, rows);
+                }
+                __syncthreads();  // forward pass done
+                __syncthreads();  // the diagonals are there
+                if (mine) {
+                    if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
+                    else whole_back(B + ol, U + ol, D + ol, F + ol, rows);
+                }
+                __syncthreads();  // solved
+                if (!more) break;
+            }
+        } else {
+            int swn = marked(mk);
+            factors(swn);
+#pragma unroll
+            for (int k0 = 0; k0 < kStreamElems; k0 += 2) rhs2(k0);
+            for (;;) {
+                const bool more = en.x == id;
+                const int nl = L.n, swp = swn;
+                const uint32_t c0 = L.c0;  // start cells of the entry being solved
+                tot = nl * n;
+                fresh();
+#pragma unroll
+                for (int k = 0; k < kStreamElems; ++k) {
+                    if (k * kStreamLoaders >= tot) break;
+                    if (!here(k)) continue;
+                    const int o = at(k), q = lq[k] & 0xffff;
+                    F[o] = q > 0 ? f[k] : 0.0;
+                    B[o] = b[k];
+                    U[o] = q < n - 1 ? u[k] : 0.0;
+                    D[o] = swp ? v[k] : d[k];
+                }
+                for (int x = lt; x < 4 * nl; x += kStreamLoaders) {
+                    const int q = n + (x & 3), o = (x >> 2) * ls + q;
+                    if (q < rows) {  // identity rows
+                        F[o] = B[o] = U[o] = 0.0;
+                        D[o] = 1.0;
+                    }
+                }
+                if (more) L.set(g, S.lstep, en.y, param, lane);
+                it += step;
+                e = en;
+                if (more) en = next();
+                __syncthreads();  // the rows are there
+                if (more) mk = mark();
+                if (!swp) {
+#pragma unroll
+                    for (int k = 0; k < kStreamElems; ++k) d[k] = refined_rcp(d[k]);
+                }
+                if (more) {
+                    fresh();
+                    rhs2(0);
+                    fresh();
+                    rhs2(2);
+                    swn = marked(mk);
+                }
+                __syncthreads();  // forward pass done
+                fresh();
+#pragma unroll
+                for (int k = 0; k < kStreamElems; ++k) {
+                    if (k * kStreamLoaders >= tot) break;
+                    if (here(k)) F[at(k)] = d[k];
+                }
+                for (int x = lt; x < 4 * nl; x += kStreamLoaders) {
+                    const int q = n + (x & 3);
+                    if (q < rows) F[(x >> 2) * ls + q] = 1.0;
+                }
+                __syncthreads();  // the diagonals are there
+                if (more) {
+                    fresh();
+                    factors(swn);
+                    fresh();
+                    rhs2(4);
+                }
+                fresh();
+                uint32_t c[kStreamElems];
+#pragma unroll
+                for (int k = 0; k < kStreamElems; ++k)
+                    c[k] = 8u * (StreamLines::of(c0, lq[k] >> 16) + (uint32_t)(lq[k] & 0xffff));
+                __syncthreads();  // solved
+                fresh();
+                int bad = 0;
+#pragma unroll
+                for (int k = 0; k < kStreamElems; ++k) {
+                    if (k * kStreamLoaders >= tot) break;
+                    if (!here(k)) continue;
+                    const double x = B[at(k)];
+                    bad |= !solution_in_range(x);
+                    *(gptr<double>)((gptr<char>)A.var + c[k]) = x;
+                }
+                if (bad) redo = 1;
+                if (!more) break;
+            }
+        }
+        __syncthreads();
+        if (!redo) return;
     }
-    __syncthreads();
-    for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
-        const int l = line_of(x), q = x - l * n;
-        // a line whose elimination hit a zero pivot keeps its values (leqsol_mod.f:910-914)
-        if (!linfo[l]) A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+    // a pivot or a value out of range: DGTSV itself, on every entry of this
+    // block (their inputs, the other colour's values, are as they were)
+    for (it = blockIdx.x; it < nmap; it += step) {
+        e = map[it];
+        if (e.x != id) break;
+        __syncthreads();
+        whole_lines(g, S.lstep, e.y, param, w);
+        whole_general<double, kStreamThreads>(S, w, linfo, which);
     }
 }
 

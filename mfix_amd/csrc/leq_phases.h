@@ -75,7 +75,10 @@ struct Sys {
     double *y;             // mixed: FP64 correction accumulator since the last reliable update
     T *line_scratch;       // 4 planes of DGTSV scratch (LINE)
     T *lf, *ld, *lu, *lu2; // LINE, FP64: every line's elimination (k_line_factor), the four planes of line_scratch
-    int lpb;               // LINE: lines per block of k_line_whole
+    int lk;                // LINE: the red-black kernel (LineKernel)
+    int lpb;               // LINE: lines per block of k_line_whole or k_line_stream, at most
+    int64_t lent;          // map entries a colour
+    uint64_t lstep;        // lines per entry times 2^32 (entry_first)
     SolverState *st;
     double *partials;      // kMaxPartials * P.nblk
     double *a64, *b64, *xa, *xb, *r64;
@@ -1087,8 +1090,8 @@ constexpr int kLongLpb = 64;     // its lines per block
 
 // Red-black line kernels with one lane per line: k_line_whole (whole lines in
 // LDS) and, for lines that do not fit there, k_line_color_sys.
-enum LineKernel : int { LINE_WHOLE = 0, LINE_LONG = 1 };
-constexpr int kLineKernels = 2;
+enum LineKernel : int { LINE_WHOLE = 0, LINE_LONG = 1, LINE_STREAM = 2 };
+constexpr int kLineKernels = 3;
 
 // Red-black line phase along J for the FP32 inner solve of the mixed path:
 // several lanes per line.  The FP64 kernel above must repeat DGTSV's

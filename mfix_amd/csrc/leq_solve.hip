@@ -350,6 +350,12 @@ int launch_msolve_line(const DGrid &g, const Shape &sh, const char *cmethod, con
 template <typename T>
 static void launch_line_color(int kernel, dim3 gs, int lds, hipStream_t s, const Sys<T> *tab, const int2 *mp,
                               int param, int which, std::pair<hipEvent_t, hipEvent_t> ev = {nullptr, nullptr}) {
+    if constexpr (sizeof(T) == sizeof(double))
+        if (kernel == LINE_STREAM) {  // (one system's entries)
+            launch_timed_lds(ev.first, ev.second, k_line_stream, dim3(std::min(gs.x, (unsigned)kStreamBlocks)),
+                             dim3(kStreamThreads), lds, s, tab, mp, (int)gs.x, param, which);
+            return;
+        }
     if (kernel == LINE_WHOLE)
         launch_timed_lds(ev.first, ev.second, k_line_whole<T>, gs, dim3(kWholeThreads), lds, s, tab, mp, param, which);
     else
@@ -360,23 +366,37 @@ static void launch_line_factor(dim3 gs, int lds, hipStream_t s, const Sys<double
     hipLaunchKernelGGL(k_line_factor, dim3(gs.x, 2), dim3(kWholeThreads), lds, s, tab, mp);
 }
 
-// The one-lane-per-line kernel for lines of n rows, its lines per block and
-// the blocks a colour takes.
-static int line_kernel(int n) { return whole_fits(n) ? LINE_WHOLE : LINE_LONG; }
+// The one-lane-per-line kernel of a system, its lines per block and the blocks
+// a colour takes.
 static int64_t colour_lines(const LineGeom &L) { return ((int64_t)L.nu * L.nv + 1) / 2; }
 // LDS of a colour of the grid's lines (k_line_whole).
 template <typename T>
 static double colour_lds(const DGrid &g) {
     const LineGeom L = line_geom(g, AX_J);
-    return line_kernel(L.n) == LINE_LONG ? 0.0 : (double)colour_lines(L) * 4.0 * whole_stride(L.n) * sizeof(T);
+    return whole_fits(L.n) ? (double)colour_lines(L) * 4.0 * whole_stride(L.n) * sizeof(T) : 0.0;
 }
-// table: that of every system of the launch (0: this grid's alone)
+// table: LDS of a colour of every system of the launch (0: this grid's alone)
 template <typename T>
-static int lines_of_block(const DGrid &g, double table = 0.0) {
+static void set_line_kernel(Sys<T> &S, double table = 0.0) {
+    const DGrid &g = S.g;
     const LineGeom L = line_geom(g, AX_J);
-    if (line_kernel(L.n) == LINE_LONG) return kLongLpb;
-    return whole_lpb(L.n, table > 0.0 ? table : colour_lds<T>(g), sizeof(T),
-                     ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block);
+    const int pin = ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block;
+    const double own = colour_lds<T>(g);
+    if (!whole_fits(L.n)) {
+        S.lk = LINE_LONG;
+        S.lpb = kLongLpb;
+    } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, own, g.n3)) {
+        S.lk = LINE_STREAM;
+        S.lent = stream_entries(L.n, colour_lines(L));
+        S.lstep = entry_step(colour_lines(L), S.lent);
+        S.lpb = (int)((S.lstep + 0xffffffffull) >> 32);
+        return;
+    } else {
+        S.lk = LINE_WHOLE;
+        S.lpb = whole_lpb(L.n, table > 0.0 ? table : own, sizeof(T), pin);
+    }
+    S.lent = (colour_lines(L) + S.lpb - 1) / S.lpb;
+    S.lstep = (uint64_t)S.lpb << 32;
 }
 template <typename T>
 static int whole_lds_bytes(const Sys<T> &S) {
@@ -398,16 +418,16 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     Context &C = ctx();
     const LineGeom L = line_geom(g, AX_J);
     const int var = sizeof(T) == sizeof(float) ? line_pcr_variant(L.n) : -1;
-    const int lk = line_kernel(L.n);
-    const int lpb = var >= 0 ? line_pcr_lpb(var) : lines_of_block<T>(g);
-    const int64_t lb = (colour_lines(L) + lpb - 1) / lpb;
+    Sys<T> S = {};
+    S.g = g;
+    set_line_kernel(S);
+    const int lk = S.lk;
+    const int64_t lb = var >= 0 ? (colour_lines(L) + line_pcr_lpb(var) - 1) / line_pcr_lpb(var) : S.lent;
     const size_t o_st = align256(sizeof(Sys<T>));
     const size_t o_map = o_st + align256(sizeof(SolverState));
     int rc;
     if ((rc = C.line1.ensure(o_map + sizeof(int2) * (size_t)(lb + kNumXcd)))) return rc;
     char *base = (char *)C.line1.ptr;
-    Sys<T> S = {};
-    S.g = g;
     S.pc = PC_LINE;
     S.a = a;
     S.p = const_cast<T *>(r);
@@ -417,7 +437,6 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     S.ld = scratch + g.n3;
     S.lu = scratch + 2 * g.n3;
     S.lu2 = scratch + 3 * g.n3;
-    S.lpb = lpb;
     S.st = (SolverState *)(base + o_st);
     std::vector<int2> map;
     push_slab_map(map, 0, lb);
@@ -431,7 +450,7 @@ int run_msolve_line_rb(const DGrid &g, const char *cmethod, const T *a, const T 
     const int2 *mp = (const int2 *)(base + o_map);
     const dim3 gs((unsigned)map.size());
     if constexpr (sizeof(T) == sizeof(double))
-        if (np > 0 && lk == LINE_WHOLE) launch_line_factor(gs, whole_lds_bytes(S), s, tab, mp);
+        if (np > 0 && lk != LINE_LONG) launch_line_factor(gs, whole_lds_bytes(S), s, tab, mp);
     for (int q = 0; q < np; ++q)
         for (int param : {1, 0}) {
             const auto ev = pf.take(0.5 * (double)g.n3 * 13.0 * sizeof(T));
@@ -531,7 +550,7 @@ void sys_carve(Sys<T> &S, const SysDesc &d, const Part &P, char *base) {
         S.ld = S.line_scratch + n3;
         S.lu = S.line_scratch + 2 * n3;
         S.lu2 = S.line_scratch + 3 * n3;
-        S.lpb = lines_of_block<T>(d.g, d.line_lds);
+        set_line_kernel(S, d.line_lds);
     }
     if (mixed) {
         S.a = (const T *)take(8 * n3 * sizeof(float));
@@ -573,7 +592,8 @@ template <typename T>
 int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStream_t s, char *ext, size_t ext_cap) {
     std::vector<int2> smap, fmap, umap, lmap[kLineKernels][kMaxRPasses], pmap[kPcrVariants][kMaxRPasses];
     std::vector<int> seq;
-    int nlpass = 0, n_line = 0, n_fused = 0, lds = 0;
+    int nlpass = 0, n_line = 0, n_fused = 0, lds = 0, slds = 0;
+    std::vector<int> streams[kMaxRPasses];
     double cells = 0.0, k1 = 0.0;
     const double sa = sizeof(T), sv = sizeof(T);
     for (int id : ids) {
@@ -601,10 +621,14 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
                 // FP32 (the mixed path's inner solve): several lanes per line
                 // where the line fits a variant; FP64: DGTSV lane per line
                 const int var = sizeof(T) == sizeof(float) ? line_pcr_variant(L.n) : -1;
-                const int lk = line_kernel(L.n);
-                const int lpb = var >= 0 ? line_pcr_lpb(var) : S.lpb;
-                const int64_t lb = (colour_lines(L) + lpb - 1) / lpb;
+                const int lk = S.lk;
+                const int64_t lb =
+                    var >= 0 ? (colour_lines(L) + line_pcr_lpb(var) - 1) / line_pcr_lpb(var) : S.lent;
                 if (var < 0 && lk == LINE_WHOLE) lds = std::max(lds, whole_lds_bytes(S));
+                if (var < 0 && lk == LINE_STREAM) {
+                    slds = std::max(slds, whole_lds_bytes(S));
+                    for (int q = 0; q < np; ++q) streams[q].push_back((int)xcd_grid(lb));
+                }
                 // the same XCD slab order as the stream kernels: XCD x takes a
                 // contiguous run of line blocks, so the I/K neighbour lines its
                 // blocks read (the other colour's, about two blocks away along
@@ -618,11 +642,12 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
         }
     }
     bool same = M.ids == ids && M.smap.size() == smap.size() && M.fmap.size() == fmap.size() &&
-                M.nlpass == nlpass && M.whole_lds == lds && M.line_seq == seq && M.dev.ptr;
+                M.nlpass == nlpass && M.whole_lds == lds && M.stream_lds == slds && M.line_seq == seq && M.dev.ptr;
     if (same) same = !std::memcmp(M.smap.data(), smap.data(), smap.size() * sizeof(int2)) &&
                      !std::memcmp(M.fmap.data(), fmap.data(), fmap.size() * sizeof(int2)) &&
                      M.umap.size() == umap.size() &&
                      !std::memcmp(M.umap.data(), umap.data(), umap.size() * sizeof(int2));
+    for (int q = 0; q < kMaxRPasses; ++q) same = same && M.streams[q] == streams[q];
     for (int q = 0; q < kMaxRPasses && same; ++q) {
         for (int v = 0; v < kLineKernels && same; ++v)
             same = M.lmap[v][q].size() == lmap[v][q].size() &&
@@ -646,6 +671,8 @@ int build_maps(const Group<T> &G, const std::vector<int> &ids, MapSet &M, hipStr
     }
     M.nlpass = nlpass;
     M.whole_lds = lds;
+    M.stream_lds = slds;
+    for (int q = 0; q < kMaxRPasses; ++q) M.streams[q].swap(streams[q]);
     M.line_seq.swap(seq);
     // one device block: ids | smap | fmap | umap | lmap[kernel][pass] | pmap[variant][pass]
     std::vector<char> blob;
@@ -731,9 +758,10 @@ static void setup_bs(Group<T> &G, const MapSet &M, hipStream_t s) {
     hipLaunchKernelGGL((k_shadow<BS, T>), gs, blk, 0, s, G.d_sys, M.d_smap);
     finish<T, FIN_SHADOW, 1>(G, M, s);
     if constexpr (sizeof(T) == sizeof(double))
-        if (!M.lmap[LINE_WHOLE][0].empty())
-            launch_line_factor(dim3((unsigned)M.lmap[LINE_WHOLE][0].size()), M.whole_lds, s, G.d_sys,
-                               M.d_lmap[LINE_WHOLE][0]);
+        for (int v : {LINE_WHOLE, LINE_STREAM})
+            if (!M.lmap[v][0].empty())
+                launch_line_factor(dim3((unsigned)M.lmap[v][0].size()), v == LINE_STREAM ? M.stream_lds : M.whole_lds,
+                                   s, G.d_sys, M.d_lmap[v][0]);
 }
 
 template <typename T>
@@ -756,6 +784,16 @@ static void line_sweeps(const Group<T> &G, const MapSet &M, int which, hipStream
             // those of every LINE system of the table (a single solve: its own)
             for (int v = 0; v < kLineKernels; ++v) {
                 if (M.lmap[v][q].empty()) continue;
+                if (v == LINE_STREAM) {
+                    int at = 0;
+                    for (int n : M.streams[q]) {
+                        const auto ev = pf.take(0.5 * (double)G.sys[M.lmap[v][q][at].x].g.n3 * 13.0 * sizeof(T));
+                        launch_line_color<T>(v, dim3((unsigned)n), M.stream_lds, s, G.d_sys, M.d_lmap[v][q] + at, param,
+                                             which, ev);
+                        at += n;
+                    }
+                    continue;
+                }
                 const auto ev = pf.take(0.5 * M.cells * 13.0 * sizeof(T));
                 launch_line_color<T>(v, dim3((unsigned)M.lmap[v][q].size()), M.whole_lds, s, G.d_sys, M.d_lmap[v][q],
                                      param, which, ev);
@@ -866,7 +904,7 @@ static int line_launch_of(const Group<T> &G, int id) {
         const int var = line_pcr_variant(line_geom(S.g, AX_J).n);
         if (var >= 0) return 1 + kLineKernels + var;
     }
-    return 1 + line_kernel(S.g.nj);
+    return 1 + S.lk;
 }
 
 // Drop finished systems from a table's block maps once the running systems
@@ -1503,7 +1541,12 @@ int autotune(int imax, int jmax, int kmax, int mixed, Shape *best_out) {
     if (rc) return rc;
     if (best_out) {
         *best_out = best;
-        if (!best.lines_per_block) best_out->lines_per_block = lines_of_block<double>(g);
+        if (!best.lines_per_block) {
+            Sys<double> S = {};
+            S.g = g;
+            set_line_kernel(S);
+            best_out->lines_per_block = S.lpb;
+        }
     }
     return 0;
 }
