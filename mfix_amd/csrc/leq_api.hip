@@ -1,6 +1,9 @@
 // C ABI of the gfx950 LEQ_BICGS solver (include/mfix_leq.h).  Every entry
 // validates its arguments, selects the context's stream and calls the solver
 // engine (leq_solve.hip); none of them computes on the host.
+#include <sched.h>
+
+#include <thread>
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -58,6 +61,109 @@ std::vector<Deferred> &sweep_queue() {
     return q;
 }
 
+struct Span {
+    void *dev, *host;
+    size_t bytes;
+};
+
+int stage_ready(Stage &st) {
+    if (!st.mem) {
+        const hipError_t e = hipHostMalloc((void **)&st.mem, kStageSlots * kStageBytes, hipHostMallocDefault);
+        if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
+    }
+    for (hipEvent_t &ev : st.moved)
+        if (!ev) {
+            const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+            if (e != hipSuccess) return hip_fail(e, "hipEventCreate");
+        }
+    return 0;
+}
+
+void stage_free(Stage &st) {
+    if (st.mem) (void)hipHostFree(st.mem);
+    for (hipEvent_t ev : st.moved)
+        if (ev) (void)hipEventDestroy(ev);
+    st = Stage{};
+}
+
+hipError_t slot_free(hipEvent_t ev) {  // (an event that was never recorded is done)
+    hipError_t e;
+    while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
+    }
+    return e;
+}
+
+// n doubles (both ends 16-byte aligned), over the link: one end is pinned host memory.
+constexpr int kMoveBlocks = 64;
+__global__ void __launch_bounds__(256) k_move(const double *__restrict__ from, double *__restrict__ to, int n) {
+    const int m = n / 2, t = (int)(blockIdx.x * 256 + threadIdx.x);
+    for (int i = t; i < m; i += kMoveBlocks * 256) ((double2 *)to)[i] = ((const double2 *)from)[i];
+    if (t == 0 && (n & 1)) to[n - 1] = from[n - 1];
+}
+
+// Pageable arrays to the device (up) or back, in chunks through the pinned
+// slots, so that the link moves some while processors copy others: several,
+// where the process may run on several and the arrays are worth it, as one
+// copies slower than the link moves.  The host arrays are free (up) or filled
+// (down) when it returns.  STAGEFIG
+int staged_copy(const std::vector<Span> &spans, bool up, hipStream_t s) {
+    Context &C = ctx();
+    Stage &st = C.stage;
+    int rc;
+    if ((rc = stage_ready(st))) return rc;
+    struct Chunk {
+        char *dev, *host;
+        size_t bytes;
+    };
+    std::vector<Chunk> ch;
+    for (const Span &sp : spans)
+        for (size_t o = 0; o < sp.bytes; o += kStageBytes)
+            ch.push_back({(char *)sp.dev + o, (char *)sp.host + o, std::min(kStageBytes, sp.bytes - o)});
+    cpu_set_t cpus;
+    const int have = sched_getaffinity(0, sizeof(cpus), &cpus) ? 1 : CPU_COUNT(&cpus);
+    const int nw = ch.size() >= kStageSlots ? std::max(1, std::min(kStageWorkers, have)) : 1;
+    const size_t per = kStageSlots / nw;  // slots of a worker
+    hipError_t err[kStageWorkers] = {};
+    // worker w's chunks, in turn through its slots
+    auto work = [&](int w) {
+        const size_t n = (ch.size() + nw - 1 - w) / nw;
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < n + (up ? 0 : per) && e == hipSuccess; ++k) {
+            const size_t q = w * per + k % per;
+            char *slot = st.mem + q * kStageBytes;
+            e = slot_free(st.moved[q]);
+            if (e == hipSuccess && !up && k >= per) {
+                const Chunk &c = ch[w + (k - per) * nw];
+                std::memcpy(c.host, slot, c.bytes);
+            }
+            if (e != hipSuccess || k >= n) continue;
+            const Chunk &c = ch[w + k * nw];
+            if (up) std::memcpy(slot, c.host, c.bytes);
+            hipLaunchKernelGGL(k_move, dim3(kMoveBlocks), dim3(256), 0, s, (const double *)(up ? slot : c.dev),
+                               (double *)(up ? c.dev : slot), (int)(c.bytes / sizeof(double)));
+            e = hipEventRecord(st.moved[q], s);
+        }
+        err[w] = e;
+    };
+    std::vector<std::thread> others;
+    int started = 1;
+    try {
+        others.reserve(nw);
+        for (; started < nw; ++started)
+            others.emplace_back([&, w = started] {
+                err[w] = hipSetDevice(C.device);
+                if (err[w] == hipSuccess) work(w);
+            });
+    } catch (...) {  // (no thread to be had: the rest is done here)
+    }
+    work(0);
+    for (int w = started; w < nw; ++w) work(w);
+    for (std::thread &t : others) t.join();
+    for (hipError_t e : err)
+        if (e != hipSuccess) return hip_fail(e, up ? "host to device copy" : "device to host copy");
+    return 0;
+}
+
 int copy_sync(void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
     int rc;
     if ((rc = ctx().ensure_init())) return rc;
@@ -79,6 +185,7 @@ int mfix_leq_finalize(void) {
     C.release_all();
     if (C.host_state) (void)hipHostFree(C.host_state);
     if (C.host_count) (void)hipHostFree(C.host_count);
+    stage_free(C.stage);
     C.host_state = nullptr;
     C.host_count = nullptr;
     (void)hipStreamDestroy(C.stream);
@@ -194,10 +301,9 @@ int mfix_leq_bicgs(const char *vname, int vname_len, int vno, double *var, doubl
         return rc;
     double *da = (double *)C.d_a.ptr, *db = (double *)C.d_b.ptr, *dx = (double *)C.d_x.ptr;
     hipError_t e;
-    if ((e = hipMemcpyAsync(da, a_m, sizeof(double) * 7 * n3, hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(db, b_m, sizeof(double) * n3, hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(dx, var, sizeof(double) * n3, hipMemcpyHostToDevice, s)) != hipSuccess)
-        return hip_fail(e, "host to device copy");
+    const std::vector<Span> system = {
+        {da, a_m, sizeof(double) * 7 * n3}, {db, b_m, sizeof(double) * n3}, {dx, var, sizeof(double) * n3}};
+    if ((rc = staged_copy(system, true, s))) return rc;
     mfix_leq_opts o = {};
     o.write_back_scaled = 1;
     if (C.host_noise) {
@@ -211,13 +317,8 @@ int mfix_leq_bicgs(const char *vname, int vname_len, int vno, double *var, doubl
     mfix_leq_stats st = {};
     rc = solve_fp64(g, p, cm, tol, itmax, dx, da, db, &o, &st, s, C.grid.minimize_dotproducts, C.grid.icheck_bicgs);
     if (rc && rc != MFIX_LEQ_EDGTSV) return rc;
-    if ((e = hipMemcpyAsync(var, dx, sizeof(double) * n3, hipMemcpyDeviceToHost, s)) != hipSuccess)
-        return hip_fail(e, "device to host copy");
-    if (C.write_back_scaled) {
-        if ((e = hipMemcpyAsync(a_m, da, sizeof(double) * 7 * n3, hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipMemcpyAsync(b_m, db, sizeof(double) * n3, hipMemcpyDeviceToHost, s)) != hipSuccess)
-            return hip_fail(e, "device to host copy");
-    }
+    const int down = staged_copy(C.write_back_scaled ? system : std::vector<Span>{system[2]}, false, s);
+    if (down) return down;
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
     *ier = st.ier;
     if (vno >= 1 && vno <= 10) C.iter_tot[vno - 1] += st.iter_tot_increment;

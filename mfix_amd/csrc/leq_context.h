@@ -114,6 +114,15 @@ struct Group {
     void drop_graph();
 };
 
+// Pinned chunks through which the host-array entry moves pageable memory, made
+// on its first call and kept (kStageSlots kStageBytes in all).
+constexpr int kStageSlots = 8, kStageWorkers = 4;
+constexpr size_t kStageBytes = 1u << 20;
+struct Stage {
+    char *mem = nullptr;
+    hipEvent_t moved[kStageSlots] = {};  // the slot's last copy
+};
+
 struct Context {
     bool initialised = false;
     double mixed_delta = 0.0;      // mixed: reliable-update trigger, 0 = by size (mfix_leq_set_mixed_delta)
@@ -129,6 +138,7 @@ struct Context {
     DevBuf partials, state, misc, tmp;
     SolverState *host_state = nullptr;  // pinned mirrors of device states
     int *host_count = nullptr;          // pinned: kPollInts of the FP64 table, then of the FP32 table
+    Stage stage;
     int poll = 0;                       // number of the last poll issued
     Group<double> g64;             // single-solve tables
     Group<float> g32;
