@@ -281,8 +281,8 @@ int mfix_leq_set_shape(int imax, int jmax, int kmax, int mixed, int block_thread
                        int cells_per_thread);
 /* Pin the lines per block (64, 32 or 16; 0 = the default for the size) of
  * the red-black line kernel that LINE solves of this grid size and
- * precision use: each block solves that many J-lines of one colour, one
- * line per lane (the LEQ_MSOLVE/LEQ_IKSWEEP line solves,
+ * precision use: each block solves that many J-lines of one colour, or as
+ * many as it holds (the LEQ_MSOLVE/LEQ_IKSWEEP line solves,
  * model/leqsol_mod.f:851-921).  The results do not depend on it.  No
  * counterpart in the reference. */
 int mfix_leq_set_line_block(int imax, int jmax, int kmax, int mixed, int lines_per_block);

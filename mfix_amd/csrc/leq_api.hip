@@ -104,8 +104,12 @@ __global__ void __launch_bounds__(256) k_move(const double *__restrict__ from, d
 // Pageable arrays to the device (up) or back, in chunks through the pinned
 // slots, so that the link moves some while processors copy others: several,
 // where the process may run on several and the arrays are worth it, as one
-// copies slower than the link moves.  The host arrays are free (up) or filled
-// (down) when it returns.  STAGEFIG
+// copies slower than the link moves.  A kernel moves a chunk: the runtime's
+// asynchronous copies leave gaps of 18 us between chunks of 1 MiB.  The host
+// arrays are free (up) or filled (down) when it returns.  LEQ_BICGS on host
+// arrays of 64^3, 20.7 MB each way: 2376 us with the runtime's copies of
+// pageable memory (16 MB: 450 us up, 921 down, where the link takes 293), 1840
+// with them through the slots in one thread, 1590 so.
 int staged_copy(const std::vector<Span> &spans, bool up, hipStream_t s) {
     Context &C = ctx();
     Stage &st = C.stage;

@@ -784,27 +784,24 @@ __global__ void __launch_bounds__(kFinishBlock) k_finish_sys(const Sys<T> *__res
         fin_apply<F, NV>(st, tot, nullptr);
 }
 
-// Red-black line phase along J for every LINE system of a table (RSRS and
-// the 2-D R sweep).  Block b takes lines [map[b].y*LPB, +LPB) of colour
+// Red-black line phase along J (RSRS and the 2-D R sweep) of systems whose
+// lines are too long for whole lines in LDS (more than 1,536 rows; the others
+// take k_line_whole).  Block b takes lines [map[b].y*LPB, +LPB) of colour
 // `param` of system map[b].x, numbered densely by color_line, with five
-// waves: lane l < LPB of wave 0 runs DGTSV on line l (the operations and
-// order of solve_line, so the result is bit-identical); waves 1-4 feed it.
-// Lines along J are contiguous, so a loader wave reads rows in runs: a tile
-// is RT = 1024/LPB rows of every line, loader w takes the lines of quarter
-// w-1, and element k of its lane is row lane % RT of line (quarter) +
-// lane / RT + (LPB/16) k, each load instruction fetching LPB/16 lines x RT
-// contiguous rows (16 rows, 128 bytes of FP64, per line at 64 lines per
-// block); it forms the right-hand side (B minus the I/K neighbour terms,
-// whose offsets are constant along a J-line) and stages it in LDS, while
-// wave 0 eliminates the previous tile: one memory round trip per tile (16
-// rows at 64 lines per block, 32 at 32, 64 at 16).
+// waves: lane l of wave 0 runs DGTSV on line l (the operations and order of
+// solve_line, so the result is bit-identical); waves 1-4 feed it.  Lines along
+// J are contiguous, so a loader wave reads rows in runs: a tile is 16 rows of
+// every line, loader w takes the lines of quarter w-1, each load instruction
+// fetching 4 lines x 16 contiguous rows; it forms the right-hand side (B minus
+// the I/K neighbour terms, whose offsets are constant along a J-line) and
+// stages it in LDS, while wave 0 eliminates the previous tile: one memory
+// round trip per tile.
 // Finished rows go to scratch in [row][lane] order; for the back solve
 // waves 1-4 stage them in LDS in groups of 8 rows, two groups ahead, and
-// waves 1-2 write the solution out through LDS, coalesced.  Fewer lines per block give more blocks (128^3: 8,450 lines per
-// colour are 133 blocks of 64 but 265 of 32); the launch shape picks LPB
-// per grid size.  Four loaders of four elements each keep the kernel at two
-// blocks per CU (a loader with eight elements needs 256 registers, one
-// block per CU).  which = 0 preconditions P into Phat, 1 S into Shat.
+// waves 1-2 write the solution out through LDS, coalesced.  Four loaders of
+// four elements each keep the kernel at two blocks per CU (a loader with eight
+// elements needs 256 registers, one block per CU).  which = 0 preconditions P
+// into Phat, 1 S into Shat.
 template <typename T, int LPB>
 __global__ void __launch_bounds__(320) k_line_color_sys(const Sys<T> *__restrict__ sys, const int2 *__restrict__ map,
                                                         int param, int which) {

@@ -1,8 +1,7 @@
 """GPU: the host-array entry moves its arrays in chunks through pinned memory
 by one or several threads.  Grids of less than a chunk, of a chunk and a
 remainder, and of more chunks than slots give what the same solve on device
-arrays gives, bit for bit: solution, scaled matrix and right-hand side, and
-arrays that the caller keeps out of the write-back stay as they are."""
+arrays gives, bit for bit: solution, scaled matrix and right-hand side."""
 import os
 
 import numpy as np
@@ -21,7 +20,7 @@ def test_same_as_on_the_device(gpu, dims, cpus):
     da, db, dx = gpu.DeviceArray.from_host(a), gpu.DeviceArray.from_host(b), gpu.DeviceArray.from_host(np.zeros(b.size))
     gpu.bicgs_dev(dx, da, db, pc="LINE", tol=1e-8, itmax=20)
     x, aa, bb = np.zeros(b.size), a.copy(), b.copy()
-    before = os.sched_getaffinity(0)
+    before = os.sched_getaffinity(0)  # (one thread a processor that the process may use, up to four)
     if cpus:
         os.sched_setaffinity(0, set(sorted(before)[:cpus]))
     try:
