@@ -429,6 +429,14 @@ __device__ __forceinline__ double row_down(double v) {
     const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x100 | N, 0xf, 0xf, true);
     return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
+// Lane l's value of lane l - N (past the row's start: 0).
+template <int N>
+__device__ __forceinline__ double row_up(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x110 | N, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x110 | N, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
 // The upper half of the wave in its lower half (32), or the odd rows of 16 in
 // the even ones (16).
 template <int N>

@@ -62,6 +62,12 @@ __host__ inline bool whole_fits(int n) { return n <= kWholeRows; }
 // Elements kept free before the first array and behind the last, for the
 // chains' reads past a line's ends.
 constexpr int kWholeFront = 16, kWholeTail = 16;
+// k_line_stream's lines hold rows in eights (whole_forward_swap8).
+__host__ __device__ constexpr int stream_rows(int n) { return (n + 7) & ~7; }
+__host__ __device__ constexpr int stream_stride(int n) { return stream_rows(n) + 2; }
+__host__ __device__ constexpr int stream_elems(int n, int lpb) {
+    return kWholeFront + 4 * lpb * stream_stride(n) + kWholeTail;
+}
 // LDS elements of a block of lpb lines: four arrays.
 __host__ __device__ constexpr int whole_elems(int n, int lpb) {
     return kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
@@ -97,7 +103,7 @@ __host__ inline bool line_streams(int n, double lds, int64_t cells) {
 // Entries of a colour of `lines` lines then: the fewest a block, of lines that
 // it holds.
 __host__ inline int64_t stream_entries(int n, int64_t lines) {
-    int64_t most = (kStreamLdsTarget / 8 - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    int64_t most = (kStreamLdsTarget / 8 - kWholeFront - kWholeTail) / (4 * stream_stride(n));
     if (most > kStreamRows / n) most = kStreamRows / n;
     if (most > kWholeLines) most = kWholeLines;
     return (lines + kStreamBlocks * most - 1) / (kStreamBlocks * most) * kStreamBlocks;
@@ -407,6 +413,67 @@ __device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const d
         run(s1, R);
     }
     if (rows > 0) run(s0, 0);
+}
+
+// These two passes by eight lanes a line (j = lane % 8), rows in eights, for a
+// wave of up to eight lines: lane j holds row j of a group of eight, and a step
+// forms every lane's row from its neighbour's, passed by a lane shift, so row j
+// is right after j + 1 steps and stays (its operands do not change), and eight
+// steps solve the group.  The row next to the group before (lane 0 forward,
+// lane 7 back) takes that group's values first and is then held by zero
+// couplings.  What does not depend on the neighbour, the marked multipliers and
+// the reciprocal, is formed for eight rows at once; in one lane a line it is
+// most of the instructions (256^3: 261 -> 226 us a phase; with more lines a
+// wave takes two turns: 11 lines a block, 150x201x180, 91 -> 121 us; without
+// interchanges there is little of it: 203 -> 205).
+__device__ __forceinline__ void whole_forward_swap8(const double *__restrict__ pf, double *__restrict__ pb, int rows,
+                                                    int j) {
+    double f = pf[j], b = pb[j], v = 0.0;
+    for (int at = j; at < rows; at += 8) {
+        const double nf = pf[at + 8], nb = pb[at + 8];
+        const double c = row_down<7>(v);
+        const bool s = swapped(f);
+        const double fact = s ? f * kSwapDown : f, m = fact * b;
+        v = s ? c - m : b - fact * c;  // (lane 0's, the others' below)
+        const bool s1 = s && j != 0;
+        const double f1 = j == 0 ? 0.0 : fact, b1 = j == 0 ? v : b;
+#pragma unroll
+        for (int k = 1; k < 8; ++k) {
+            const double p = row_up<1>(v), keep = b1 - f1 * p, trade = p - m;
+            v = s1 ? trade : keep;
+        }
+        const double p = row_up<1>(v);
+        pb[at - 1] = s ? b : j == 0 ? c : p;  // (row 0 writes in front of the line, an element that is not used)
+        f = nf;
+        b = nb;
+    }
+    if (j == 7) pb[rows - 1] = v;
+}
+
+__device__ __forceinline__ void whole_back_swap8(double *__restrict__ pb, const double *__restrict__ pu,
+                                                 const double *__restrict__ pv, const double *__restrict__ pd,
+                                                 int rows, int j) {
+    int at = rows - 8 + j;
+    double b = pb[at], u = pu[at], v = pv[at], d = pd[at], x = 0.0;
+    for (; at >= 0; at -= 8) {
+        const double nb = pb[at - 8], nu = pu[at - 8], nv = pv[at - 8], nd = pd[at - 8], r = refined_rcp(d);
+        // the group after's first row in lane 7; its first two in lanes 6 and 7
+        const double c1 = row_up<7>(x), c2 = row_up<6>(x);
+        b = j == 7 ? b - u * c1 - v * c2 : b;
+        u = j == 7 ? 0.0 : u;
+        v = j == 7 ? 0.0 : v;
+        x = corrected_quotient(b, d, r);
+#pragma unroll
+        for (int k = 1; k < 8; ++k) {
+            const double two = row_down<2>(x);
+            x = corrected_quotient(b - u * row_down<1>(x) - v * (j >= 6 ? c2 : two), d, r);
+        }
+        pb[at] = x;
+        b = nb;
+        u = nu;
+        v = nv;
+        d = nd;
+    }
 }
 
 // DGTSV's elimination of every line of the listed FP64 systems, both colours
@@ -834,7 +901,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     if (threadIdx.x == 0) redo = st->line_general;
     __syncthreads();
     const DGrid &g = S.g;
-    const int n = g.nj, ls = whole_stride(n), do_k = g.do_k, rows = whole_rows(n), lpb = S.lpb;
+    const int n = g.nj, ls = stream_stride(n), do_k = g.do_k, rows = stream_rows(n), lpb = S.lpb;
     double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ B = F + lpb * ls,
                          *__restrict__ U = B + lpb * ls, *__restrict__ D = U + lpb * ls;
     if (!redo) {
@@ -923,21 +990,28 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
         if (wave == solver) {
             for (;;) {
                 if (e.y == 0 && lane == 0) st->line_launches += 1;  // (timing: working launches)
-                const bool more = en.x == id, mine = lane < L.n;
+                const int nl = L.n;
+                const bool more = en.x == id, mine = lane < nl;
                 const int swp = marked(mk), ol = lane * ls;
+                // (eight lanes a line; past the last line: it again, the same values)
+                const int o8 = (lane >> 3 < nl ? lane >> 3 : nl - 1) * ls;
                 if (more) L.set(g, S.lstep, en.y, param, lane);
                 it += step;
                 e = en;
                 if (more) en = next();
                 if (more) mk = mark();
                 __syncthreads();  // the rows are there
-                if (mine) {
+                if (swp && nl > 0 && nl <= 8) {
+                    whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
+                } else if (mine) {
                     if (swp) whole_forward_swap(F + ol, B + ol, rows);
                     else whole_forward(F + ol, B + ol, rows);
                 }
                 __syncthreads();  // forward pass done
                 __syncthreads();  // the diagonals are there
-                if (mine) {
+                if (swp && nl > 0 && nl <= 8) {
+                    whole_back_swap8(B + o8, U + o8, D + o8, F + o8, rows, lane & 7);
+                } else if (mine) {
                     if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
                     else whole_back(B + ol, U + ol, D + ol, F + ol, rows);
                 }
@@ -965,8 +1039,8 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                     U[o] = q < n - 1 ? u[k] : 0.0;
                     D[o] = swp ? v[k] : d[k];
                 }
-                for (int x = lt; x < 4 * nl; x += kStreamLoaders) {
-                    const int q = n + (x & 3), o = (x >> 2) * ls + q;
+                for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
+                    const int q = n + (x & 7), o = (x >> 3) * ls + q;
                     if (q < rows) {  // identity rows
                         F[o] = B[o] = U[o] = 0.0;
                         D[o] = 1.0;
@@ -996,9 +1070,9 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                     if (k * kStreamLoaders >= tot) break;
                     if (here(k)) F[at(k)] = d[k];
                 }
-                for (int x = lt; x < 4 * nl; x += kStreamLoaders) {
-                    const int q = n + (x & 3);
-                    if (q < rows) F[(x >> 2) * ls + q] = 1.0;
+                for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
+                    const int q = n + (x & 7);
+                    if (q < rows) F[(x >> 3) * ls + q] = 1.0;
                 }
                 __syncthreads();  // the diagonals are there
                 if (more) {

@@ -400,7 +400,7 @@ static void set_line_kernel(Sys<T> &S, double table = 0.0) {
 }
 template <typename T>
 static int whole_lds_bytes(const Sys<T> &S) {
-    return (int)sizeof(T) * whole_elems(S.g.nj, S.lpb);
+    return (int)sizeof(T) * (S.lk == LINE_STREAM ? stream_elems(S.g.nj, S.lpb) : whole_elems(S.g.nj, S.lpb));
 }
 
 template <typename T>

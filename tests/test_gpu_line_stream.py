@@ -37,7 +37,7 @@ def _both(gpu, dims, no_k, kind, change=None, rhs=None):
 
 
 @pytest.mark.parametrize("dims,no_k,kind", [((511, 34, 511), False, 1), ((195, 255, 195), False, 0),
-                                            ((194, 254, 196), False, 1), ((80, 1534, 78), False, 0),
+                                            ((194, 254, 196), False, 1), ((200, 246, 198), False, 0), ((80, 1534, 78), False, 0),
                                             ((6500, 1534, 1), True, 1)])
 def test_sizes(gpu, dims, no_k, kind):
     _both(gpu, dims, no_k, kind)
