@@ -62,15 +62,17 @@ __host__ inline bool whole_fits(int n) { return n <= kWholeRows; }
 // Elements kept free before the first array and behind the last, for the
 // chains' reads past a line's ends.
 constexpr int kWholeFront = 16, kWholeTail = 16;
-// k_line_stream's lines hold rows in eights (whole_forward_swap8).
+// Lines of k_line_stream, and of blocks of up to eight, hold rows in eights
+// (whole_forward_swap8).
 __host__ __device__ constexpr int stream_rows(int n) { return (n + 7) & ~7; }
 __host__ __device__ constexpr int stream_stride(int n) { return stream_rows(n) + 2; }
 __host__ __device__ constexpr int stream_elems(int n, int lpb) {
     return kWholeFront + 4 * lpb * stream_stride(n) + kWholeTail;
 }
+__host__ __device__ constexpr bool whole_few(int lpb) { return lpb <= 8; }
 // LDS elements of a block of lpb lines: four arrays.
 __host__ __device__ constexpr int whole_elems(int n, int lpb) {
-    return kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
+    return whole_few(lpb) ? stream_elems(n, lpb) : kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
 }
 
 // Lines per block.  `table` is the LDS that all lines of one colour of every
@@ -743,8 +745,9 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
     if (st->done || (which == 1 && st->s_exit)) return;
     if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
     const DGrid &g = S.g;
-    const int n = g.nj, ls = whole_stride(n), do_k = g.do_k;
-    const int rows = whole_rows(n);
+    const bool few = whole_few(S.lpb);
+    const int n = g.nj, ls = few ? stream_stride(n) : whole_stride(n), do_k = g.do_k;
+    const int rows = whole_rows(n), held = few ? stream_rows(n) : rows;
     whole_lines(g, S.lstep, e.y, param, w);
     const int nl = w.n, tot = nl * n;
     // right-hand side (then the solution), upper coupling, and: multipliers
@@ -787,9 +790,9 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
                     td[k0 + k] = r[k].d;
                 }
             }
-            for (int x = threadIdx.x; x < 4 * nl; x += kWholeThreads) {
-                const int q = n + (x & 3), at = (x >> 2) * ls + q;
-                if (q < rows) {  // identity rows
+            for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
+                const int q = n + (x & 7), at = (x >> 3) * ls + q;
+                if (q < held) {  // identity rows
                     F[at] = B[at] = U[at] = 0.0;
                     D[at] = 1.0;
                 }
@@ -809,7 +812,14 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             const int solver = (int)threadIdx.x - 64 * ((blockIdx.x >> 8) & 3);
             const bool mine = solver >= 0 && solver < nl;
             const int ol = solver * ls;
-            if (mine) {
+            // with interchanges eight lanes a line where they are few (past the
+            // last line: it again, the same values): 30x90x3 13.5 -> 11.4 us, 64^3
+            // 13.7 -> 12.0, 40x200x40 30 -> 21
+            const bool eight = swaps && few && nl > 0 && solver >= 0 && solver < 64;
+            const int o8 = (solver >> 3 < nl ? solver >> 3 : nl - 1) * ls;
+            if (eight) {
+                whole_forward_swap8(F + o8, B + o8, held, threadIdx.x & 7);
+            } else if (mine) {
                 if (swaps) whole_forward_swap(F + ol, B + ol, rows);
                 else whole_forward(F + ol, B + ol, rows);
             }
@@ -817,12 +827,14 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
 #pragma unroll
             for (int k = 0; k < kWholeElems; ++k)
                 if (k / K * K * kWholeThreads < tot) F[o[k]] = td[k];
-            for (int x = threadIdx.x; x < 4 * nl; x += kWholeThreads) {
-                const int q = n + (x & 3);
-                if (q < rows) F[(x >> 2) * ls + q] = 1.0;
+            for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
+                const int q = n + (x & 7);
+                if (q < held) F[(x >> 3) * ls + q] = 1.0;
             }
             __syncthreads();
-            if (mine) {
+            if (eight) {
+                whole_back_swap8(B + o8, U + o8, D + o8, F + o8, held, threadIdx.x & 7);
+            } else if (mine) {
                 if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
                 else whole_back(B + ol, U + ol, F + ol, D + ol, rows);
             }
@@ -1004,16 +1016,16 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                 if (swp && nl > 0 && nl <= 8) {
                     whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
                 } else if (mine) {
-                    if (swp) whole_forward_swap(F + ol, B + ol, rows);
-                    else whole_forward(F + ol, B + ol, rows);
+                    if (swp) whole_forward_swap(F + ol, B + ol, whole_rows(n));
+                    else whole_forward(F + ol, B + ol, whole_rows(n));
                 }
                 __syncthreads();  // forward pass done
                 __syncthreads();  // the diagonals are there
                 if (swp && nl > 0 && nl <= 8) {
                     whole_back_swap8(B + o8, U + o8, D + o8, F + o8, rows, lane & 7);
                 } else if (mine) {
-                    if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
-                    else whole_back(B + ol, U + ol, D + ol, F + ol, rows);
+                    if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
+                    else whole_back(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
                 }
                 __syncthreads();  // solved
                 if (!more) break;
