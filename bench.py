@@ -209,7 +209,7 @@ def bench_line(args):
                    "iterations": f["its"], "line_phase_us": f["line_us"], "line_phase_alg_GBps": f["line_GBps"],
                    "mixed_solves_per_s": m["value"], "mixed_iterations": m["its"],
                    "solve_alg_GBps": alg / 1e9, "solve_roofline_frac": alg / HBM_PEAK},
-        "roofline": {"bound": "hbm", "kernel": "k_line_color_sys<double> (one red-black colour of line solves)",
+        "roofline": {"bound": "hbm", "kernel": "k_line_whole<double> (one red-black colour of line solves)",
                      "achieved": f["line_GBps"], "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": f["line_GBps"] * 1e9 / HBM_PEAK, "traffic": None},
         "cpu_baseline": None,
