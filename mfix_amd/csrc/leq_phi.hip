@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(kPhiBlock) k_conv_dif_phi(PhiArgs R, int64_t n
     // compiler could sink them into, and kept only on fluid rows (in 2-D
     // KM = KP = the cell and the K faces are dropped).
     const Nb n = neighbours(g, c);
-    const int iw = nb_minus(i, g.ni, g.cyc_x), js = nb_minus(j, g.nj, g.cyc_y), kb = nb_minus(k, g.nk, g.cyc_z);
+    const int iw = nb_minus(i, g.ni, g.cyc_x), js = nb_minus(j, g.nj, g.cyc_y);
     const int fc = flag[c];
     const int f_ip = flag[n.ip], f_jp = flag[n.jp], f_kp = flag[n.kp];
     const int f_im = flag[n.im], f_jm = flag[n.jm], f_km = flag[n.km];
@@ -100,10 +100,30 @@ __global__ void __launch_bounds__(kPhiBlock) k_conv_dif_phi(PhiArgs R, int64_t n
     const double fec = fe[c], fnc = fn[c], ftc = ft[c], fe_im = fe[n.im], fn_jm = fn[n.jm], ft_km = ft[n.km];
     const double ayc = ayz[c], axzc = axz[c], axyc = axy[c];
     const double ay_im = ayz[n.im], axz_jm = axz[n.jm], axy_km = axy[n.km];
-    const double gx = fx_e[i], gxb = fx_eb[i], ox_e = odx_e[i], gxw = fx_e[iw], gxwb = fx_eb[iw], ox_w = odx_e[iw];
+    // The kernel is bound by its vector memory instructions (59 for 64 cells
+    // when each took its axis tables by lane: 150x201x180 267 -> 242 us), so the
+    // tables of K, one value for the block's plane, and of I, one or two for a
+    // wave along J, come by scalar loads.
+    const int i0 = __builtin_amdgcn_readfirstlane(i), i1 = i0 + 1 < g.ni ? i0 + 1 : i0;
+    const bool hi = i != i0;
+    auto along_i = [&](auto t) __attribute__((always_inline)) {
+        const double lo = t[i0], up = t[i1];
+        return hi ? up : lo;
+    };
+    const int w0 = nb_minus(i0, g.ni, g.cyc_x), w1 = nb_minus(i1, g.ni, g.cyc_x);
+    auto west_i = [&](auto t) __attribute__((always_inline)) {
+        const double lo = t[w0], up = t[w1];
+        return hi ? up : lo;
+    };
+    double gx = along_i(fx_e), gxb = along_i(fx_eb), ox_e = along_i(odx_e), oxi = along_i(ox);
+    double gxw = west_i(fx_e), gxwb = west_i(fx_eb), ox_w = west_i(odx_e);
+    if (__any(i > i1)) {  // (rows of fewer cells than lanes)
+        gx = fx_e[i], gxb = fx_eb[i], ox_e = odx_e[i], oxi = ox[i];
+        gxw = fx_e[iw], gxwb = fx_eb[iw], ox_w = odx_e[iw];
+    }
+    const int ku = __builtin_amdgcn_readfirstlane(k), kd = nb_minus(ku, g.nk, g.cyc_z);
     const double gy = fy_n[j], gyb = fy_nb[j], oy_n = ody_n[j], gys = fy_n[js], gysb = fy_nb[js], oy_s = ody_n[js];
-    const double gz = fz_t[k], gzb = fz_tb[k], oz_t = odz_t[k], gzb_ = fz_t[kb], gzbb = fz_tb[kb], oz_b = odz_t[kb];
-    const double oxi = ox[i];
+    const double gz = fz_t[ku], gzb = fz_tb[ku], oz_t = odz_t[ku], gzb_ = fz_t[kd], gzbb = fz_tb[kd], oz_b = odz_t[kd];
     // own east/north/top faces; EAST_OF is IP_OF unless that is a wall
     const double de = wall_at(f_ip) ? dc : d_ip;
     const double dn = wall_at(f_jp) ? dc : d_jp;
