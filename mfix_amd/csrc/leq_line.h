@@ -910,6 +910,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     const Sys<double> &S = sys[id];
     auto *__restrict__ st = to_global(S.st);
     if (st->done || (which == 1 && st->s_exit)) return;
+    if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
     if (threadIdx.x == 0) redo = st->line_general;
     __syncthreads();
     const DGrid &g = S.g;
@@ -1001,7 +1002,6 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
         double mk = mark();
         if (wave == solver) {
             for (;;) {
-                if (e.y == 0 && lane == 0) st->line_launches += 1;  // (timing: working launches)
                 const int nl = L.n;
                 const bool more = en.x == id, mine = lane < nl;
                 const int swp = marked(mk), ol = lane * ls;
