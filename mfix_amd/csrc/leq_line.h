@@ -51,6 +51,7 @@ constexpr int kWholeLines = 64;  // one lane of the solving wave per line
 constexpr int kStreamThreads = 512, kStreamLoaders = kStreamThreads - 64, kStreamElems = 5,
               kStreamRows = kStreamLoaders * kStreamElems, kStreamBlocks = 2 * kNumCus,
               kStreamLdsTarget = 160 * 1024 / 2 - 3072;
+constexpr int kStreamMost = 1024;  // entries of a block, a bit each in k_line_stream
 
 // A line holds whole_rows rows (its own and up to three identity rows, so that
 // the chains take four rows a step) and lines sit an odd number of 16-byte
@@ -97,11 +98,6 @@ __host__ inline int whole_lpb(int n, double table, size_t elem, int pin) {
     return lpb < 1 ? 1 : (int)lpb;
 }
 
-// Whether the lines of a system, `lds` bytes a colour in all, stream: they
-// take more than one round of k_line_whole's blocks.
-__host__ inline bool line_streams(int n, double lds, int64_t cells) {
-    return lds > 4.0 * kNumCus * kWholeLdsTarget && n <= kWholeRows && cells < (1ll << 29);
-}
 // Entries of a colour of `lines` lines then: the fewest a block, of lines that
 // it holds.
 __host__ inline int64_t stream_entries(int n, int64_t lines) {
@@ -109,6 +105,12 @@ __host__ inline int64_t stream_entries(int n, int64_t lines) {
     if (most > kStreamRows / n) most = kStreamRows / n;
     if (most > kWholeLines) most = kWholeLines;
     return (lines + kStreamBlocks * most - 1) / (kStreamBlocks * most) * kStreamBlocks;
+}
+// Whether the lines of a system, `lines` of `lds` bytes a colour in all, stream:
+// they take more than one round of k_line_whole's blocks.
+__host__ inline bool line_streams(int n, int64_t lines, double lds, int64_t cells) {
+    return lds > 4.0 * kNumCus * kWholeLdsTarget && n <= kWholeRows && cells < (1ll << 29) &&
+           stream_entries(n, lines) <= (int64_t)kStreamBlocks * kStreamMost;
 }
 // Lines of entry j of a colour: [first(j), first(j + 1)), where first(j) = j
 // step / 2^32.  step = lines / entries, rounded up, shares them evenly (the last
@@ -870,7 +872,8 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
 // 4.2 of the 5.1 TB/s of a copy: 256^3 233 -> 201 us, 170^3 71 -> 59 us,
 // 150x201x180 76 -> 69 us.  Non-temporal loads of the arrays read once: 195 us
 // at 256^3, but 48 for 42 us at 200x100x200, whose arrays the last-level cache
-// holds.
+// holds.  An entry with a value out of range is left to DGTSV at the end.
+
 // Start cell and I/K neighbour offsets of line `lane` of a block, in every wave.
 struct StreamLines {
     uint32_t c0, im, ip, km, kp;
@@ -897,7 +900,8 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     extern __shared__ __align__(16) char whole_lds[];
     __shared__ WholeLines w;
     __shared__ int linfo[kWholeLines];
-    __shared__ int redo;
+    __shared__ int odd;                           // the entry has a value out of range
+    __shared__ uint32_t again[kStreamMost / 32];  // this block's entries that are left to DGTSV itself
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // another solving wave in each of the blocks that share a CU (every 256th)
     const int solver = (blockIdx.x >> 8) & 1;
@@ -911,13 +915,15 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     auto *__restrict__ st = to_global(S.st);
     if (st->done || (which == 1 && st->s_exit)) return;
     if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
-    if (threadIdx.x == 0) redo = st->line_general;
+    const bool general = st->line_general;
+    if (threadIdx.x == 0) odd = 0;
+    if (threadIdx.x < kStreamMost / 32) again[threadIdx.x] = general ? ~0u : 0u;
     __syncthreads();
     const DGrid &g = S.g;
     const int n = g.nj, ls = stream_stride(n), do_k = g.do_k, rows = stream_rows(n), lpb = S.lpb;
     double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ B = F + lpb * ls,
                          *__restrict__ U = B + lpb * ls, *__restrict__ D = U + lpb * ls;
-    if (!redo) {
+    if (!general) {
         WholeArrays<double> A = whole_arrays(S, which);
         A.f = to_global((const double *)S.lf);
         A.d = to_global((const double *)S.ld);
@@ -991,7 +997,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
         };
         auto mark = [&]() __attribute__((always_inline)) { return ld(A.f, 8u * StreamLines::of(L.c0, 0)); };  // (in every wave alike)
         auto marked = [](double f) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)swapped(f)); };
-        // (both loops below take the same entries and meet at the same four
+        // (both loops below take the same entries and meet at the same five
         // barriers an entry; apart, the solving wave's chains and the others'
         // rows do not share registers)
         auto next = [&]() __attribute__((always_inline)) {
@@ -1013,6 +1019,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                 if (more) en = next();
                 if (more) mk = mark();
                 __syncthreads();  // the rows are there
+                if (lane == 0) odd = 0;
                 if (swp && nl > 0 && nl <= 8) {
                     whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
                 } else if (mine) {
@@ -1028,6 +1035,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                     else whole_back(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
                 }
                 __syncthreads();  // solved
+                __syncthreads();  // looked at
                 if (!more) break;
             }
         } else {
@@ -1035,7 +1043,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
             factors(swn);
 #pragma unroll
             for (int k0 = 0; k0 < kStreamElems; k0 += 2) rhs2(k0);
-            for (;;) {
+            for (int nth = 0;; ++nth) {
                 const bool more = en.x == id;
                 const int nl = L.n, swp = swn;
                 const uint32_t c0 = L.c0;  // start cells of the entry being solved
@@ -1104,25 +1112,33 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
 #pragma unroll
                 for (int k = 0; k < kStreamElems; ++k) {
                     if (k * kStreamLoaders >= tot) break;
-                    if (!here(k)) continue;
-                    const double x = B[at(k)];
-                    bad |= !solution_in_range(x);
-                    *(gptr<double>)((gptr<char>)A.var + c[k]) = x;
+                    if (here(k)) bad |= !solution_in_range(B[at(k)]);
                 }
-                if (bad) redo = 1;
+                if (bad) odd = 1;
+                // nothing of an entry is stored before all of it is in range:
+                // the lines on a clamped end of I or K read their own values
+                __syncthreads();  // looked at
+                if (odd) {
+                    if (lt == 0) again[nth >> 5] |= 1u << (nth & 31);
+                } else {
+                    fresh();
+#pragma unroll
+                    for (int k = 0; k < kStreamElems; ++k) {
+                        if (k * kStreamLoaders >= tot) break;
+                        if (here(k)) *(gptr<double>)((gptr<char>)A.var + c[k]) = B[at(k)];
+                    }
+                }
                 if (!more) break;
             }
         }
         __syncthreads();
-        if (!redo) return;
     }
-    // a pivot or a value out of range: DGTSV itself, on every entry of this
-    // block (their inputs, the other colour's values, are as they were)
-    for (it = blockIdx.x; it < nmap; it += step) {
-        e = map[it];
-        if (e.x != id) break;
+    // a pivot or a value out of range: DGTSV itself (the entries' inputs are as
+    // they were: the other colour's values and, on clamped ends, their own)
+    for (int k = 0, at = blockIdx.x; at < nmap && map[at].x == id; ++k, at += step) {
+        if (!(again[k >> 5] >> (k & 31) & 1u)) continue;
         __syncthreads();
-        whole_lines(g, S.lstep, e.y, param, w);
+        whole_lines(g, S.lstep, map[at].y, param, w);
         whole_general<double, kStreamThreads>(S, w, linfo, which);
     }
 }

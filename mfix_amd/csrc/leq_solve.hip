@@ -385,7 +385,7 @@ static void set_line_kernel(Sys<T> &S, double table = 0.0) {
     if (!whole_fits(L.n)) {
         S.lk = LINE_LONG;
         S.lpb = kLongLpb;
-    } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, own, g.n3)) {
+    } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, colour_lines(L), own, g.n3)) {
         S.lk = LINE_STREAM;
         S.lent = stream_entries(L.n, colour_lines(L));
         S.lstep = entry_step(colour_lines(L), S.lent);

@@ -1,9 +1,10 @@
 """GPU: LINE systems some of whose lines cannot run on their factored rows (a
-pivot out of the corrected quotient's range)."""
+pivot, or values of the solution, out of the corrected quotient's range)."""
 import numpy as np
 import pytest
 
 from tests.cases import make_system
+from tests.test_gpu_line_stream import _both
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +32,32 @@ def test_working_launches_are_counted(gpu):
         gpu.prof_enable(1, False)
     assert r.stats["iterations"] == 2
     assert p["launches"] == 2 * 2 * 4     # two applications an iteration, four phases each
+
+
+@pytest.mark.parametrize("dims,no_k", [((195, 255, 195), False), ((6500, 1534, 1), True)])
+def test_clamped_lines_read_their_own_start_values(gpu, dims, no_k):
+    """The lines on an end of I or K have themselves as outward neighbour: with
+    an outward coupling their right-hand side holds the values they start from,
+    also when part of a block's solution is out of range and it is solved
+    again.  Streamed lines against k_line_whole, the same bits."""
+    im, jm, km = dims
+    nk, ni, nj = 1 if no_k else km + 2, im + 2, jm + 2
+
+    def change(p):
+        q = p.reshape(7, nk, ni, nj)
+        q[2, :, 0] = 0.21
+        q[4, :, -1] = 0.17
+        if not no_k:
+            q[0, 0] = 0.13
+            q[6, -1] = 0.11
+
+    def rhs(n):
+        r = np.random.default_rng(9).uniform(-1.0, 1.0, (nk, ni, nj))
+        r[:, 0, ::3] *= 1e-303            # out of range beside values in range
+        r[:, -1, nj // 2] = np.inf
+        r[nk // 2, ni // 2:ni // 2 + 20, :9] *= 1e-300
+        if not no_k:
+            r[0, ::7] *= 1e-305
+            r[-1, ni // 3, 5] = -np.inf
+        return r.reshape(-1)
+    _both(gpu, dims, no_k, 1, change, rhs)
