@@ -57,7 +57,6 @@ struct SolverState {
     int k1_launches;        // launches of the first stencil pass that worked on this system (timing)
     int line_launches;      // colour-phase launches that worked on this system (timing)
     int resident_gone;      // a block of k_resident gave up waiting for another
-    int line_general;       // LINE: some line needs DGTSV itself (row interchange, zero pivot, range): k_line_factor
     double l2[4 * kFinishBlocks];  // level-2 sums of the finish launches
 };
 

@@ -23,9 +23,9 @@
 // Blocks with a row interchange carry it through both passes.  Every value is
 // the one DGTSV's own operations give, bit for bit (but for the sign of a
 // zero), as long as no operand leaves the range in which the correction is
-// exact; a system with a pivot outside it or zero (SolverState::line_general)
-// runs DGTSV itself in LDS, and so does a block whose solution holds a value
-// outside the range.
+// exact; a block with a pivot outside it or zero (marked by k_line_factor) runs
+// DGTSV itself in LDS, and so does one whose solution holds a value outside the
+// range.
 //
 // Measured (events of the dispatches, LINE solve, colour phase; before, one
 // DGTSV lane per line over 16-row tiles with the finished rows in global
@@ -181,6 +181,13 @@ __device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j
 // exactly.
 constexpr double kSwapUp = 0x1p600, kSwapDown = 0x1p-600;
 __device__ __forceinline__ bool swapped(double f) { return fabs(f) > 2.0; }
+// A block's mark, in the place of its first row's multiplier (which has none):
+// kSwapUp where it has an interchanged row, this where it has a pivot of zero or
+// out of range.  By block, so that one such line does not cost the others: with
+// DGTSV in every block of a system that has one 150x201x180 took 208 us a phase
+// and 256^3 690, now 94 and 228 (109 and 399 with k_line_color_sys).
+constexpr double kOwnDgtsv = 0x1p620;
+__device__ __forceinline__ bool own_dgtsv(double mark) { return fabs(mark) > 0x1p610; }
 
 // The elimination of one line without row interchanges and the two passes on
 // its factored rows, in the lane that solves the line, over whole_rows(n)
@@ -557,10 +564,10 @@ static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<
     }
     load();
     int any = 0;
+    bool ok = true;
     if ((int)threadIdx.x < nl) {
         const int o = threadIdx.x * ls;
         double d = D[o], u = U[o];
-        bool ok = true;
         double dl1 = F[o + 1], d1 = D[o + 1], u1 = U[o + 1];  // (a line has at least three rows)
         for (int i = 0; i < n - 1; ++i) {
             const int nx = i + 2 < n ? i + 2 : n - 1;  // the next row is read ahead of this one's division
@@ -598,13 +605,13 @@ static __global__ void __launch_bounds__(kWholeThreads) k_line_factor(const Sys<
         U[o + n - 1] = 0.0;
         V[o + n - 1] = 0.0;
         ok = ok && factor_in_range(d);
-        if (!ok) atomicOr((int *)&st->line_general, 1);
     }
     any = __syncthreads_or(any);
+    const int own = __syncthreads_or(!ok);
     for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
         const int l = (int)div_by((uint32_t)x, g.mnj, g.snj), q = x - l * n, at = l * ls + q;
         const uint32_t c = w.c0[l] + (uint32_t)q;
-        lf[c] = any && x == 0 ? kSwapUp : F[at];  // (the block's mark: a first row has no multiplier)
+        lf[c] = x > 0 || !(any || own) ? F[at] : own ? kOwnDgtsv : kSwapUp;
         ld[c] = D[at];
         if (any) {
             lu[c] = U[at];
@@ -761,45 +768,46 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
     // (a line's rows are consecutive elements: element x is row x % n of line x / n)
     auto line_of = [&](int x) { return (int)div_by((uint32_t)x, g.mnj, g.snj); };
     if constexpr (sizeof(T) == sizeof(double)) {
-        if (!st->line_general) {
-            A.f = to_global((const T *)S.lf);
-            A.d = to_global((const T *)S.ld);
-            constexpr int K = 3;  // rows in flight per thread
-            T td[kWholeElems];    // the diagonals wait for the multipliers' place
-            int o[kWholeElems], any = 0;
+        A.f = to_global((const T *)S.lf);
+        A.d = to_global((const T *)S.ld);
+        const double mark = nl > 0 ? (double)A.f[w.c0[0]] : 0.0;
+        constexpr int K = 3;  // rows in flight per thread
+        T td[kWholeElems];    // the diagonals wait for the multipliers' place
+        int o[kWholeElems], any = 0;
 #pragma unroll
-            for (int k0 = 0; k0 < kWholeElems; k0 += K) {
-                if (k0 * kWholeThreads >= tot) break;
-                WholeRow<T> r[K];
-                bool first[K], last[K];
+        for (int k0 = 0; k0 < kWholeElems; k0 += K) {
+            if (k0 * kWholeThreads >= tot) break;
+            WholeRow<T> r[K];
+            bool first[K], last[K];
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
-                    const int x = x0 < tot ? x0 : tot - 1;  // (past the end: the last row again)
-                    const int l = line_of(x), q = x - l * n;
-                    o[k0 + k] = l * ls + q;
-                    r[k].load(A, w, l, w.c0[l] + (uint32_t)q);
-                    first[k] = q == 0;
-                    last[k] = q == n - 1;
-                }
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    F[o[k0 + k]] = first[k] ? (T)0 : r[k].f;
-                    any |= swapped(r[k].f);
-                    B[o[k0 + k]] = r[k].rhs(do_k);
-                    U[o[k0 + k]] = last[k] ? (T)0 : r[k].u;
-                    D[o[k0 + k]] = (T)refined_rcp(r[k].d);
-                    td[k0 + k] = r[k].d;
-                }
+            for (int k = 0; k < K; ++k) {
+                const int x0 = (int)threadIdx.x + (k0 + k) * kWholeThreads;
+                const int x = x0 < tot ? x0 : tot - 1;  // (past the end: the last row again)
+                const int l = line_of(x), q = x - l * n;
+                o[k0 + k] = l * ls + q;
+                r[k].load(A, w, l, w.c0[l] + (uint32_t)q);
+                first[k] = q == 0;
+                last[k] = q == n - 1;
             }
-            for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
-                const int q = n + (x & 7), at = (x >> 3) * ls + q;
-                if (q < held) {  // identity rows
-                    F[at] = B[at] = U[at] = 0.0;
-                    D[at] = 1.0;
-                }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                F[o[k0 + k]] = first[k] ? (T)0 : r[k].f;
+                any |= swapped(r[k].f);
+                B[o[k0 + k]] = r[k].rhs(do_k);
+                U[o[k0 + k]] = last[k] ? (T)0 : r[k].u;
+                D[o[k0 + k]] = (T)refined_rcp(r[k].d);
+                td[k0 + k] = r[k].d;
             }
-            const bool swaps = __syncthreads_or(any);
+        }
+        for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
+            const int q = n + (x & 7), at = (x >> 3) * ls + q;
+            if (q < held) {  // identity rows
+                F[at] = B[at] = U[at] = 0.0;
+                D[at] = 1.0;
+            }
+        }
+        const bool swaps = __syncthreads_or(any);
+        if (!own_dgtsv(mark)) {
             if (swaps) {
                 const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
                 for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
@@ -900,7 +908,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     extern __shared__ __align__(16) char whole_lds[];
     __shared__ WholeLines w;
     __shared__ int linfo[kWholeLines];
-    __shared__ int odd;                           // the entry has a value out of range
+    __shared__ int odd;                           // the entry has a pivot or a value out of range
     __shared__ uint32_t again[kStreamMost / 32];  // this block's entries that are left to DGTSV itself
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // another solving wave in each of the blocks that share a CU (every 256th)
@@ -915,224 +923,224 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     auto *__restrict__ st = to_global(S.st);
     if (st->done || (which == 1 && st->s_exit)) return;
     if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
-    const bool general = st->line_general;
     if (threadIdx.x == 0) odd = 0;
-    if (threadIdx.x < kStreamMost / 32) again[threadIdx.x] = general ? ~0u : 0u;
+    if (threadIdx.x < kStreamMost / 32) again[threadIdx.x] = 0;
     __syncthreads();
     const DGrid &g = S.g;
     const int n = g.nj, ls = stream_stride(n), do_k = g.do_k, rows = stream_rows(n), lpb = S.lpb;
     double *__restrict__ F = (double *)whole_lds + kWholeFront, *__restrict__ B = F + lpb * ls,
                          *__restrict__ U = B + lpb * ls, *__restrict__ D = U + lpb * ls;
-    if (!general) {
-        WholeArrays<double> A = whole_arrays(S, which);
-        A.f = to_global((const double *)S.lf);
-        A.d = to_global((const double *)S.ld);
-        const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
-        // rows lt + k kStreamLoaders of the block's: row q of line l
-        double b[kStreamElems], f[kStreamElems], u[kStreamElems], v[kStreamElems], d[kStreamElems];
-        int lq[kStreamElems];
+    WholeArrays<double> A = whole_arrays(S, which);
+    A.f = to_global((const double *)S.lf);
+    A.d = to_global((const double *)S.ld);
+    const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
+    // rows lt + k kStreamLoaders of the block's: row q of line l
+    double b[kStreamElems], f[kStreamElems], u[kStreamElems], v[kStreamElems], d[kStreamElems];
+    int lq[kStreamElems];
+#pragma unroll
+    for (int k = 0; k < kStreamElems; ++k) {
+        const int x0 = lt + k * kStreamLoaders, x = x0 < lpb * n ? x0 : lpb * n - 1;
+        const int l = (int)div_by((uint32_t)x, g.mnj, g.snj);
+        lq[k] = l << 16 | (x - l * n);
+    }
+    StreamLines L;
+    int tot = 0;
+    // (opaque: what is formed from lq is formed again in each step and
+    // not held in registers over the loop)
+    auto fresh = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kStreamElems; ++k) asm volatile("" : "+v"(lq[k]));
+    };
+    auto at = [&](int k) __attribute__((always_inline)) { return (lq[k] >> 16) * ls + (lq[k] & 0xffff); };
+    auto here = [&](int k) __attribute__((always_inline)) { return lt + k * kStreamLoaders < tot; };
+    // byte offset of its cell (a row past the entry's last: a row of
+    // line 0, not used)
+    auto cell = [&](int k) __attribute__((always_inline)) {
+        const int l = lq[k] >> 16;
+        return 8u * (StreamLines::of(L.c0, l < L.n ? l : 0) + (uint32_t)(lq[k] & 0xffff));
+    };
+    auto ld = [](gptr<const double> p, uint32_t o) __attribute__((always_inline)) {
+        return *(gptr<const double>)((gptr<const char>)p + o);
+    };
+    auto rhs2 = [&](int k0) __attribute__((always_inline)) {
+        if (k0 * kStreamLoaders >= L.n * n) return;
+        double bb[2], m[2][4], y[2][4];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (k0 + k >= kStreamElems) break;
+            const int l0 = lq[k0 + k] >> 16, l = l0 < L.n ? l0 : 0;
+            const uint32_t c = cell(k0 + k);
+            bb[k] = ld(A.bm, c);
+            m[k][0] = ld(A.im, c);
+            m[k][1] = ld(A.ip, c);
+            m[k][2] = ld(A.km, c);  // (in 2-D the K offsets are 0: in bounds, not used)
+            m[k][3] = ld(A.kp, c);
+            y[k][0] = ld(A.var, c + 8u * StreamLines::of(L.im, l));
+            y[k][1] = ld(A.var, c + 8u * StreamLines::of(L.ip, l));
+            y[k][2] = ld(A.var, c + 8u * StreamLines::of(L.km, l));
+            y[k][3] = ld(A.var, c + 8u * StreamLines::of(L.kp, l));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (k0 + k >= kStreamElems) break;
+            const double two = bb[k] - m[k][0] * y[k][0] - m[k][1] * y[k][1];
+            b[k0 + k] = do_k ? two - m[k][2] * y[k][2] - m[k][3] * y[k][3] : two;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto factors = [&](int sw) __attribute__((always_inline)) {
+        const gptr<const double> up = sw ? lu : A.jp;
 #pragma unroll
         for (int k = 0; k < kStreamElems; ++k) {
-            const int x0 = lt + k * kStreamLoaders, x = x0 < lpb * n ? x0 : lpb * n - 1;
-            const int l = (int)div_by((uint32_t)x, g.mnj, g.snj);
-            lq[k] = l << 16 | (x - l * n);
+            if (k * kStreamLoaders >= L.n * n) break;
+            const uint32_t c = cell(k);
+            f[k] = ld(A.f, c);
+            d[k] = ld(A.d, c);
+            u[k] = ld(up, c);
+            if (sw) v[k] = ld(lu2, c);
         }
-        StreamLines L;
-        int tot = 0;
-        // (opaque: what is formed from lq is formed again in each step and
-        // not held in registers over the loop)
-        auto fresh = [&]() __attribute__((always_inline)) {
-#pragma unroll
-            for (int k = 0; k < kStreamElems; ++k) asm volatile("" : "+v"(lq[k]));
-        };
-        auto at = [&](int k) __attribute__((always_inline)) { return (lq[k] >> 16) * ls + (lq[k] & 0xffff); };
-        auto here = [&](int k) __attribute__((always_inline)) { return lt + k * kStreamLoaders < tot; };
-        // byte offset of its cell (a row past the entry's last: a row of
-        // line 0, not used)
-        auto cell = [&](int k) __attribute__((always_inline)) {
-            const int l = lq[k] >> 16;
-            return 8u * (StreamLines::of(L.c0, l < L.n ? l : 0) + (uint32_t)(lq[k] & 0xffff));
-        };
-        auto ld = [](gptr<const double> p, uint32_t o) __attribute__((always_inline)) {
-            return *(gptr<const double>)((gptr<const char>)p + o);
-        };
-        auto rhs2 = [&](int k0) __attribute__((always_inline)) {
-            if (k0 * kStreamLoaders >= L.n * n) return;
-            double bb[2], m[2][4], y[2][4];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                if (k0 + k >= kStreamElems) break;
-                const int l0 = lq[k0 + k] >> 16, l = l0 < L.n ? l0 : 0;
-                const uint32_t c = cell(k0 + k);
-                bb[k] = ld(A.bm, c);
-                m[k][0] = ld(A.im, c);
-                m[k][1] = ld(A.ip, c);
-                m[k][2] = ld(A.km, c);  // (in 2-D the K offsets are 0: in bounds, not used)
-                m[k][3] = ld(A.kp, c);
-                y[k][0] = ld(A.var, c + 8u * StreamLines::of(L.im, l));
-                y[k][1] = ld(A.var, c + 8u * StreamLines::of(L.ip, l));
-                y[k][2] = ld(A.var, c + 8u * StreamLines::of(L.km, l));
-                y[k][3] = ld(A.var, c + 8u * StreamLines::of(L.kp, l));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mark = [&]() __attribute__((always_inline)) { return ld(A.f, 8u * StreamLines::of(L.c0, 0)); };  // (in every wave alike)
+    // 1: rows interchanged, 2: DGTSV itself
+    auto marked = [](double f) __attribute__((always_inline)) {
+        return __builtin_amdgcn_readfirstlane((int)swapped(f) + (int)own_dgtsv(f));
+    };
+    // (both loops below take the same entries and meet at the same five
+    // barriers an entry; apart, the solving wave's chains and the others'
+    // rows do not share registers)
+    auto next = [&]() __attribute__((always_inline)) {
+        return it + step < nmap ? map[it + step] : make_int2(-1, 0);
+    };
+    int2 en = next();
+    L.set(g, S.lstep, e.y, param, lane);
+    double mk = mark();
+    if (wave == solver) {
+        for (;;) {
+            const int nl = L.n;
+            const bool more = en.x == id, mine = lane < nl;
+            const int swp = marked(mk), ol = lane * ls;
+            // (eight lanes a line; past the last line: it again, the same values)
+            const int o8 = (lane >> 3 < nl ? lane >> 3 : nl - 1) * ls;
+            if (more) L.set(g, S.lstep, en.y, param, lane);
+            it += step;
+            e = en;
+            if (more) en = next();
+            if (more) mk = mark();
+            __syncthreads();  // the rows are there
+            if (lane == 0) odd = 0;
+            if (swp && nl > 0 && nl <= 8) {
+                whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
+            } else if (mine) {
+                if (swp) whole_forward_swap(F + ol, B + ol, whole_rows(n));
+                else whole_forward(F + ol, B + ol, whole_rows(n));
             }
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                if (k0 + k >= kStreamElems) break;
-                const double two = bb[k] - m[k][0] * y[k][0] - m[k][1] * y[k][1];
-                b[k0 + k] = do_k ? two - m[k][2] * y[k][2] - m[k][3] * y[k][3] : two;
+            __syncthreads();  // forward pass done
+            __syncthreads();  // the diagonals are there
+            if (swp && nl > 0 && nl <= 8) {
+                whole_back_swap8(B + o8, U + o8, D + o8, F + o8, rows, lane & 7);
+            } else if (mine) {
+                if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
+                else whole_back(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
             }
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        auto factors = [&](int sw) __attribute__((always_inline)) {
-            const gptr<const double> up = sw ? lu : A.jp;
+            __syncthreads();  // solved
+            __syncthreads();  // looked at
+            if (!more) break;
+        }
+    } else {
+        int swn = marked(mk);
+        factors(swn);
+#pragma unroll
+        for (int k0 = 0; k0 < kStreamElems; k0 += 2) rhs2(k0);
+        for (int nth = 0;; ++nth) {
+            const bool more = en.x == id;
+            const int nl = L.n, swp = swn;
+            const uint32_t c0 = L.c0;  // start cells of the entry being solved
+            tot = nl * n;
+            fresh();
 #pragma unroll
             for (int k = 0; k < kStreamElems; ++k) {
-                if (k * kStreamLoaders >= L.n * n) break;
-                const uint32_t c = cell(k);
-                f[k] = ld(A.f, c);
-                d[k] = ld(A.d, c);
-                u[k] = ld(up, c);
-                if (sw) v[k] = ld(lu2, c);
+                if (k * kStreamLoaders >= tot) break;
+                if (!here(k)) continue;
+                const int o = at(k), q = lq[k] & 0xffff;
+                F[o] = q > 0 ? f[k] : 0.0;
+                B[o] = b[k];
+                U[o] = q < n - 1 ? u[k] : 0.0;
+                D[o] = swp ? v[k] : d[k];
             }
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        auto mark = [&]() __attribute__((always_inline)) { return ld(A.f, 8u * StreamLines::of(L.c0, 0)); };  // (in every wave alike)
-        auto marked = [](double f) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)swapped(f)); };
-        // (both loops below take the same entries and meet at the same five
-        // barriers an entry; apart, the solving wave's chains and the others'
-        // rows do not share registers)
-        auto next = [&]() __attribute__((always_inline)) {
-            return it + step < nmap ? map[it + step] : make_int2(-1, 0);
-        };
-        int2 en = next();
-        L.set(g, S.lstep, e.y, param, lane);
-        double mk = mark();
-        if (wave == solver) {
-            for (;;) {
-                const int nl = L.n;
-                const bool more = en.x == id, mine = lane < nl;
-                const int swp = marked(mk), ol = lane * ls;
-                // (eight lanes a line; past the last line: it again, the same values)
-                const int o8 = (lane >> 3 < nl ? lane >> 3 : nl - 1) * ls;
-                if (more) L.set(g, S.lstep, en.y, param, lane);
-                it += step;
-                e = en;
-                if (more) en = next();
-                if (more) mk = mark();
-                __syncthreads();  // the rows are there
-                if (lane == 0) odd = 0;
-                if (swp && nl > 0 && nl <= 8) {
-                    whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
-                } else if (mine) {
-                    if (swp) whole_forward_swap(F + ol, B + ol, whole_rows(n));
-                    else whole_forward(F + ol, B + ol, whole_rows(n));
+            for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
+                const int q = n + (x & 7), o = (x >> 3) * ls + q;
+                if (q < rows) {  // identity rows
+                    F[o] = B[o] = U[o] = 0.0;
+                    D[o] = 1.0;
                 }
-                __syncthreads();  // forward pass done
-                __syncthreads();  // the diagonals are there
-                if (swp && nl > 0 && nl <= 8) {
-                    whole_back_swap8(B + o8, U + o8, D + o8, F + o8, rows, lane & 7);
-                } else if (mine) {
-                    if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
-                    else whole_back(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
-                }
-                __syncthreads();  // solved
-                __syncthreads();  // looked at
-                if (!more) break;
             }
-        } else {
-            int swn = marked(mk);
-            factors(swn);
+            if (more) L.set(g, S.lstep, en.y, param, lane);
+            it += step;
+            e = en;
+            if (more) en = next();
+            __syncthreads();  // the rows are there
+            if (more) mk = mark();
+            if (!swp) {
 #pragma unroll
-            for (int k0 = 0; k0 < kStreamElems; k0 += 2) rhs2(k0);
-            for (int nth = 0;; ++nth) {
-                const bool more = en.x == id;
-                const int nl = L.n, swp = swn;
-                const uint32_t c0 = L.c0;  // start cells of the entry being solved
-                tot = nl * n;
+                for (int k = 0; k < kStreamElems; ++k) d[k] = refined_rcp(d[k]);
+            }
+            if (more) {
+                fresh();
+                rhs2(0);
+                fresh();
+                rhs2(2);
+                swn = marked(mk);
+            }
+            __syncthreads();  // forward pass done
+            fresh();
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k) {
+                if (k * kStreamLoaders >= tot) break;
+                if (here(k)) F[at(k)] = d[k];
+            }
+            for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
+                const int q = n + (x & 7);
+                if (q < rows) F[(x >> 3) * ls + q] = 1.0;
+            }
+            __syncthreads();  // the diagonals are there
+            if (more) {
+                fresh();
+                factors(swn);
+                fresh();
+                rhs2(4);
+            }
+            fresh();
+            uint32_t c[kStreamElems];
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k)
+                c[k] = 8u * (StreamLines::of(c0, lq[k] >> 16) + (uint32_t)(lq[k] & 0xffff));
+            __syncthreads();  // solved
+            fresh();
+            int bad = swp == 2;
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k) {
+                if (k * kStreamLoaders >= tot) break;
+                if (here(k)) bad |= !solution_in_range(B[at(k)]);
+            }
+            if (bad) odd = 1;
+            // nothing of an entry is stored before all of it is in range:
+            // the lines on a clamped end of I or K read their own values
+            __syncthreads();  // looked at
+            if (odd) {
+                if (lt == 0) again[nth >> 5] |= 1u << (nth & 31);
+            } else {
                 fresh();
 #pragma unroll
                 for (int k = 0; k < kStreamElems; ++k) {
                     if (k * kStreamLoaders >= tot) break;
-                    if (!here(k)) continue;
-                    const int o = at(k), q = lq[k] & 0xffff;
-                    F[o] = q > 0 ? f[k] : 0.0;
-                    B[o] = b[k];
-                    U[o] = q < n - 1 ? u[k] : 0.0;
-                    D[o] = swp ? v[k] : d[k];
+                    if (here(k)) *(gptr<double>)((gptr<char>)A.var + c[k]) = B[at(k)];
                 }
-                for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
-                    const int q = n + (x & 7), o = (x >> 3) * ls + q;
-                    if (q < rows) {  // identity rows
-                        F[o] = B[o] = U[o] = 0.0;
-                        D[o] = 1.0;
-                    }
-                }
-                if (more) L.set(g, S.lstep, en.y, param, lane);
-                it += step;
-                e = en;
-                if (more) en = next();
-                __syncthreads();  // the rows are there
-                if (more) mk = mark();
-                if (!swp) {
-#pragma unroll
-                    for (int k = 0; k < kStreamElems; ++k) d[k] = refined_rcp(d[k]);
-                }
-                if (more) {
-                    fresh();
-                    rhs2(0);
-                    fresh();
-                    rhs2(2);
-                    swn = marked(mk);
-                }
-                __syncthreads();  // forward pass done
-                fresh();
-#pragma unroll
-                for (int k = 0; k < kStreamElems; ++k) {
-                    if (k * kStreamLoaders >= tot) break;
-                    if (here(k)) F[at(k)] = d[k];
-                }
-                for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
-                    const int q = n + (x & 7);
-                    if (q < rows) F[(x >> 3) * ls + q] = 1.0;
-                }
-                __syncthreads();  // the diagonals are there
-                if (more) {
-                    fresh();
-                    factors(swn);
-                    fresh();
-                    rhs2(4);
-                }
-                fresh();
-                uint32_t c[kStreamElems];
-#pragma unroll
-                for (int k = 0; k < kStreamElems; ++k)
-                    c[k] = 8u * (StreamLines::of(c0, lq[k] >> 16) + (uint32_t)(lq[k] & 0xffff));
-                __syncthreads();  // solved
-                fresh();
-                int bad = 0;
-#pragma unroll
-                for (int k = 0; k < kStreamElems; ++k) {
-                    if (k * kStreamLoaders >= tot) break;
-                    if (here(k)) bad |= !solution_in_range(B[at(k)]);
-                }
-                if (bad) odd = 1;
-                // nothing of an entry is stored before all of it is in range:
-                // the lines on a clamped end of I or K read their own values
-                __syncthreads();  // looked at
-                if (odd) {
-                    if (lt == 0) again[nth >> 5] |= 1u << (nth & 31);
-                } else {
-                    fresh();
-#pragma unroll
-                    for (int k = 0; k < kStreamElems; ++k) {
-                        if (k * kStreamLoaders >= tot) break;
-                        if (here(k)) *(gptr<double>)((gptr<char>)A.var + c[k]) = B[at(k)];
-                    }
-                }
-                if (!more) break;
             }
+            if (!more) break;
         }
-        __syncthreads();
     }
+    __syncthreads();
     // a pivot or a value out of range: DGTSV itself (the entries' inputs are as
     // they were: the other colour's values and, on clamped ends, their own)
     for (int k = 0, at = blockIdx.x; at < nmap && map[at].x == id; ++k, at += step) {

@@ -5,6 +5,7 @@ import pytest
 
 from tests.cases import make_system
 from tests.test_gpu_line_stream import _both
+from tests.test_gpu_line_whole import _msolve
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,24 @@ def test_clamped_lines_read_their_own_start_values(gpu, dims, no_k):
             r[-1, ni // 3, 5] = -np.inf
         return r.reshape(-1)
     _both(gpu, dims, no_k, 1, change, rhs)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_small_pivots_beside_interchanges(gpu, oracle_mod, kind):
+    """Blocks with a pivot out of range, with interchanged rows (kind 0 has
+    them) and with neither, in one system: the oracle's bits."""
+    def change(p):
+        nj = 31
+        for line in (0, 17, 40, 41, 42, 150, 215):
+            _small_pivot(p, line * nj + 3 + line % 20)
+        _small_pivot(p, 100 * nj)            # a first row
+        p[3, 120 * nj + 30] = 1e19           # a last row's pivot, above the range
+    _msolve(gpu, oracle_mod, (14, 29, 12), False, kind, change)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_small_pivots_in_streamed_lines(gpu, kind):
+    def change(p):
+        for line in range(1, 197 * 197, 2411):
+            _small_pivot(p, line * 257 + 1 + line % 255)
+    _both(gpu, (195, 255, 195), False, kind, change)
