@@ -23,9 +23,9 @@
 // Blocks with a row interchange carry it through both passes.  Every value is
 // the one DGTSV's own operations give, bit for bit (but for the sign of a
 // zero), as long as no operand leaves the range in which the correction is
-// exact; a block with a pivot outside it or zero (marked by k_line_factor) runs
-// DGTSV itself in LDS, and so does one whose solution holds a value outside the
-// range.
+// exact; a block whose solution holds a value outside the range divides instead
+// (whole_back_exact), and one with a pivot outside it or zero (marked by
+// k_line_factor) runs DGTSV itself in LDS.
 //
 // Measured (events of the dispatches, LINE solve, colour phase; before, one
 // DGTSV lane per line over 16-row tiles with the finished rows in global
@@ -154,6 +154,7 @@ __device__ __forceinline__ double corrected_quotient(double n, double d, double 
 struct WholeLines {
     uint32_t c0[kWholeLines], im[kWholeLines], ip[kWholeLines], km[kWholeLines], kp[kWholeLines];
     int n;
+    int odd;  // (k_line_whole: a right-hand side is out of range)
 };
 __device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j, int param, WholeLines &w) {
     const int l = threadIdx.x;
@@ -171,7 +172,10 @@ __device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j
             w.kp[l] = g.do_k ? (uint32_t)(nb_plus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
         }
         const uint64_t have = __ballot(ok);
-        if (l == 0) w.n = __popcll(have);
+        if (l == 0) {
+            w.n = __popcll(have);
+            w.odd = 0;
+        }
     }
     __syncthreads();
 }
@@ -379,8 +383,12 @@ __device__ __forceinline__ void whole_forward_swap(const double *__restrict__ pf
     pb[-1] = b;
 }
 
+// EXACT: by DGTSV's own operations, the division and (V false) the product with
+// a second super-diagonal of 0 included, from the rows after on (x1, x2).
+template <bool EXACT = false, bool V = true>
 __device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const double *__restrict__ pu,
-                                                const double *__restrict__ pv, const double *__restrict__ pd, int rows) {
+                                                const double *__restrict__ pv, const double *__restrict__ pd, int rows,
+                                                double x1 = 0.0, double x2 = 0.0) {
     constexpr int R = 4;
     struct Rows {
         pair2 b[R / 2], u[R / 2], v[R / 2], d[R / 2];
@@ -389,19 +397,18 @@ __device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const d
     pu += rows - 2;
     pv += rows - 2;
     pd += rows - 2;
-    double x1 = 0.0, x2 = 0.0;
     auto get = [&](Rows &w, int at) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < R / 2; ++k) {
             w.b[k] = *(const pair2 *)&pb[-at - 2 * k];
             w.u[k] = *(const pair2 *)&pu[-at - 2 * k];
-            w.v[k] = *(const pair2 *)&pv[-at - 2 * k];
+            w.v[k] = V ? *(const pair2 *)&pv[-at - 2 * k] : pair2{0.0, 0.0};
             w.d[k] = *(const pair2 *)&pd[-at - 2 * k];
         }
         __builtin_amdgcn_sched_barrier(0);
     };
     auto one = [&](double b, double u, double v, double d) __attribute__((always_inline)) {
-        const double x = corrected_quotient(b - u * x1 - v * x2, d, refined_rcp(d));
+        const double num = b - u * x1 - v * x2, x = EXACT ? num / d : corrected_quotient(num, d, refined_rcp(d));
         x2 = x1;
         x1 = x;
         return x;
@@ -424,6 +431,27 @@ __device__ __forceinline__ void whole_back_swap(double *__restrict__ pb, const d
         run(s1, R);
     }
     if (rows > 0) run(s0, 0);
+}
+
+// The back pass by DGTSV's own operations: for values out of range, infinities
+// and NaN (the forward passes are DGTSV's as they are; the identity rows behind
+// the line, which may hold a NaN then, are left out).  A solution that decays
+// along its line leaves the range, so such blocks must not cost much more than
+// others: with every value out of range a colour phase takes 12.8 us at 64^3
+// (10.4 in range), 85 at 150x201x180 (68) and 248 at 256^3 (196), where DGTSV
+// itself, its elimination included, took 32, 253 and 847.  Looking at the
+// right-hand sides first costs 1-2 % of a phase.
+template <bool V>
+__device__ __forceinline__ void whole_back_exact(double *__restrict__ pb, const double *__restrict__ pu,
+                                                 const double *__restrict__ pv, const double *__restrict__ pd, int n) {
+    double x1 = 0.0, x2 = 0.0;
+    for (int q = n - 1; q >= (n & ~3); --q) {  // (the last row's couplings are 0)
+        const double x = (pb[q] - pu[q] * x1 - (V ? pv[q] : 0.0) * x2) / pd[q];
+        pb[q] = x;
+        x2 = x1;
+        x1 = x;
+    }
+    whole_back_swap<true, V>(pb, pu, pv, pd, n & ~3, x1, x2);
 }
 
 // These two passes by eight lanes a line (j = lane % 8), rows in eights, for a
@@ -737,6 +765,53 @@ __device__ void whole_general(const Sys<T> &S, const WholeLines &w, int *linfo, 
     }
 }
 
+// The block's lines on their factored rows by DGTSV's own operations.
+template <int NT>
+__device__ void whole_exact(const Sys<double> &S, const WholeLines &w, int which, bool swaps) {
+    extern __shared__ __align__(16) char whole_lds[];
+    const DGrid &g = S.g;
+    const int n = g.nj, ls = whole_stride(n), nl = w.n, tot = nl * n, do_k = g.do_k;
+    double *F = (double *)whole_lds + kWholeFront, *B = F + S.lpb * ls, *U = B + S.lpb * ls, *D = U + S.lpb * ls;
+    WholeArrays<double> A = whole_arrays(S, which);
+    A.f = to_global((const double *)S.lf);
+    if (swaps) A.jp = to_global((const double *)S.lu);
+    const gptr<const double> ld = to_global((const double *)S.ld), lu2 = to_global((const double *)S.lu2);
+    auto line_of = [&](int x) { return (int)div_by((uint32_t)x, g.mnj, g.snj); };
+    const int ol = threadIdx.x * ls;
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += NT) {
+        const int l = line_of(x), q = x - l * n, at = l * ls + q;
+        const uint32_t c = w.c0[l] + (uint32_t)q;
+        WholeRow<double> r;
+        r.load(A, w, l, c);
+        F[at] = q > 0 ? r.f : 0.0;
+        B[at] = r.rhs(do_k);
+        U[at] = q < n - 1 ? r.u : 0.0;
+        D[at] = swaps ? lu2[c] : 0.0;
+    }
+    for (int x = threadIdx.x; x < 4 * nl; x += NT) {
+        const int q = n + (x & 3);
+        if (q < whole_rows(n)) F[(x >> 2) * ls + q] = 0.0;  // (no interchange behind the line)
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) {
+        if (swaps) whole_forward_swap(F + ol, B + ol, whole_rows(n));
+        else whole_forward(F + ol, B + ol, whole_rows(n));
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += NT) {
+        const int l = line_of(x), q = x - l * n;
+        F[l * ls + q] = ld[w.c0[l] + (uint32_t)q];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) whole_back_exact<true>(B + ol, U + ol, D + ol, F + ol, n);
+    __syncthreads();
+    for (int x = threadIdx.x; x < tot; x += NT) {
+        const int l = line_of(x), q = x - l * n;
+        A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+    }
+}
+
 // One colour phase: block e takes lines [e.y*S.lpb, +S.lpb) of colour
 // `param` (color_line).  which = 0 preconditions P into Phat, 1 S into Shat.
 // FP32 tables (lines longer than the k_line_pcr_sys variants hold) always run
@@ -773,7 +848,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
         const double mark = nl > 0 ? (double)A.f[w.c0[0]] : 0.0;
         constexpr int K = 3;  // rows in flight per thread
         T td[kWholeElems];    // the diagonals wait for the multipliers' place
-        int o[kWholeElems], any = 0;
+        int o[kWholeElems], any = 0, out = 0;
 #pragma unroll
         for (int k0 = 0; k0 < kWholeElems; k0 += K) {
             if (k0 * kWholeThreads >= tot) break;
@@ -793,12 +868,15 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             for (int k = 0; k < K; ++k) {
                 F[o[k0 + k]] = first[k] ? (T)0 : r[k].f;
                 any |= swapped(r[k].f);
-                B[o[k0 + k]] = r[k].rhs(do_k);
+                const T b = r[k].rhs(do_k);
+                out |= !solution_in_range((double)b);
+                B[o[k0 + k]] = b;
                 U[o[k0 + k]] = last[k] ? (T)0 : r[k].u;
                 D[o[k0 + k]] = (T)refined_rcp(r[k].d);
                 td[k0 + k] = r[k].d;
             }
         }
+        if (out) w.odd = 1;
         for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
             const int q = n + (x & 7), at = (x >> 3) * ls + q;
             if (q < held) {  // identity rows
@@ -825,7 +903,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             // with interchanges eight lanes a line where they are few (past the
             // last line: it again, the same values): 30x90x3 13.5 -> 11.4 us, 64^3
             // 13.7 -> 12.0, 40x200x40 30 -> 21
-            const bool eight = swaps && few && nl > 0 && solver >= 0 && solver < 64;
+            const bool eight = swaps && few && nl > 0 && solver >= 0 && solver < 64 && !w.odd;
             const int o8 = (solver >> 3 < nl ? solver >> 3 : nl - 1) * ls;
             if (eight) {
                 whole_forward_swap8(F + o8, B + o8, held, threadIdx.x & 7);
@@ -841,26 +919,33 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
                 const int q = n + (x & 7);
                 if (q < held) F[(x >> 3) * ls + q] = 1.0;
             }
+            // a right-hand side out of range, and its solution most likely is:
+            // DGTSV's own operations at once
+            const bool exact = __builtin_amdgcn_readfirstlane(w.odd);
             __syncthreads();
             if (eight) {
                 whole_back_swap8(B + o8, U + o8, D + o8, F + o8, held, threadIdx.x & 7);
             } else if (mine) {
-                if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
+                if (exact && swaps) whole_back_exact<true>(B + ol, U + ol, D + ol, F + ol, n);
+                else if (exact) whole_back_exact<false>(B + ol, U + ol, U + ol, F + ol, n);
+                else if (swaps) whole_back_swap(B + ol, U + ol, D + ol, F + ol, rows);
                 else whole_back(B + ol, U + ol, F + ol, D + ol, rows);
             }
             __syncthreads();
             int bad = 0;
             for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
                 const int l = line_of(x);
-                bad |= !solution_in_range((double)B[l * ls + (x - l * n)]);
+                bad |= !exact && !solution_in_range((double)B[l * ls + (x - l * n)]);
             }
-            if (!__syncthreads_or(bad)) {
-                for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
-                    const int l = line_of(x), q = x - l * n;
-                    A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
-                }
+            if (__syncthreads_or(bad)) {
+                whole_exact<kWholeThreads>(S, w, which, swaps);
                 return;
             }
+            for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+                const int l = line_of(x), q = x - l * n;
+                A.var[w.c0[l] + (uint32_t)q] = B[l * ls + q];
+            }
+            return;
         }
     }
     whole_general<T, kWholeThreads>(S, w, linfo, which);
@@ -880,12 +965,14 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
 // 4.2 of the 5.1 TB/s of a copy: 256^3 233 -> 201 us, 170^3 71 -> 59 us,
 // 150x201x180 76 -> 69 us.  Non-temporal loads of the arrays read once: 195 us
 // at 256^3, but 48 for 42 us at 200x100x200, whose arrays the last-level cache
-// holds.  An entry with a value out of range is left to DGTSV at the end.
+// holds.  An entry with a pivot or a value of its solution out of range
+// is left for the end; with a right-hand side out of range it divides at once.
 
 // Start cell and I/K neighbour offsets of line `lane` of a block, in every wave.
 struct StreamLines {
     uint32_t c0, im, ip, km, kp;
     int n;
+    int ends;  // some line is on a clamped end of I or K: its own neighbour
     __device__ __forceinline__ void set(const DGrid &g, uint64_t step, int j, int param, int lane) {
         int u = 0, v = 0;
         const int64_t first = entry_first(step, j);
@@ -898,6 +985,7 @@ struct StreamLines {
         km = g.do_k ? (uint32_t)(nb_minus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
         kp = g.do_k ? (uint32_t)(nb_plus(v, g.nk, g.cyc_z) - v) * c2 : 0u;
         n = __popcll(__ballot(ok));
+        ends = __any(ok && (im == 0 || ip == 0 || (g.do_k && (km == 0 || kp == 0))));
     }
     static __device__ __forceinline__ uint32_t of(uint32_t v, int l) { return (uint32_t)__shfl((int)v, l, 64); }
 };
@@ -908,8 +996,9 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     extern __shared__ __align__(16) char whole_lds[];
     __shared__ WholeLines w;
     __shared__ int linfo[kWholeLines];
-    __shared__ int odd;                           // the entry has a pivot or a value out of range
-    __shared__ uint32_t again[kStreamMost / 32];  // this block's entries that are left to DGTSV itself
+    __shared__ int tiny;                          // the entry has a right-hand side out of range
+    __shared__ int odd;                           // the entry has a pivot or a value of its solution out of range
+    __shared__ uint32_t again[kStreamMost / 32];  // this block's entries that are left for the end
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // another solving wave in each of the blocks that share a CU (every 256th)
     const int solver = (blockIdx.x >> 8) & 1;
@@ -923,7 +1012,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     auto *__restrict__ st = to_global(S.st);
     if (st->done || (which == 1 && st->s_exit)) return;
     if (e.y == 0 && threadIdx.x == 0) st->line_launches += 1;  // (timing: working launches)
-    if (threadIdx.x == 0) odd = 0;
+    if (threadIdx.x == 0) odd = tiny = 0;
     if (threadIdx.x < kStreamMost / 32) again[threadIdx.x] = 0;
     __syncthreads();
     const DGrid &g = S.g;
@@ -944,7 +1033,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
         lq[k] = l << 16 | (x - l * n);
     }
     StreamLines L;
-    int tot = 0;
+    int tot = 0, out = 0;  // out: a right-hand side of the next entry is out of range
     // (opaque: what is formed from lq is formed again in each step and
     // not held in registers over the loop)
     auto fresh = [&]() __attribute__((always_inline)) {
@@ -985,6 +1074,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
             if (k0 + k >= kStreamElems) break;
             const double two = bb[k] - m[k][0] * y[k][0] - m[k][1] * y[k][1];
             b[k0 + k] = do_k ? two - m[k][2] * y[k][2] - m[k][3] * y[k][3] : two;
+            out |= !solution_in_range(b[k0 + k]);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1006,8 +1096,8 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     auto marked = [](double f) __attribute__((always_inline)) {
         return __builtin_amdgcn_readfirstlane((int)swapped(f) + (int)own_dgtsv(f));
     };
-    // (both loops below take the same entries and meet at the same five
-    // barriers an entry; apart, the solving wave's chains and the others'
+    // (both loops below take the same entries and meet at the same four
+    // or five barriers an entry; apart, the solving wave's chains and the others'
     // rows do not share registers)
     auto next = [&]() __attribute__((always_inline)) {
         return it + step < nmap ? map[it + step] : make_int2(-1, 0);
@@ -1017,7 +1107,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
     double mk = mark();
     if (wave == solver) {
         for (;;) {
-            const int nl = L.n;
+            const int nl = L.n, ends = L.ends;
             const bool more = en.x == id, mine = lane < nl;
             const int swp = marked(mk), ol = lane * ls;
             // (eight lanes a line; past the last line: it again, the same values)
@@ -1029,7 +1119,8 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
             if (more) mk = mark();
             __syncthreads();  // the rows are there
             if (lane == 0) odd = 0;
-            if (swp && nl > 0 && nl <= 8) {
+            const bool exact = tiny, eight = swp && nl > 0 && nl <= 8 && !exact;
+            if (eight) {
                 whole_forward_swap8(F + o8, B + o8, rows, lane & 7);
             } else if (mine) {
                 if (swp) whole_forward_swap(F + ol, B + ol, whole_rows(n));
@@ -1037,14 +1128,16 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
             }
             __syncthreads();  // forward pass done
             __syncthreads();  // the diagonals are there
-            if (swp && nl > 0 && nl <= 8) {
+            if (eight) {
                 whole_back_swap8(B + o8, U + o8, D + o8, F + o8, rows, lane & 7);
             } else if (mine) {
-                if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
+                if (exact && swp) whole_back_exact<true>(B + ol, U + ol, D + ol, F + ol, n);
+                else if (exact) whole_back_exact<false>(B + ol, U + ol, U + ol, D + ol, n);
+                else if (swp) whole_back_swap(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
                 else whole_back(B + ol, U + ol, D + ol, F + ol, whole_rows(n));
             }
             __syncthreads();  // solved
-            __syncthreads();  // looked at
+            if (ends) __syncthreads();  // looked at
             if (!more) break;
         }
     } else {
@@ -1054,7 +1147,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
         for (int k0 = 0; k0 < kStreamElems; k0 += 2) rhs2(k0);
         for (int nth = 0;; ++nth) {
             const bool more = en.x == id;
-            const int nl = L.n, swp = swn;
+            const int nl = L.n, ends = L.ends, swp = swn;
             const uint32_t c0 = L.c0;  // start cells of the entry being solved
             tot = nl * n;
             fresh();
@@ -1068,6 +1161,8 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                 U[o] = q < n - 1 ? u[k] : 0.0;
                 D[o] = swp ? v[k] : d[k];
             }
+            if (out) tiny = 1;
+            out = 0;
             for (int x = lt; x < 8 * nl; x += kStreamLoaders) {
                 const int q = n + (x & 7), o = (x >> 3) * ls + q;
                 if (q < rows) {  // identity rows
@@ -1080,6 +1175,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
             e = en;
             if (more) en = next();
             __syncthreads();  // the rows are there
+            const int exact = tiny;
             if (more) mk = mark();
             if (!swp) {
 #pragma unroll
@@ -1093,6 +1189,7 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                 swn = marked(mk);
             }
             __syncthreads();  // forward pass done
+            if (lt == 0) tiny = 0;
             fresh();
 #pragma unroll
             for (int k = 0; k < kStreamElems; ++k) {
@@ -1117,37 +1214,45 @@ static __global__ void __launch_bounds__(kStreamThreads, 4) k_line_stream(const 
                 c[k] = 8u * (StreamLines::of(c0, lq[k] >> 16) + (uint32_t)(lq[k] & 0xffff));
             __syncthreads();  // solved
             fresh();
+            // An entry out of range is left for the end.  Where a line is its
+            // own neighbour, nothing of it may be stored before all of it has
+            // been looked at.  (A barrier for every entry: 200x100x200 40.8 ->
+            // 42.0 us.)
             int bad = swp == 2;
-#pragma unroll
-            for (int k = 0; k < kStreamElems; ++k) {
-                if (k * kStreamLoaders >= tot) break;
-                if (here(k)) bad |= !solution_in_range(B[at(k)]);
-            }
-            if (bad) odd = 1;
-            // nothing of an entry is stored before all of it is in range:
-            // the lines on a clamped end of I or K read their own values
-            __syncthreads();  // looked at
-            if (odd) {
-                if (lt == 0) again[nth >> 5] |= 1u << (nth & 31);
-            } else {
-                fresh();
+            if (ends) {
 #pragma unroll
                 for (int k = 0; k < kStreamElems; ++k) {
                     if (k * kStreamLoaders >= tot) break;
-                    if (here(k)) *(gptr<double>)((gptr<char>)A.var + c[k]) = B[at(k)];
+                    if (here(k)) bad |= !exact && !solution_in_range(B[at(k)]);
                 }
+                if (bad) odd = 1;
+                __syncthreads();  // looked at
+                bad = odd;
+                fresh();
             }
+            const bool keep = ends ? !bad : swp != 2;
+#pragma unroll
+            for (int k = 0; k < kStreamElems; ++k) {
+                if (k * kStreamLoaders >= tot) break;
+                if (!here(k) || !keep) continue;
+                const double x = B[at(k)];
+                bad |= !exact && !solution_in_range(x);
+                *(gptr<double>)((gptr<char>)A.var + c[k]) = x;
+            }
+            if (bad) again[nth >> 5] |= 1u << (nth & 31);
             if (!more) break;
         }
     }
     __syncthreads();
-    // a pivot or a value out of range: DGTSV itself (the entries' inputs are as
-    // they were: the other colour's values and, on clamped ends, their own)
+    // the entries left (their inputs are as they were: the other colour's values
+    // and, on clamped ends, their own, which were not stored)
     for (int k = 0, at = blockIdx.x; at < nmap && map[at].x == id; ++k, at += step) {
         if (!(again[k >> 5] >> (k & 31) & 1u)) continue;
         __syncthreads();
         whole_lines(g, S.lstep, map[at].y, param, w);
-        whole_general<double, kStreamThreads>(S, w, linfo, which);
+        const double m = w.n > 0 ? (double)to_global((const double *)S.lf)[w.c0[0]] : 0.0;
+        if (own_dgtsv(m)) whole_general<double, kStreamThreads>(S, w, linfo, which);
+        else whole_exact<kStreamThreads>(S, w, which, swapped(m));
     }
 }
 

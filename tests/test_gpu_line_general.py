@@ -3,7 +3,7 @@ pivot, or values of the solution, out of the corrected quotient's range)."""
 import numpy as np
 import pytest
 
-from tests.cases import make_system
+from tests.cases import make_system, rng_vec
 from tests.test_gpu_line_stream import _both
 from tests.test_gpu_line_whole import _msolve
 
@@ -83,3 +83,42 @@ def test_small_pivots_in_streamed_lines(gpu, kind):
         for line in range(1, 197 * 197, 2411):
             _small_pivot(p, line * 257 + 1 + line % 255)
     _both(gpu, (195, 255, 195), False, kind, change)
+
+
+def _decaying(n, rows):
+    """A few sources in J lines whose solution falls below the range within the line."""
+    r = np.zeros(n)
+    r[5::7 * rows] = 1.0
+    r[rows * 11 + rows - 2::13 * rows] = -3.0
+    return r
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("what", ["decay", "small", "large", "mixed"])
+@pytest.mark.parametrize("dims", [(14, 29, 12), (5, 61, 4), (2, 1, 2), (9, 383, 3)])
+def test_values_out_of_range(gpu, oracle_mod, dims, what, kind):
+    """Right-hand sides out of range and solutions that leave it: the oracle's bits."""
+    def change(p):
+        if what == "decay":      # 2^-30 a row
+            for q in (1, 5):
+                p[q] *= 1e-9
+
+    def rhs(n):
+        r = rng_vec(n, 8)
+        if what == "decay":
+            return _decaying(n, dims[1] + 2)
+        if what == "mixed":
+            r[n // 3:n // 2] *= 1e-300
+            r[n // 4] = np.nan
+            r[n - 5] = -np.inf
+            return r
+        return r * {"small": 1e-290, "large": 1e290}[what]
+    _msolve(gpu, oracle_mod, dims, False, kind, change, rhs=rhs)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_decaying_solutions_in_streamed_lines(gpu, kind):
+    def change(p):
+        for q in (1, 5):
+            p[q, ::2] *= 1e-9
+    _both(gpu, (195, 255, 195), False, kind, change, lambda n: _decaying(n, 257))
