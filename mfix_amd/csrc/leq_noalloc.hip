@@ -95,7 +95,7 @@ static int solve_fp64_noalloc(char *base, const SysDesc &d, const Shape &sh, mfi
     // others' stay in the map region
     char *map = base + o_map;
     size_t map_cap = maps;
-    if (d.pc == PC_LINE && rb_passes(d.sweep, d.g.do_k != 0) >= 0 && whole_fits(d.g.nj)) {
+    if (d.pc == PC_LINE && rb_passes(d.sweep, d.g.do_k != 0) >= 0 && G.sys[0].lk != LINE_LONG) {
         const size_t used = up256(4 * (size_t)d.g.n3 * sizeof(double));
         map = (char *)G.sys[0].line_scratch + used;
         map_cap = (size_t)line_scratch_elems(d.g) * sizeof(double) - used;

@@ -375,6 +375,14 @@ static double colour_lds(const DGrid &g) {
     const LineGeom L = line_geom(g, AX_J);
     return whole_fits(L.n) ? (double)colour_lines(L) * 4.0 * whole_stride(L.n) * sizeof(T) : 0.0;
 }
+// Whether lines of one colour are neighbours: across a cyclic axis with an odd
+// number of cells.  k_line_color_sys then, which reads all of a block's
+// right-hand sides before it stores a line, 64 lines a block: a colour of up to
+// 64 lines takes the values it started from.  (Blocks of a few lines would read
+// what others are storing.)
+static bool neighbours_alike(const DGrid &g) {
+    return (g.cyc_x && (g.ni & 1)) || (g.cyc_z && (g.nk & 1));
+}
 // table: LDS of a colour of every system of the launch (0: this grid's alone)
 template <typename T>
 static void set_line_kernel(Sys<T> &S, double table = 0.0) {
@@ -382,7 +390,7 @@ static void set_line_kernel(Sys<T> &S, double table = 0.0) {
     const LineGeom L = line_geom(g, AX_J);
     const int pin = ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block;
     const double own = colour_lds<T>(g);
-    if (!whole_fits(L.n)) {
+    if (!whole_fits(L.n) || neighbours_alike(g)) {
         S.lk = LINE_LONG;
         S.lpb = kLongLpb;
     } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, colour_lines(L), own, g.n3)) {
