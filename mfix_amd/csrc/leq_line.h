@@ -100,11 +100,25 @@ __host__ inline int whole_lpb(int n, double table, size_t elem, int pin) {
 
 // Entries of a colour of `lines` lines then: the fewest a block, of lines that
 // it holds.
-__host__ inline int64_t stream_entries(int n, int64_t lines) {
+__host__ inline int64_t stream_most(int n) {
     int64_t most = (kStreamLdsTarget / 8 - kWholeFront - kWholeTail) / (4 * stream_stride(n));
     if (most > kStreamRows / n) most = kStreamRows / n;
     if (most > kWholeLines) most = kWholeLines;
+    return most;
+}
+__host__ inline int64_t stream_entries(int n, int64_t lines) {
+    const int64_t most = stream_most(n);
     return (lines + kStreamBlocks * most - 1) / (kStreamBlocks * most) * kStreamBlocks;
+}
+// Whether a colour's lines are better in k_line_color_sys, 64 a block in no more
+// LDS than one or two take here: lines of more than 746 rows, one or two an
+// entry, from the eighth entry a block on (one line an entry: the seventh).
+// Colour phase, in whole lines and there: 1,002 rows, 6,272 lines (seven
+// entries) 411 and 429 us, 8,450 (nine) 520 and 457; 1,502 rows, 2,738 lines
+// (six) 518 and 579, 3,362 (seven) 598 and 591, 11,552 (23) 1,897 and 742.
+__host__ inline bool long_lines(int n, int64_t lines) {
+    const int64_t most = stream_most(n);
+    return most <= 2 && stream_entries(n, lines) > (5 + most) * kStreamBlocks;
 }
 // Whether the lines of a system, `lines` of `lds` bytes a colour in all, stream:
 // they take more than one round of k_line_whole's blocks.

@@ -390,7 +390,7 @@ static void set_line_kernel(Sys<T> &S, double table = 0.0) {
     const LineGeom L = line_geom(g, AX_J);
     const int pin = ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block;
     const double own = colour_lds<T>(g);
-    if (!whole_fits(L.n) || neighbours_alike(g)) {
+    if (!whole_fits(L.n) || neighbours_alike(g) || (sizeof(T) == sizeof(double) && long_lines(L.n, colour_lines(L)))) {
         S.lk = LINE_LONG;
         S.lpb = kLongLpb;
     } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, colour_lines(L), own, g.n3)) {
