@@ -147,6 +147,7 @@ int admit(mfix_leq_server *S, Group<T> &G, Req &q, int slot, hipStream_t s) {
     d.b = b;
     d.noise = nullptr;
     d.seed = q.r.noise_seed;
+    d.line_past = INT64_MAX;  // (others may join)
     sys_carve<T>(G.sys[slot], d, P, ws);
     // states live in one contiguous array so a round reads them back at once
     G.sys[slot].st = (SolverState *)S->states.ptr + (sizeof(T) == sizeof(float) ? S->max_slots : 0) + slot;

@@ -383,14 +383,28 @@ static double colour_lds(const DGrid &g) {
 static bool neighbours_alike(const DGrid &g) {
     return (g.cyc_x && (g.ni & 1)) || (g.cyc_z && (g.nk & 1));
 }
-// table: LDS of a colour of every system of the launch (0: this grid's alone)
+// Whether an FP32 table's lines (longer than the k_line_pcr_sys variants hold)
+// are whole lines in LDS: a colour of at most one block a CU.  Colour phase,
+// whole and k_line_color_sys: 602 rows, 201 lines 120 and 157 us, 501 lines 166
+// and 165, 2,178 lines 214 and 159; 1,502 rows, 201 lines 296 and 381, 501 lines
+// 423 and 349 (3-D), 2,178 lines 820 and 411.
+static bool few_lines32(int64_t lines) { return lines <= kNumCus; }
+// Lines of a colour of an FP32 system past the several-lane kernels.
+static int64_t lines_past_pcr(const DGrid &g) {
+    const LineGeom L = line_geom(g, AX_J);
+    return line_pcr_variant(L.n) < 0 ? colour_lines(L) : 0;
+}
+// table: LDS of a colour of every system of the launch (0: this grid's alone);
+// past: FP32, lines_past_pcr of them all likewise
 template <typename T>
-static void set_line_kernel(Sys<T> &S, double table = 0.0) {
+static void set_line_kernel(Sys<T> &S, double table = 0.0, int64_t past = 0) {
     const DGrid &g = S.g;
     const LineGeom L = line_geom(g, AX_J);
     const int pin = ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block;
     const double own = colour_lds<T>(g);
-    if (!whole_fits(L.n) || neighbours_alike(g) || (sizeof(T) == sizeof(double) && long_lines(L.n, colour_lines(L)))) {
+    const int64_t lines = colour_lines(L);
+    const bool rows_behind_tiles = sizeof(T) == sizeof(double) ? long_lines(L.n, lines) : !few_lines32(past > 0 ? past : lines);
+    if (!whole_fits(L.n) || neighbours_alike(g) || rows_behind_tiles) {
         S.lk = LINE_LONG;
         S.lpb = kLongLpb;
     } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, colour_lines(L), own, g.n3)) {
@@ -558,7 +572,7 @@ void sys_carve(Sys<T> &S, const SysDesc &d, const Part &P, char *base) {
         S.ld = S.line_scratch + n3;
         S.lu = S.line_scratch + 2 * n3;
         S.lu2 = S.line_scratch + 3 * n3;
-        set_line_kernel(S, d.line_lds);
+        set_line_kernel(S, d.line_lds, d.line_past);
     }
     if (mixed) {
         S.a = (const T *)take(8 * n3 * sizeof(float));
@@ -1251,6 +1265,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<size_t> offs((size_t)nsys);
     size_t total = 0;
     double line_lds = 0.0;
+    int64_t line_past = 0;
     const int bs = 256;
     for (int q = 0; q < nsys; ++q) {
         const mfix_leq_batch_item &it = items[q];
@@ -1275,6 +1290,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
         const Shape sh = C.shape_for(g.n3, it.mixed != 0);
         parts[q] = make_part(g.n3, bs, sh.bs == bs ? sh.cpt : 1);
         if (pc == PC_LINE && !it.mixed) line_lds += colour_lds<double>(g);
+        if (pc == PC_LINE && it.mixed) line_past += lines_past_pcr(g);
         offs[q] = total;
         total += sys_bytes(g, parts[q], pc, it.mixed != 0);
     }
@@ -1292,6 +1308,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<int> ids64, ids32;
     for (int q = 0; q < nsys; ++q) {
         descs[q].line_lds = items[q].mixed ? 0.0 : line_lds;
+        descs[q].line_past = line_past;
         char *base = (char *)C.bws.ptr + offs[q];
         if (items[q].mixed) {
             G32.sys.emplace_back();
