@@ -147,6 +147,7 @@ struct Context {
     Group<double> gna;             // table of the no-allocation entry (device side in its fixed array)
     Prof prof[kNumProf];
     Shape tuned[2][kSizeClasses];  // [fp32][size class]; bs == 0 means untuned
+    int resident_spins = kResidentSpins;  // tries of a wait in k_resident (MFIX_LEQ_RESIDENT_SPINS)
     int use_graphs = 1;            // capture chunks of iterations in HIP graphs
     int unit_diag = 1;             // mixed DIAG: negate instead of reading a 1/A0 plane of -1s
     hipError_t last_hip_error = hipSuccess;

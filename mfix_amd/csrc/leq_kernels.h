@@ -56,7 +56,6 @@ struct SolverState {
     int nonunit_diag;       // some unit-scaled A0 differs from -1 (DIAG must read the A0 plane)
     int k1_launches;        // launches of the first stencil pass that worked on this system (timing)
     int line_launches;      // colour-phase launches that worked on this system (timing)
-    int resident_gone;      // a block of k_resident gave up waiting for another
     double l2[4 * kFinishBlocks];  // level-2 sums of the finish launches
 };
 

@@ -41,15 +41,31 @@ constexpr int kResidentBlock = 256;
 constexpr int kResidentPerCu = 2;  // blocks a CU holds (200 VGPRs)
 constexpr int kResidentBlocks = kResidentPerCu * kNumCus;
 constexpr unsigned long long kNoSum = 0x7ff4a5a5a5a5a5a5ull;
-constexpr int kResidentSpins = 1 << 23;  // tries of a wait (about a microsecond each) before the solve is given up
+constexpr int kResidentSpins = 1 << 23;  // tries of a wait (about a microsecond each) before the launch gives up
 
-// Slots of the partial sums, one 128-byte line per set and block (in the
-// solve's P, S and T arrays, which this path does not use: 48 of the 768
-// values of a block), and the totals, one line per set and XCD (in the
-// partial sums' array).
+// The launch gives up when a wait runs out (another stream or process holds the
+// CUs).  Nothing that a launched solve starts from is touched before all blocks
+// have ended, so that one can follow: R stays, its exchange goes through T; the
+// solution and the final state wait in S and in the partial sums' array for
+// k_resident_end, which takes them over unless a block gave up.
+
+// Slots of the partial sums, one 128-byte line per set and block, in the
+// solve's P array, 48 of the 256 values of a block (a system of one block that
+// has fewer goes on into S, which is written when no slot is read any more);
+// and in the partial sums' array the totals, one line per set and XCD, the two
+// flags and the final state.
 constexpr int kSlotLine = 16;
 __host__ __device__ inline int64_t resident_slots(int64_t nblk) { return 3 * nblk * kSlotLine; }
 constexpr int kResidentTotals = 3 * kNumXcd * kSlotLine;
+struct ResidentEnd {
+    int gone;   // a block gave up waiting for another
+    int ended;  // the iteration ran, to `st`
+    SolverState st;
+};
+__device__ __forceinline__ auto resident_end(double *partials) {
+    return to_global((ResidentEnd *)(partials + kResidentTotals));
+}
+static_assert(sizeof(double) * kResidentTotals + sizeof(ResidentEnd) <= sizeof(double) * kUpdateBlocks, "in the partial sums");
 
 static __global__ void __launch_bounds__(256) k_resident_slots(const Sys<double> *__restrict__ sys) {
     const int64_t n = resident_slots(sys->P.nblk);
@@ -59,6 +75,7 @@ static __global__ void __launch_bounds__(256) k_resident_slots(const Sys<double>
     for (int64_t k = k0; k < n; k += (int64_t)gridDim.x * 256) q[k] = kNoSum;
     if (k0 < kResidentTotals) tot[k0] = kNoSum;
     if (k0 + 256 < kResidentTotals && blockIdx.x == 0) tot[k0 + 256] = kNoSum;
+    if (k0 == 0) resident_end(sys->partials)->gone = resident_end(sys->partials)->ended = 0;
 }
 static_assert(kResidentTotals <= 512, "cleared by the first block");
 
@@ -73,10 +90,10 @@ struct ResidentShared {
     SolverState st;
 };
 
-// Waits for a slot's value; nothing after kResidentSpins tries (ok = false).
-__device__ __forceinline__ double await_agent(gptr<double> p, int &spins) {
+// Waits for a slot's value, up to `most` tries in all.
+__device__ __forceinline__ double await_agent(gptr<double> p, int &spins, int most) {
     double x = load_agent(p);
-    while ((unsigned long long)__double_as_longlong(x) == kNoSum && ++spins < kResidentSpins) x = load_agent(p);
+    while ((unsigned long long)__double_as_longlong(x) == kNoSum && ++spins < most) x = load_agent(p);
     return x;
 }
 
@@ -98,7 +115,7 @@ __device__ __forceinline__ void resident_clear(gptr<double> slots, gptr<double> 
 // a wait was given up.
 template <int NV, int PAIR0, int NPAIR>
 __device__ __forceinline__ void resident_sum(double (&v)[NV], gptr<double> slots, gptr<double> totals, int64_t nblk,
-                                             int64_t blk, int red, ResidentShared &sh) {
+                                             int64_t blk, int red, int most, ResidentShared &sh) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int set = red % 3;
     if (NPAIR > 0) {
@@ -148,7 +165,7 @@ __device__ __forceinline__ void resident_sum(double (&v)[NV], gptr<double> slots
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
                 s[q][j] = 0.0;
-                if (b < nblk) s[q][j] = 0.0 + await_agent(slots + (set * nblk + b) * kSlotLine + q, spins);
+                if (b < nblk) s[q][j] = 0.0 + await_agent(slots + (set * nblk + b) * kSlotLine + q, spins, most);
             }
         }
         __syncthreads();  // (the waves' sums above were read)
@@ -176,13 +193,13 @@ __device__ __forceinline__ void resident_sum(double (&v)[NV], gptr<double> slots
     } else if (t == 0) {
         const gptr<double> mine = totals + (set * kNumXcd + (int)(blockIdx.x % kNumXcd)) * kSlotLine;
 #pragma unroll
-        for (int q = 0; q < NV; ++q) v[q] = await_agent(mine + q, spins);
+        for (int q = 0; q < NV; ++q) v[q] = await_agent(mine + q, spins, most);
     }
-    if (spins >= kResidentSpins) sh.gone = 1;
+    if (spins >= most) sh.gone = 1;
 }
 
 template <int OP>
-__global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(const Sys<double> *__restrict__ sys) {
+__global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(const Sys<double> *__restrict__ sys, int most) {
     __shared__ ResidentShared sh;
     const Sys<double> &S = *sys;
     const DGrid &g = S.g;
@@ -203,18 +220,19 @@ __global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(con
     const bool dots = mine && (g.dot_all || n.interior);
     const bool dots1 = mine && ((g.dot_all && !sh.st.minimize) || n.interior);  // (the second pass's domain)
     const gptr<const double> a = to_global(S.a);
-    const gptr<double> gr = to_global(S.r), gv = to_global(S.v), slots = to_global(S.p), totals = to_global(S.partials);
+    const gptr<const double> r0 = to_global((const double *)S.r);
+    const gptr<double> gr = to_global(S.t), gv = to_global(S.v), slots = to_global(S.p), totals = to_global(S.partials);
     double A[7], D[6];
 #pragma unroll
     for (int p = 0; p < 7; ++p) A[p] = a[p * n3 + c];
 #pragma unroll
     for (int k = 0; k < 6; ++k) D[k] = OP == OP_DIAG ? a[3 * n3 + nb[k]] : 1.0;
-    double r = load_agent(gr + c), x = to_global(S.x)[c], p = 0.0, v = 0.0;
+    double r = r0[c], x = to_global(S.x)[c], p = 0.0, v = 0.0;
     const double rt = to_global(S.rt)[c];
     double rn[6], pn[6], vn[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-        rn[k] = load_agent(gr + nb[k]);
+        rn[k] = r0[nb[k]];
         pn[k] = vn[k] = 0.0;
     }
     auto pre = [&](double z, double d) { return OP == OP_DIAG ? diag_apply(z, d) : z; };
@@ -234,7 +252,7 @@ __global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(con
         v = row(pn, ph);
         if (mine) store_agent(gv + c, v);
         double s1[1] = {dots ? rt * v : 0.0};
-        resident_sum<1, 0, 0>(s1, slots, totals, nblk, blk, red, sh);
+        resident_sum<1, 0, 0>(s1, slots, totals, nblk, blk, red, most, sh);
         if (threadIdx.x == 0) fin_apply<FIN_ALPHA, 1>(&sh.st, s1, nullptr);
         __syncthreads();
         if (sh.gone) break;
@@ -250,7 +268,7 @@ __global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(con
         const double shv = pre(s, A[3]);
         const double tt = row(sn, shv);
         double s3[3] = {dots1 ? tt * s : 0.0, dots1 ? tt * tt : 0.0, dots ? s * s : 0.0};
-        resident_sum<3, 2, 1>(s3, slots, totals, nblk, blk, red + 1, sh);
+        resident_sum<3, 2, 1>(s3, slots, totals, nblk, blk, red + 1, most, sh);
         if (threadIdx.x == 0) fin_apply<FIN_OMEGA, 3>(&sh.st, s3, nullptr);
         __syncthreads();
         if (sh.gone) break;
@@ -269,7 +287,7 @@ __global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(con
                 s2[1] = rt * r;
             }
         }
-        resident_sum<2, 0, 2>(s2, slots, totals, nblk, blk, red + 2, sh);
+        resident_sum<2, 0, 2>(s2, slots, totals, nblk, blk, red + 2, most, sh);
         if (threadIdx.x == 0) fin_apply<FIN_XR, 2>(&sh.st, s2, nullptr);
         __syncthreads();
         if (sh.gone) break;
@@ -277,15 +295,32 @@ __global__ void __launch_bounds__(kResidentBlock, kResidentPerCu) k_resident(con
 #pragma unroll
         for (int k = 0; k < 6; ++k) rn[k] = load_agent(gr + nb[k]);
     }
-    if (mine) to_global(S.x)[c] = x;
+    const auto end = resident_end(S.partials);
     if (sh.gone) {
-        if (threadIdx.x == 0) atomicOr((int *)&to_global(S.st)->resident_gone, 1);
+        if (threadIdx.x == 0) end->gone = 1;
         return;
     }
+    if (mine) to_global(S.s)[c] = x;
     if (blk == 0) {
         __syncthreads();
-        const gptr<double> dst = to_global((double *)S.st);
+        const gptr<double> dst = (gptr<double>)&end->st;
         for (int k = threadIdx.x; k < (int)(sizeof(SolverState) / 8); k += kResidentBlock) dst[k] = ((double *)&sh.st)[k];
+        if (threadIdx.x == 0) end->ended = 1;
+    }
+}
+
+// The solution and the state of a launch that ended (one that had nothing to do
+// leaves them as they are).
+static __global__ void __launch_bounds__(kResidentBlock) k_resident_end(const Sys<double> *__restrict__ sys) {
+    const Sys<double> &S = *sys;
+    const auto end = resident_end(S.partials);
+    if (end->gone || !end->ended) return;
+    const int64_t c = (int64_t)blockIdx.x * kResidentBlock + threadIdx.x;
+    if (c < S.g.n3) to_global(S.x)[c] = to_global((const double *)S.s)[c];
+    if (blockIdx.x == 0) {
+        const gptr<double> dst = to_global((double *)S.st);
+        const gptr<const double> src = (gptr<const double>)&end->st;
+        for (int k = threadIdx.x; k < (int)(sizeof(SolverState) / 8); k += kResidentBlock) dst[k] = src[k];
     }
 }
 

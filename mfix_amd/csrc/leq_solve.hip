@@ -115,6 +115,8 @@ int Context::init(int dev) {
     std::memset(host_count, 0, sizeof(int) * 2 * kPollInts);
     poll = 0;
     if (const char *v = std::getenv("MFIX_LEQ_GRAPHS")) use_graphs = std::atoi(v);
+    const char *spins = std::getenv("MFIX_LEQ_RESIDENT_SPINS");
+    resident_spins = spins ? std::atoi(spins) : kResidentSpins;
     initialised = true;
     return 0;
 }
@@ -1120,13 +1122,15 @@ static bool launch_resident(Group<double> &G, hipStream_t s) {
     const int64_t nblk = G.sys[0].P.nblk;
     const Sys<double> *tab = G.d_sys;
     hipLaunchKernelGGL(k_resident_slots, dim3((unsigned)((resident_slots(nblk) + 255) / 256)), dim3(256), 0, s, tab);
-    void *args[] = {(void *)&tab};
+    int most = ctx().resident_spins;
+    void *args[] = {(void *)&tab, (void *)&most};
     const void *f = G.sys[0].pc == PC_DIAG ? (const void *)k_resident<OP_DIAG> : (const void *)k_resident<OP_PLAIN>;
-    if (hipLaunchCooperativeKernel(f, dim3((unsigned)nblk), dim3(kResidentBlock), args, 0, s) ==
-        hipSuccess)
-        return true;
-    (void)hipGetLastError();
-    return false;
+    if (hipLaunchCooperativeKernel(f, dim3((unsigned)nblk), dim3(kResidentBlock), args, 0, s) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    hipLaunchKernelGGL(k_resident_end, dim3((unsigned)nblk), dim3(kResidentBlock), 0, s, tab);
+    return true;
 }
 
 template <typename T>
@@ -1165,14 +1169,22 @@ static int solve_one(Group<T> &G, const SysDesc &d, const Shape &sh, mfix_leq_st
     if constexpr (sizeof(T) == sizeof(double))
         if (graphs && !C.prof[0].on && resident_fits(G.sys[0], G.bs)) whole = launch_resident(G, s);
     if (!whole) rc = run_group<T>(G, d.itmax, s, graphs);
-    (void)hipEventRecord(e1, s);
-    (void)hipEventSynchronize(e1);
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
+    SolverState *h = C.host_state;
+    auto read = [&]() {
+        (void)hipEventRecord(e1, s);
+        (void)hipEventSynchronize(e1);
+        (void)hipEventElapsedTime(&ms, e0, e1);
+        if (!rc) rc = read_states<T>(G, std::vector<int>{0}, h, s);
+    };
+    read();
+    if (whole && !rc && !h->done) {  // a wait of the resident launch ran out, and it changed nothing
+        rc = run_group<T>(G, d.itmax, s, graphs);
+        read();
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    SolverState *h = C.host_state;
-    if (rc || (rc = read_states<T>(G, std::vector<int>{0}, h, s))) {
+    if (rc) {
         for (auto &p : C.prof) p.collect();
         return rc;
     }
@@ -1195,7 +1207,6 @@ static int solve_one(Group<T> &G, const SysDesc &d, const Shape &sh, mfix_leq_st
     fill_stats(*h, stats);
     if (stats) stats->device_ms = ms;
     if (h->msolve_fatal) return MFIX_LEQ_EDGTSV;
-    if (h->resident_gone) return hip_fail(hipErrorLaunchTimeOut, "resident solve");
     return 0;
 }
 
