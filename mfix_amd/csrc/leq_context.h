@@ -137,7 +137,7 @@ struct Context {
     DevBuf bws;                    // batch workspace
     DevBuf partials, state, misc, tmp;
     SolverState *host_state = nullptr;  // pinned mirrors of device states
-    int *host_count = nullptr;          // pinned: kPollInts of the FP64 table, then of the FP32 table
+    int *host_count = nullptr;          // pinned: kPollInts of the FP64 table's even and odd polls, then of the FP32 table's
     Stage stage;
     int poll = 0;                       // number of the last poll issued
     Group<double> g64;             // single-solve tables

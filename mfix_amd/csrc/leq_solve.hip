@@ -110,9 +110,9 @@ int Context::init(int dev) {
     if (e != hipSuccess) return hip_fail(e, "hipStreamCreate");
     e = hipHostMalloc((void **)&host_state, sizeof(SolverState) * kHostStates, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
-    e = hipHostMalloc((void **)&host_count, sizeof(int) * 2 * kPollInts, hipHostMallocDefault);
+    e = hipHostMalloc((void **)&host_count, sizeof(int) * 4 * kPollInts, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
-    std::memset(host_count, 0, sizeof(int) * 2 * kPollInts);
+    std::memset(host_count, 0, sizeof(int) * 4 * kPollInts);
     poll = 0;
     if (const char *v = std::getenv("MFIX_LEQ_GRAPHS")) use_graphs = std::atoi(v);
     const char *spins = std::getenv("MFIX_LEQ_RESIDENT_SPINS");
@@ -992,7 +992,9 @@ static int capture_chunk(Group<double> *G64, Group<float> *G32, int iters, hipSt
 static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
     Context &C = ctx();
     int rc;
-    int *h64 = C.host_count, *h32 = C.host_count + kPollInts;
+    // a poll's words: the next one, which may be under way, writes others, so
+    // that its count and its flags are of one moment
+    auto words = [&](int table, int poll) { return C.host_count + (2 * table + (poll & 1)) * kPollInts; };
     if (G64 && G64->iter.ids.empty()) G64 = nullptr;
     if (G32 && G32->iter.ids.empty()) G32 = nullptr;
     if (!G64 && !G32) return 0;
@@ -1002,8 +1004,8 @@ static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipS
     const bool line = (G64 && G64->iter.n_line) || (G32 && G32->iter.n_line);
     const int first = line ? 1 : 4, most = line ? 4 : 16;
     auto count = [&](int poll) {
-        if (G64) enqueue_count<double>(*G64, G64->iter, h64, poll, s);
-        if (G32) enqueue_count<float>(*G32, G32->iter, h32, poll, s);
+        if (G64) enqueue_count<double>(*G64, G64->iter, words(0, poll), poll, s);
+        if (G32) enqueue_count<float>(*G32, G32->iter, words(1, poll), poll, s);
     };
     // `iters` iterations, by a replay of the captured chunk of that length
     // where there is one (kept in the float table's slots when present)
@@ -1044,6 +1046,7 @@ static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipS
             issued += chunk;
             count(++C.poll);
         }
+        const int *h64 = words(0, poll), *h32 = words(1, poll);
         if ((rc = wait_poll(G64 ? h64 : nullptr, G32 ? h32 : nullptr, poll, s))) return rc;
         const int run64 = G64 ? __atomic_load_n(h64, __ATOMIC_RELAXED) : 0;
         const int run32 = G32 ? __atomic_load_n(h32, __ATOMIC_RELAXED) : 0;

@@ -1,0 +1,49 @@
+"""The host side of the solver without a GPU: a stand-in HIP runtime
+(tests/fake_hip.c), preloaded into a process of its own, whose kernels do
+nothing, shows what the driver launches, polls and waits for."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+
+PRELUDE = """
+import ctypes as C, numpy as np
+from mfix_amd import _lib, leq
+L = _lib.load()
+leq.init(0)
+def arrays(n3):
+    return [leq.DeviceArray(k * n3) for k in (1, 7, 1)]
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory, native_lib):
+    so = tmp_path_factory.mktemp("fake") / "fake_hip.so"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-pthread", "-o", str(so), str(ROOT / "tests" / "fake_hip.c")],
+                   check=True)
+
+    def run(mode, code, log):
+        env = dict(os.environ, LD_PRELOAD=str(so), FAKE_HIP=mode, FAKE_HIP_LOG=str(log))
+        p = subprocess.run([sys.executable, "-c", PRELUDE + code], cwd=ROOT, env=env, capture_output=True, text=True,
+                           timeout=120)
+        assert p.returncode == 0, p.stderr
+        return p.stdout.strip(), log.read_text().splitlines() if log.exists() else []
+    return run
+
+
+@pytest.mark.parametrize("pc", ["DIAG", "LINE"])
+def test_a_poll_leaves_the_words_of_the_one_before_alone(fake, tmp_path, pc):
+    """The next poll is under way while the host reads one: its words are others."""
+    _, log = fake("count", f"""
+leq.grid_init(60, 60, 60)
+dx, da, db = arrays(62 ** 3)
+leq.bicgs_dev(dx, da, db, pc="{pc}", tol=1e-10, itmax=40)
+""", tmp_path / "log")
+    polls = [(int(p, 16), int(n), int(k)) for _, p, n, k in (s.split() for s in log if s.startswith("poll"))]
+    assert len(polls) >= 4 and [k for _, _, k in polls] == list(range(polls[0][2], polls[0][2] + len(polls)))
+    for (p, n, _), (q, m, _) in zip(polls, polls[1:]):
+        assert p + 4 * (2 + n) <= q or q + 4 * (2 + m) <= p
