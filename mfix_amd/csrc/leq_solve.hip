@@ -989,7 +989,7 @@ static int capture_chunk(Group<double> *G64, Group<float> *G32, int iters, hipSt
 // iterations are 5-9 short launches, hundreds a solve) with four.  Chunks of
 // a fixed 16 iterations, each polled with a copy, ran a 128^3 LINE momentum
 // solve of four iterations in 2,101 us; now 1,695.  No chunk runs past ITMAX.
-static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
+static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
     Context &C = ctx();
     int rc;
     // a poll's words: the next one, which may be under way, writes others, so
@@ -1062,6 +1062,14 @@ static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipS
         // rebuild are not looked at (they ran before its upload)
         if (rebuilt) count(++C.poll);
     }
+}
+
+// With an error the chunk and the poll under way end first: they write the
+// caller's arrays and the polls' words.
+static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
+    const int rc = drive_tables(G64, G32, max_iters, s, graphs);
+    if (rc) (void)hipStreamSynchronize(s);
+    return rc;
 }
 
 template <typename T>

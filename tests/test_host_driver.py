@@ -47,3 +47,19 @@ leq.bicgs_dev(dx, da, db, pc="{pc}", tol=1e-10, itmax=40)
     assert len(polls) >= 4 and [k for _, _, k in polls] == list(range(polls[0][2], polls[0][2] + len(polls)))
     for (p, n, _), (q, m, _) in zip(polls, polls[1:]):
         assert p + 4 * (2 + n) <= q or q + 4 * (2 + m) <= p
+
+
+def test_an_error_returns_when_nothing_runs_any_more(fake, tmp_path):
+    """No poll is answered: the call ends with an error, and with a wait for what
+    it had under way, also without the events that other entries wait for."""
+    out, log = fake("silent", """
+leq.grid_init(20, 20, 20)
+dx, da, db = arrays(22 ** 3)
+st, o = _lib.Stats(), _lib.Opts()
+f = L.mfix_leq_bicgs_dev_noalloc
+f.argtypes = [C.c_char_p, C.c_double, C.c_char_p, C.c_int] + [C.c_void_p] * 6
+print(f(b"RSRS", 1e-10, b"DIAG", 40, dx.ptr, da.ptr, db.ptr, C.addressof(o), C.addressof(st), None))
+""", tmp_path / "log")
+    assert int(out) < 0
+    last = max(k for k, s in enumerate(log) if s.startswith(("launch", "poll")))
+    assert "wait" in log[last:]
