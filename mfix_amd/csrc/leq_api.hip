@@ -143,9 +143,12 @@ int staged_copy(const std::vector<Span> &spans, bool up, hipStream_t s) {
             if (e != hipSuccess || k >= n) continue;
             const Chunk &c = ch[w + k * nw];
             if (up) std::memcpy(slot, c.host, c.bytes);
-            hipLaunchKernelGGL(k_move, dim3(kMoveBlocks), dim3(256), 0, s, (const double *)(up ? slot : c.dev),
-                               (double *)(up ? c.dev : slot), (int)(c.bytes / sizeof(double)));
-            e = hipEventRecord(st.moved[q], s);
+            const void *from = up ? slot : c.dev, *to = up ? c.dev : slot;
+            int n8 = (int)(c.bytes / sizeof(double));
+            void *args[] = {&from, &to, &n8};
+            // (its own status: hipGetLastError is by thread)
+            e = hipLaunchKernel((const void *)k_move, dim3(kMoveBlocks), dim3(256), args, 0, s);
+            if (e == hipSuccess) e = hipEventRecord(st.moved[q], s);
         }
         err[w] = e;
     };

@@ -63,3 +63,17 @@ print(f(b"RSRS", 1e-10, b"DIAG", 40, dx.ptr, da.ptr, db.ptr, C.addressof(o), C.a
     assert int(out) < 0
     last = max(k for k, s in enumerate(log) if s.startswith(("launch", "poll")))
     assert "wait" in log[last:]
+
+
+@pytest.mark.skipif(len(os.sched_getaffinity(0)) < 2, reason="one processor: the caller's thread copies")
+def test_a_failed_launch_of_a_copying_thread_is_an_error(fake, tmp_path):
+    out, log = fake("threads", """
+leq.grid_init(60, 60, 60)
+n = 62 ** 3
+ier = C.c_int(7)
+x, a, b = np.zeros(n), np.zeros(7 * n), np.zeros(n)
+print(L.mfix_leq_bicgs(b"u", 1, 1, *(v.ctypes.data_as(_lib.c_double_p) for v in (x, a, b)), b"RSRS", 4, 1e-4, b"DIAG", 99,
+                       C.byref(ier)))
+""", tmp_path / "log")
+    assert any("k_move" in s for s in log)      # the caller's own launches
+    assert int(out) == -103                     # MFIX_LEQ_EHIP
