@@ -93,6 +93,15 @@ hipError_t slot_free(hipEvent_t ev) {  // (an event that was never recorded is d
     return e;
 }
 
+// Whether the runtime can move an array by itself at the link's rate: one that it
+// knows (pinned, managed, a device's).
+bool known_to_hip(const void *p) {
+    hipPointerAttribute_t at = {};
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 // n doubles (both ends 16-byte aligned), over the link: one end is pinned host memory.
 constexpr int kMoveBlocks = 64;
 __global__ void __launch_bounds__(256) k_move(const double *__restrict__ from, double *__restrict__ to, int n) {
@@ -101,15 +110,16 @@ __global__ void __launch_bounds__(256) k_move(const double *__restrict__ from, d
     if (t == 0 && (n & 1)) to[n - 1] = from[n - 1];
 }
 
-// Pageable arrays to the device (up) or back, in chunks through the pinned
-// slots, so that the link moves some while processors copy others: several,
+// Host arrays to the device (up) or back: pageable ones in chunks through the
+// pinned slots, so that the link moves some while processors copy others: several,
 // where the process may run on several and the arrays are worth it, as one
 // copies slower than the link moves.  A kernel moves a chunk: the runtime's
-// asynchronous copies leave gaps of 18 us between chunks of 1 MiB.  The host
-// arrays are free (up) or filled (down) when it returns.  LEQ_BICGS on host
-// arrays of 64^3, 20.7 MB each way: 2376 us with the runtime's copies of
+// asynchronous copies leave gaps of 18 us between chunks of 1 MiB.  Pageable
+// arrays are free (up) or filled (down) when it returns, others when the stream
+// has come so far.  LEQ_BICGS on host arrays of 64^3, 20.7 MB each way: 2376 us with the runtime's copies of
 // pageable memory (16 MB: 450 us up, 921 down, where the link takes 293), 1840
-// with them through the slots in one thread, 1590 so.
+// with them through the slots in one thread, 1590 so; pinned arrays 1711 through
+// the slots, 1186 from where they are (128^3 8710 and 6660; 7136 before both).
 int staged_copy(const std::vector<Span> &spans, bool up, hipStream_t s) {
     Context &C = ctx();
     Stage &st = C.stage;
@@ -120,9 +130,17 @@ int staged_copy(const std::vector<Span> &spans, bool up, hipStream_t s) {
         size_t bytes;
     };
     std::vector<Chunk> ch;
-    for (const Span &sp : spans)
+    for (const Span &sp : spans) {
+        if (known_to_hip(sp.host)) {
+            const hipError_t e = up ? hipMemcpyAsync(sp.dev, sp.host, sp.bytes, hipMemcpyHostToDevice, s)
+                                    : hipMemcpyAsync(sp.host, sp.dev, sp.bytes, hipMemcpyDeviceToHost, s);
+            if (e != hipSuccess) return hip_fail(e, up ? "host to device copy" : "device to host copy");
+            continue;
+        }
         for (size_t o = 0; o < sp.bytes; o += kStageBytes)
             ch.push_back({(char *)sp.dev + o, (char *)sp.host + o, std::min(kStageBytes, sp.bytes - o)});
+    }
+    if (ch.empty()) return 0;
     cpu_set_t cpus;
     const int have = sched_getaffinity(0, sizeof(cpus), &cpus) ? 1 : CPU_COUNT(&cpus);
     const int nw = ch.size() >= kStageSlots ? std::max(1, std::min(kStageWorkers, have)) : 1;
