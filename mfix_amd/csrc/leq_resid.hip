@@ -6,6 +6,8 @@
 // the partials in a fixed order and applies the reference's normalisation.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/mfix_leq.h"
 #include "leq_context.h"
 
@@ -25,25 +27,30 @@ struct ResidArgs {
     const int *flag;
     double *partials;                          // kResidVals x nblk
     int64_t nblk;
+    int run;                                   // consecutive blocks of one XCD
     mfix_leq_resid *out;
 };
 
 __device__ __forceinline__ void better(double &v, double &i, double ov, double oi) { resid_better(v, i, ov, oi); }
 
-// The rows of kResidStep cells of a thread are loaded together, whether or not
-// the sums take them (a cell past the end: the last one's), and the blocks
-// are dealt to the XCDs in slabs, so that a row's I/K neighbours are in the
-// L2 that loaded them: with one cell at a time behind the reference's tests,
-// each a round trip, the pass ran 139 us at 200x230x170 (76 B a cell: 4.4
-// TB/s) where it now takes 111-119 us (5.2-5.5 TB/s, the copy rate).  Sums, order and candidates are the same.
-constexpr int kResidStep = 2;
+// A thread looks at the flags of its eight cells first and then loads the rows
+// of two cells together, unless the sums take neither; XCDs take turns of about
+// eight planes, so that a row's I/K neighbours are mostly in the L2 that loaded
+// them, and none has more than its share of a domain's fluid.  200x230x170, us a
+// call of C (one cell at a time behind the reference's tests; all rows in pairs,
+// one slab an XCD; now): all fluid 165, 134, 135 (the pass 139, 111, 112: 76 B
+// a cell at the copy rate); a cylinder of a fifth 68, 131, 62; the lower 30 %
+// 95, 130, 92.  PP, whose rows are B alone, loads all eight at once: 61, 42, 42.
+// Sums, order and candidates are the same.
+constexpr int kResidStep = 2, kResidPlanes = 8;
 
 template <int KIND>
 __global__ void __launch_bounds__(kResidBlock) k_resid(ResidArgs R) {
     __shared__ double lds[(kResidBlock / 64) * 3];
     __shared__ double lv[kResidBlock / 64], li[kResidBlock / 64];
-    if (!xcd_valid(R.nblk)) return;
-    const int64_t blk = xcd_block(R.nblk);
+    const int turn = (int)(blockIdx.x / kNumXcd), part = turn / R.run;
+    const int64_t blk = ((int64_t)part * kNumXcd + blockIdx.x % kNumXcd) * R.run + (turn - part * R.run);
+    if (blk >= R.nblk) return;
     const DGrid &g = R.g;
     // candidates must beat the scan's start value: RESID_IJK(1) = 0 for C
     // and S (:114-115), -1 for PP (:423)
@@ -58,53 +65,62 @@ __global__ void __launch_bounds__(kResidBlock) k_resid(ResidArgs R) {
     const auto *__restrict__ eps = to_global(R.ep_s);
     const int64_t n3 = g.n3;
     const int64_t c0 = blk * (kResidBlock * kResidCells) + threadIdx.x;
-    for (int q = 0; q < kResidCells; q += kResidStep) {
+    auto cell = [&](int q) {  // increasing per thread; past the end: the last one's row, not taken
+        const int64_t c = c0 + (int64_t)q * kResidBlock;
+        return c < n3 ? c : n3 - 1;
+    };
+    // cells of the sums: IS_ON_myPE_wobnd, FLUID_AT
+    uint32_t in = 0;
+    double bp[kResidCells];
+#pragma unroll
+    for (int q = 0; q < kResidCells; ++q) {
+        const int64_t c = cell(q);
+        if (KIND == RESID_PP) bp[q] = ld_stream(&b[c]);
+        if (fluid_at(flag[c]) && c0 + (int64_t)q * kResidBlock < n3 && is_interior(g, c)) in |= 1u << q;
+    }
+    auto add = [&](int q, double num1, double den1) {
+        sums[0] += num1;
+        sums[1] += den1;
+        sums[2] += 1.0;
+        if (num1 > init) better(bv, bi, num1, (double)(c0 + (int64_t)q * kResidBlock));
+    };
+    if (KIND == RESID_PP) {
+#pragma unroll
+        for (int q = 0; q < kResidCells; ++q)
+            if (in >> q & 1u) add(q, fabs(bp[q]), 1.0);
+    }
+#pragma unroll 1
+    for (int q = 0; q < (KIND == RESID_PP ? 0 : kResidCells); q += kResidStep) {
+        if (!(in >> q & 3u)) continue;
         double ar[kResidStep][7], vn[kResidStep][6], bc[kResidStep], vc[kResidStep], ep[kResidStep];
-        int fn[kResidStep][6], fc[kResidStep];
-        bool in[kResidStep];
+        int fn[kResidStep][6];
 #pragma unroll
         for (int u = 0; u < kResidStep; ++u) {
-            const int64_t c1 = c0 + (int64_t)(q + u) * kResidBlock;   // increasing per thread
-            const int64_t c = c1 < n3 ? c1 : n3 - 1;
+            const int64_t c = cell(q + u);
             const Nb n = neighbours_fast(g, c);
-            in[u] = c1 < n3 && n.interior;
-            fc[u] = flag[c];
             bc[u] = ld_stream(&b[c]);
-            if (KIND != RESID_PP) {
-                vc[u] = var[c];
+            vc[u] = var[c];
 #pragma unroll
-                for (int p = 0; p < 7; ++p) ar[u][p] = ld_stream(&a[p * n3 + c]);
-                const int64_t nb[6] = {n.km, n.im, n.jm, n.ip, n.jp, n.kp};  // of the couplings 0, 2, 1, 4, 5, 6
+            for (int p = 0; p < 7; ++p) ar[u][p] = ld_stream(&a[p * n3 + c]);
+            const int64_t nb[6] = {n.km, n.im, n.jm, n.ip, n.jp, n.kp};  // of the couplings 0, 2, 1, 4, 5, 6
 #pragma unroll
-                for (int k = 0; k < 6; ++k) {
-                    vn[u][k] = var[nb[k]];
-                    if (KIND == RESID_C) fn[u][k] = flag[nb[k]];
-                }
-                if (KIND == RESID_S) ep[u] = R.ep_s ? eps[c] : 0.0;
+            for (int k = 0; k < 6; ++k) {
+                vn[u][k] = var[nb[k]];
+                if (KIND == RESID_C) fn[u][k] = flag[nb[k]];
             }
+            if (KIND == RESID_S) ep[u] = R.ep_s ? eps[c] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < kResidStep; ++u) {
-            double num1 = fabs(bc[u]), den1 = 1.0;
-            bool take = in[u] && fluid_at(fc[u]);  // IS_ON_myPE_wobnd, FLUID_AT
-            if (KIND != RESID_PP) {
-                double v[6];
+            double v[6];
 #pragma unroll
-                for (int k = 0; k < 6; ++k) v[k] = KIND == RESID_C && wall_at(fn[u][k]) ? vc[u] : vn[u][k];
-                // (the sums of resid_row_vals, in its order)
-                double r = bc[u] - (ar[u][3] * vc[u] + ar[u][4] * v[3] + ar[u][2] * v[1] + ar[u][5] * v[4] +
-                                    ar[u][1] * v[2]);
-                if (g.do_k) r = r - (ar[u][6] * v[5] + ar[u][0] * v[0]);
-                num1 = fabs(r);
-                den1 = fabs(ar[u][3] * vc[u]);
-                if (KIND == RESID_S) take = take && fabs(vc[u]) > R.tol && !(R.ep_s && ep[u] <= R.dil_ep_s);
-            }
-            if (take) {
-                sums[0] += num1;
-                sums[1] += den1;
-                sums[2] += 1.0;
-                if (num1 > init) better(bv, bi, num1, (double)(c0 + (int64_t)(q + u) * kResidBlock));
-            }
+            for (int k = 0; k < 6; ++k) v[k] = KIND == RESID_C && wall_at(fn[u][k]) ? vc[u] : vn[u][k];
+            // (the sums of resid_row_vals, in its order)
+            double r = bc[u] - (ar[u][3] * vc[u] + ar[u][4] * v[3] + ar[u][2] * v[1] + ar[u][5] * v[4] + ar[u][1] * v[2]);
+            if (g.do_k) r = r - (ar[u][6] * v[5] + ar[u][0] * v[0]);
+            bool take = in >> (q + u) & 1u;
+            if (KIND == RESID_S) take = take && fabs(vc[u]) > R.tol && !(R.ep_s && ep[u] <= R.dil_ep_s);
+            if (take) add(q + u, fabs(r), fabs(ar[u][3] * vc[u]));
         }
     }
     block_sum<kResidBlock, 3>(sums, lds);
@@ -237,7 +253,10 @@ static int run_resid(ResidArgs R, mfix_leq_resid *out, hipStream_t s) {
     R.partials = (double *)C.partials.ptr;
     static_assert(sizeof(mfix_leq_resid) <= sizeof(SolverState), "the first state mirror holds the result");
     R.out = (mfix_leq_resid *)C.host_state;
-    const dim3 grid((unsigned)xcd_grid(R.nblk)), block(kResidBlock);
+    const int64_t want = std::max<int64_t>(1, kResidPlanes * R.g.c2 / (kResidBlock * kResidCells));
+    const int64_t runs = std::max<int64_t>(4, (R.nblk + kNumXcd * want - 1) / (kNumXcd * want));  // of an XCD
+    R.run = (int)((R.nblk + kNumXcd * runs - 1) / (kNumXcd * runs));
+    const dim3 grid((unsigned)(runs * R.run * kNumXcd)), block(kResidBlock);
     if (R.kind == RESID_C) hipLaunchKernelGGL(k_resid<RESID_C>, grid, block, 0, s, R);
     else if (R.kind == RESID_S) hipLaunchKernelGGL(k_resid<RESID_S>, grid, block, 0, s, R);
     else hipLaunchKernelGGL(k_resid<RESID_PP>, grid, block, 0, s, R);
