@@ -184,7 +184,7 @@ struct SysDesc {
     double *x, *a, *b;            // VAR, A_M, B_M (FP64, device)
     const double *noise;
     uint64_t seed;
-    double line_lds = 0.0;        // LINE, FP64: LDS of a colour's lines of all systems of the launch (0: this one's)
+    double line_part = 0.0;       // LINE, FP64: part of the device a colour's lines of all systems of the launch take (0: this one's)
     int64_t line_past = 0;        // LINE, FP32: lines of a colour too long for the several-lane kernels, likewise
     Prologue pro;                 // residual / under-relaxation in the set-up pass
     mfix_leq_resid *resid_out = nullptr;  // host: the residual's result (pro.resid_kind >= 0)

@@ -6,7 +6,7 @@
 // rows in LDS: all threads load them (consecutive lanes take consecutive rows
 // of a line, every load of a thread issued before its first use) and form the
 // right-hand side, one lane per line runs the tridiagonal solve in LDS, and
-// all threads store the solution.  One memory round trip and four barriers a
+// all threads store the solution.  One memory round trip and six barriers a
 // block; blocks of a CU overlap each other's loads and chains.
 //
 // What bounds a phase is the serial chain of a line where few blocks share a
@@ -42,8 +42,9 @@ constexpr int kWholeThreads = 256;
 // Rows a thread loads at most (their diagonals stay in its registers through
 // the forward pass); longer lines take k_line_color_sys.
 constexpr int kWholeElems = 6, kWholeRows = kWholeThreads * kWholeElems;
-// LDS of one block's lines: four blocks fit on a CU.
-constexpr int kWholeLdsTarget = 160 * 1024 / 4 - 2048;
+// LDS of a block beside its lines (WholeLines, DGTSV's INFO, block sums), and what
+// is left for them where four blocks fit on a CU (as the launch bound allows).
+constexpr int kWholeFixed = 2048, kWholePerCu = 4, kWholeLdsTarget = 160 * 1024 / kWholePerCu - kWholeFixed;
 constexpr int kWholeLines = 64;  // one lane of the solving wave per line
 
 // k_line_stream: two blocks per CU, one wave of each solving, the other
@@ -76,24 +77,33 @@ __host__ __device__ constexpr int whole_elems(int n, int lpb) {
     return whole_few(lpb) ? stream_elems(n, lpb) : kWholeFront + 4 * lpb * whole_stride(n) + kWholeTail;
 }
 
-// Lines per block.  `table` is the LDS that all lines of one colour of every
-// system of the launch take together.  Where it fits the device in one round
-// (four blocks per CU), blocks are sized for two per CU: fewer would leave CUs
-// with one more block than others, more only share them (64^3 10.2 us a phase
-// with five lines a block, 13.2 with three).  Else the blocks' shares are even
-// over the fewest rounds that hold it: a round more costs a whole load, chain
-// and store (nine 64^3 systems 45 us a phase with five lines a block, four
-// rounds, 34 us with ten, two rounds).  pin: mfix_leq_set_line_block's value, 0
-// = none.
+// Lines whose LDS leaves room for four blocks on a CU (one line of more than
+// 1,200 rows leaves room for three).
+__host__ inline int whole_most(int n, size_t elem) {
+    int most = (kWholeLdsTarget / (int)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
+    while (most > 1 && whole_elems(n, most) * elem > kWholeLdsTarget) --most;
+    return most > 1 ? most : 1;
+}
+// Lines whose LDS the device holds at once.
+__host__ inline double whole_at_once(int n, size_t elem) {
+    return (double)kNumCus * kWholePerCu * whole_most(n, elem);
+}
+
+// Lines per block.  `table` is the part of the device that all lines of one
+// colour of every system of the launch take together.  Where they fit in one
+// round, blocks are sized for two per CU: fewer would leave CUs with one more
+// block than others, more only share them (64^3 10.2 us a phase with five lines a
+// block, 13.2 with three).  Else the blocks' shares are even over the fewest
+// rounds that hold them: a round more costs a whole load, chain and store (nine
+// 64^3 systems 45 us a phase with five lines a block, four rounds, 34 us with
+// ten, two rounds).  pin: mfix_leq_set_line_block's value, 0 = none.
 __host__ inline int whole_lpb(int n, double table, size_t elem, int pin) {
-    const double line = 4.0 * whole_stride(n) * (double)elem;
-    const double rounds = std::ceil(table / (4.0 * kNumCus * kWholeLdsTarget));
-    int64_t lpb = (int64_t)std::ceil(table / ((rounds > 1.0 ? 4.0 * rounds : 2.0) * kNumCus) / line);
-    const int64_t most = (kWholeLdsTarget / (int64_t)elem - kWholeFront - kWholeTail) / (4 * whole_stride(n));
-    const int64_t rows = kWholeRows / n;
-    if (lpb > most) lpb = most;
+    const double rounds = std::ceil(table), blocks = kNumCus * (rounds > 1.0 ? rounds * kWholePerCu : 2.0);
+    // (a share that is a whole number of lines stays it)
+    int64_t lpb = (int64_t)std::ceil(table * whole_at_once(n, elem) / blocks - 1e-6);
+    if (lpb > whole_most(n, elem)) lpb = whole_most(n, elem);
     if (pin > 0) lpb = pin;
-    if (lpb > rows) lpb = rows;
+    if (lpb > kWholeRows / n) lpb = kWholeRows / n;
     if (lpb > kWholeLines) lpb = kWholeLines;
     return lpb < 1 ? 1 : (int)lpb;
 }
@@ -120,10 +130,13 @@ __host__ inline bool long_lines(int n, int64_t lines) {
     const int64_t most = stream_most(n);
     return most <= 2 && stream_entries(n, lines) > (5 + most) * kStreamBlocks;
 }
-// Whether the lines of a system, `lines` of `lds` bytes a colour in all, stream:
-// they take more than one round of k_line_whole's blocks.
-__host__ inline bool line_streams(int n, int64_t lines, double lds, int64_t cells) {
-    return lds > 4.0 * kNumCus * kWholeLdsTarget && n <= kWholeRows && cells < (1ll << 29) &&
+// Whether the lines of a system stream: their LDS is more than one round of
+// k_line_whole's blocks.  Colour phase of whole lines and of streamed ones:
+// 7,320 lines of 146 rows (seven a block) 32.2 and 26.1 us; but 800 of 1,502 rows,
+// two rounds at three blocks a CU, 163 and 183, and 72,962 of 10 rows, which the
+// 64 lanes of a block hold before its LDS is full, 21 and 24.
+__host__ inline bool line_streams(int n, int64_t lines, int64_t cells) {
+    return n <= kWholeRows && (double)lines > whole_at_once(n, sizeof(double)) && cells < (1ll << 29) &&
            stream_entries(n, lines) <= (int64_t)kStreamBlocks * kStreamMost;
 }
 // Lines of entry j of a colour: [first(j), first(j + 1)), where first(j) = j

@@ -371,11 +371,11 @@ static void launch_line_factor(dim3 gs, int lds, hipStream_t s, const Sys<double
 // The one-lane-per-line kernel of a system, its lines per block and the blocks
 // a colour takes.
 static int64_t colour_lines(const LineGeom &L) { return ((int64_t)L.nu * L.nv + 1) / 2; }
-// LDS of a colour of the grid's lines (k_line_whole).
+// Part of the device that a colour of the grid's lines takes (k_line_whole).
 template <typename T>
-static double colour_lds(const DGrid &g) {
+static double colour_part(const DGrid &g) {
     const LineGeom L = line_geom(g, AX_J);
-    return whole_fits(L.n) ? (double)colour_lines(L) * 4.0 * whole_stride(L.n) * sizeof(T) : 0.0;
+    return whole_fits(L.n) ? (double)colour_lines(L) / whole_at_once(L.n, sizeof(T)) : 0.0;
 }
 // Whether lines of one colour are neighbours: across a cyclic axis with an odd
 // number of cells.  k_line_color_sys then, which reads all of a block's
@@ -396,30 +396,29 @@ static int64_t lines_past_pcr(const DGrid &g) {
     const LineGeom L = line_geom(g, AX_J);
     return line_pcr_variant(L.n) < 0 ? colour_lines(L) : 0;
 }
-// table: LDS of a colour of every system of the launch (0: this grid's alone);
+// table: colour_part of every system of the launch (0: this grid's alone);
 // past: FP32, lines_past_pcr of them all likewise
 template <typename T>
 static void set_line_kernel(Sys<T> &S, double table = 0.0, int64_t past = 0) {
     const DGrid &g = S.g;
     const LineGeom L = line_geom(g, AX_J);
     const int pin = ctx().shape_for(g.n3, sizeof(T) == sizeof(float)).lines_per_block;
-    const double own = colour_lds<T>(g);
     const int64_t lines = colour_lines(L);
     const bool rows_behind_tiles = sizeof(T) == sizeof(double) ? long_lines(L.n, lines) : !few_lines32(past > 0 ? past : lines);
     if (!whole_fits(L.n) || neighbours_alike(g) || rows_behind_tiles) {
         S.lk = LINE_LONG;
         S.lpb = kLongLpb;
-    } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, colour_lines(L), own, g.n3)) {
+    } else if (sizeof(T) == sizeof(double) && !pin && line_streams(L.n, lines, g.n3)) {
         S.lk = LINE_STREAM;
-        S.lent = stream_entries(L.n, colour_lines(L));
-        S.lstep = entry_step(colour_lines(L), S.lent);
+        S.lent = stream_entries(L.n, lines);
+        S.lstep = entry_step(lines, S.lent);
         S.lpb = (int)((S.lstep + 0xffffffffull) >> 32);
         return;
     } else {
         S.lk = LINE_WHOLE;
-        S.lpb = whole_lpb(L.n, table > 0.0 ? table : own, sizeof(T), pin);
+        S.lpb = whole_lpb(L.n, table > 0.0 ? table : colour_part<T>(g), sizeof(T), pin);
     }
-    S.lent = (colour_lines(L) + S.lpb - 1) / S.lpb;
+    S.lent = (lines + S.lpb - 1) / S.lpb;
     S.lstep = (uint64_t)S.lpb << 32;
 }
 template <typename T>
@@ -574,7 +573,7 @@ void sys_carve(Sys<T> &S, const SysDesc &d, const Part &P, char *base) {
         S.ld = S.line_scratch + n3;
         S.lu = S.line_scratch + 2 * n3;
         S.lu2 = S.line_scratch + 3 * n3;
-        set_line_kernel(S, d.line_lds, d.line_past);
+        set_line_kernel(S, d.line_part, d.line_past);
     }
     if (mixed) {
         S.a = (const T *)take(8 * n3 * sizeof(float));
@@ -1286,7 +1285,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<Part> parts((size_t)nsys);
     std::vector<size_t> offs((size_t)nsys);
     size_t total = 0;
-    double line_lds = 0.0;
+    double line_part = 0.0;
     int64_t line_past = 0;
     const int bs = 256;
     for (int q = 0; q < nsys; ++q) {
@@ -1311,7 +1310,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
         descs[q].seed = it.noise_seed;
         const Shape sh = C.shape_for(g.n3, it.mixed != 0);
         parts[q] = make_part(g.n3, bs, sh.bs == bs ? sh.cpt : 1);
-        if (pc == PC_LINE && !it.mixed) line_lds += colour_lds<double>(g);
+        if (pc == PC_LINE && !it.mixed) line_part += colour_part<double>(g);
         if (pc == PC_LINE && it.mixed) line_past += lines_past_pcr(g);
         offs[q] = total;
         total += sys_bytes(g, parts[q], pc, it.mixed != 0);
@@ -1329,7 +1328,7 @@ int solve_batch(int nsys, const mfix_leq_batch_item *items, mfix_leq_stats *stat
     std::vector<std::pair<int, int>> where((size_t)nsys);  // (precision, row)
     std::vector<int> ids64, ids32;
     for (int q = 0; q < nsys; ++q) {
-        descs[q].line_lds = items[q].mixed ? 0.0 : line_lds;
+        descs[q].line_part = items[q].mixed ? 0.0 : line_part;
         descs[q].line_past = line_past;
         char *base = (char *)C.bws.ptr + offs[q];
         if (items[q].mixed) {
