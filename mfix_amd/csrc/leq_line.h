@@ -872,7 +872,6 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
     if constexpr (sizeof(T) == sizeof(double)) {
         A.f = to_global((const T *)S.lf);
         A.d = to_global((const T *)S.ld);
-        const double mark = nl > 0 ? (double)A.f[w.c0[0]] : 0.0;
         constexpr int K = 3;  // rows in flight per thread
         T td[kWholeElems];    // the diagonals wait for the multipliers' place
         int o[kWholeElems], any = 0, out = 0;
@@ -912,16 +911,19 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             }
         }
         const bool swaps = __syncthreads_or(any);
-        if (!own_dgtsv(mark)) {
-            if (swaps) {
-                const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
-                for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
-                    const int l = line_of(x), q = x - l * n;
-                    const uint32_t c = w.c0[l] + (uint32_t)q;
-                    U[l * ls + q] = lu[c];
-                    D[l * ls + q] = lu2[c];
-                }
+        int own = 0;
+        if (swaps) {  // (or the block's mark is kOwnDgtsv, and the planes hold nothing)
+            const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
+            const double mark = (double)A.f[w.c0[0]];
+            for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
+                const int l = line_of(x), q = x - l * n;
+                const uint32_t c = w.c0[l] + (uint32_t)q;
+                U[l * ls + q] = lu[c];
+                D[l * ls + q] = lu2[c];
             }
+            own = __builtin_amdgcn_readfirstlane((int)own_dgtsv(mark));
+        }
+        if (!own) {
             // the solving wave: another one in each of the blocks that share a
             // CU (every 256th), so that they do not share a SIMD
             const int solver = (int)threadIdx.x - 64 * ((blockIdx.x >> 8) & 3);
