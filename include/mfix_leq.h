@@ -270,7 +270,8 @@ void mfix_leq_sweep_discard(void);  /* drop the queued calls unsolved */
 /* Autotuner: pick the block shape of the fused kernels (timed on a DIAG
  * solve) and the lines per block of the red-black line kernel (timed on a
  * LINE solve) for one grid size; results are cached per (n3 class,
- * precision).  Returns the chosen threads-per-block and lines-per-block. */
+ * precision).  Returns the chosen threads-per-block and lines-per-block, the
+ * latter as mfix_leq_set_line_block takes it (0: the kernel's own rule). */
 int mfix_leq_autotune(int imax, int jmax, int kmax, int mixed, int *block,
                       int *lines_per_block);
 /* Pin the launch shape the autotuner would record for this grid size and

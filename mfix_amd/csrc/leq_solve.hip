@@ -1585,15 +1585,7 @@ int autotune(int imax, int jmax, int kmax, int mixed, Shape *best_out) {
     slot = rc ? saved : best;
     for (double *q : {da, db, dx, dp, dm, dbp, dbm}) (void)hipFree(q);
     if (rc) return rc;
-    if (best_out) {
-        *best_out = best;
-        if (!best.lines_per_block) {
-            Sys<double> S = {};
-            S.g = g;
-            set_line_kernel(S);
-            best_out->lines_per_block = S.lpb;
-        }
-    }
+    if (best_out) *best_out = best;
     return 0;
 }
 
