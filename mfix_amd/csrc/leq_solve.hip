@@ -988,7 +988,8 @@ static int capture_chunk(Group<double> *G64, Group<float> *G32, int iters, hipSt
 // iterations are 5-9 short launches, hundreds a solve) with four.  Chunks of
 // a fixed 16 iterations, each polled with a copy, ran a 128^3 LINE momentum
 // solve of four iterations in 2,101 us; now 1,695.  No chunk runs past ITMAX.
-static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
+static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs,
+                        std::vector<hipGraphExec_t> &retired) {
     Context &C = ctx();
     int rc;
     // a poll's words: the next one, which may be under way, writes others, so
@@ -1021,7 +1022,7 @@ static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hi
         const uint64_t version = (G64 ? G64->iter.version * 1000003ull : 0) ^ (G32 ? G32->iter.version : 0) ^
                                  ((G64 ? 1ull : 0) << 62) ^ ((G32 ? 1ull : 0) << 63);
         if (!K.exec || K.iters != iters || K.version != version || K.sys != sys_key) {
-            if (K.exec) (void)hipGraphExecDestroy(K.exec);
+            if (K.exec) retired.push_back(K.exec);  // (its last launch may be under way)
             K.exec = nullptr;
             int e;
             if ((e = capture_chunk(G64, G32, iters, s, &K.exec))) return e;
@@ -1064,10 +1065,13 @@ static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hi
 }
 
 // With an error the chunk and the poll under way end first: they write the
-// caller's arrays and the polls' words.
+// caller's arrays and the polls' words.  So they do before a graph that was
+// replaced is destroyed.
 static int run_tables(Group<double> *G64, Group<float> *G32, int max_iters, hipStream_t s, bool graphs) {
-    const int rc = drive_tables(G64, G32, max_iters, s, graphs);
-    if (rc) (void)hipStreamSynchronize(s);
+    std::vector<hipGraphExec_t> retired;
+    const int rc = drive_tables(G64, G32, max_iters, s, graphs, retired);
+    if (rc || !retired.empty()) (void)hipStreamSynchronize(s);
+    for (hipGraphExec_t g : retired) (void)hipGraphExecDestroy(g);
     return rc;
 }
 

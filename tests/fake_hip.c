@@ -1,8 +1,8 @@
 /* A HIP runtime for host-side tests, preloaded over the real one: device memory
  * is host memory, kernels do nothing, and each launch, query and wait is written
  * to the file FAKE_HIP_LOG.  FAKE_HIP: "silent" (streams are idle at once),
- * "count" (k_count_running answers: every listed system runs for three polls,
- * then none does), "threads" (count, and launches from threads other than the
+ * "count" (k_count_running answers: FP64 systems run for three polls, FP32 ones
+ * for eight), "threads" (count, and launches from threads other than the
  * first one fail, with an error that only that thread's hipGetLastError shows). */
 #define _GNU_SOURCE
 #include <pthread.h>
@@ -68,7 +68,7 @@ int hipLaunchKernel(const void *fn, dim3 g, dim3 b, void **args, size_t m, void 
         const int nids = *(int *)args[2], poll = *(int *)args[4];
         note("poll %.0s%p %d %d", "", out, nids, poll);
         if (!mode("silent")) {
-            const int run = poll <= 3;
+            const int run = poll <= (strstr(name, "IfE") ? 8 : 3);
             out[0] = run ? nids : 0;
             for (int k = 0; k < nids; ++k) out[2 + k] = run;
             __atomic_store_n(out + 1, poll, __ATOMIC_RELEASE);
@@ -112,13 +112,13 @@ int hipEventCreateWithFlags(void **e, unsigned f) { return (void)f, *e = &nfns, 
 int hipEventDestroy(void *e) { return (void)e, 0; }
 int hipEventRecord(void *e, void *s) { return (void)e, (void)s, 0; }
 int hipEventQuery(void *e) { return (void)e, 0; }
-int hipEventSynchronize(void *e) { return (void)e, 0; }
+int hipEventSynchronize(void *e) { return (void)e, note("wait%.0s", "", 0, 0, 0), 0; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { return (void)a, (void)b, *ms = 0, 0; }
 int hipStreamBeginCapture(void *s, int m) { return (void)s, (void)m, 0; }
 int hipStreamEndCapture(void *s, void **g) { return (void)s, *g = &nfns, 0; }
 int hipGraphInstantiate(void **e, void *g, void *n, char *b, size_t z) {
-    return (void)g, (void)n, (void)b, (void)z, *e = &nfns, 0;
+    return (void)g, (void)n, (void)b, (void)z, hipMalloc(e, 1);
 }
 int hipGraphDestroy(void *g) { return (void)g, 0; }
-int hipGraphExecDestroy(void *g) { return (void)g, 0; }
-int hipGraphLaunch(void *g, void *s) { return (void)g, (void)s, note("launch graph%.0s", "", 0, 0, 0), 0; }
+int hipGraphExecDestroy(void *g) { return note("destroy%.0s %p", "", g, 0, 0), 0; }
+int hipGraphLaunch(void *g, void *s) { return (void)s, note("launch%.0s %p", "", g, 0, 0), 0; }

@@ -77,3 +77,26 @@ print(L.mfix_leq_bicgs(b"u", 1, 1, *(v.ctypes.data_as(_lib.c_double_p) for v in 
 """, tmp_path / "log")
     assert any("k_move" in s for s in log)      # the caller's own launches
     assert int(out) == -103                     # MFIX_LEQ_EHIP
+
+
+def test_graphs_are_destroyed_when_they_do_not_run(fake, tmp_path):
+    """The FP64 systems of a batch end before the FP32 ones: the chunk of both
+    that is under way by then is let run to its end before its graph goes."""
+    _, log = fake("count", """
+items = []
+for q in range(6):
+    n = 12 + 2 * q
+    dx, da, db = arrays((n + 2) ** 3)
+    items.append(leq.BatchSystem(n, n, n, dx, da, db, pc="DIAG", tol=1e-10, itmax=200, mixed=q % 2 == 1))
+leq.batch_solve(items)
+leq.finalize()
+""", tmp_path / "log")
+    launched, destroyed = {}, 0
+    for k, s in enumerate(log):
+        what, _, graph = s.partition(" ")
+        if what == "launch" and graph.startswith("0x"):
+            launched[graph] = k
+        elif what == "destroy" and graph in launched:
+            destroyed += 1
+            assert "wait" in log[launched[graph]:k], f"{graph} destroyed while it ran"
+    assert destroyed >= 2
