@@ -98,6 +98,7 @@ struct ChunkGraph {
     int iters = 0;
     uint64_t version = 0;
     const void *sys = nullptr;
+    bool launched = false;  // in the solve that runs
 };
 
 // A table of systems of one storage type and its device copy.

@@ -1007,6 +1007,8 @@ static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hi
         if (G64) enqueue_count<double>(*G64, G64->iter, words(0, poll), poll, s);
         if (G32) enqueue_count<float>(*G32, G32->iter, words(1, poll), poll, s);
     };
+    if (G64) for (ChunkGraph &K : G64->chunks) K.launched = false;  // (every solve before this one has ended)
+    if (G32) for (ChunkGraph &K : G32->chunks) K.launched = false;
     // `iters` iterations, by a replay of the captured chunk of that length
     // where there is one (kept in the float table's slots when present)
     auto issue = [&](int iters) -> int {
@@ -1022,7 +1024,8 @@ static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hi
         const uint64_t version = (G64 ? G64->iter.version * 1000003ull : 0) ^ (G32 ? G32->iter.version : 0) ^
                                  ((G64 ? 1ull : 0) << 62) ^ ((G32 ? 1ull : 0) << 63);
         if (!K.exec || K.iters != iters || K.version != version || K.sys != sys_key) {
-            if (K.exec) retired.push_back(K.exec);  // (its last launch may be under way)
+            if (K.exec && K.launched) retired.push_back(K.exec);  // (it may be under way)
+            else if (K.exec) (void)hipGraphExecDestroy(K.exec);
             K.exec = nullptr;
             int e;
             if ((e = capture_chunk(G64, G32, iters, s, &K.exec))) return e;
@@ -1030,6 +1033,7 @@ static int drive_tables(Group<double> *G64, Group<float> *G32, int max_iters, hi
             K.version = version;
             K.sys = sys_key;
         }
+        K.launched = true;
         const hipError_t e = hipGraphLaunch(K.exec, s);
         return e == hipSuccess ? 0 : hip_fail(e, "hipGraphLaunch");
     };
