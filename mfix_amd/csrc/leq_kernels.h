@@ -357,7 +357,10 @@ __host__ __device__ inline LineGeom line_geom(const DGrid &g, int axis) {
 }
 
 // Scratch elements a line launch needs: 4 arrays of (lanes x line length);
-// every launch here uses at most n3/n + 64 lanes of at most 64 threads.
+// every launch here uses at most n3/n + 64 lanes of at most 64 threads.  Factored
+// lines (k_line_factor) take n3 elements of each; the no-allocation entry keeps
+// their block maps in the 256 nmax behind: one 8-byte entry a 256-cell block and
+// one a few lines and pass, of at most 0.7 M cells.
 __host__ __device__ inline int64_t line_scratch_elems(const DGrid &g) {
     const int nmax = g.ni > g.nj ? (g.ni > g.nk ? g.ni : g.nk) : (g.nj > g.nk ? g.nj : g.nk);
     return 4 * (g.n3 + 64 * (int64_t)nmax);

@@ -489,7 +489,7 @@ __device__ __forceinline__ void whole_back_exact(double *__restrict__ pb, const 
 // lane 7 back) takes that group's values first and is then held by zero
 // couplings.  What does not depend on the neighbour, the marked multipliers and
 // the reciprocal, is formed for eight rows at once; in one lane a line it is
-// most of the instructions (256^3: 261 -> 226 us a phase; with more lines a
+// most of the instructions (256^3: 261 -> 228 us a phase; with more lines a
 // wave takes two turns: 11 lines a block, 150x201x180, 91 -> 121 us; without
 // interchanges there is little of it: 203 -> 205).
 __device__ __forceinline__ void whole_forward_swap8(const double *__restrict__ pf, double *__restrict__ pb, int rows,

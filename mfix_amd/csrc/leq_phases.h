@@ -784,9 +784,10 @@ __global__ void __launch_bounds__(kFinishBlock) k_finish_sys(const Sys<T> *__res
         fin_apply<F, NV>(st, tot, nullptr);
 }
 
-// Red-black line phase along J (RSRS and the 2-D R sweep) of systems whose
-// lines are too long for whole lines in LDS (more than 1,536 rows; the others
-// take k_line_whole).  Block b takes lines [map[b].y*LPB, +LPB) of colour
+// Red-black line phase along J (RSRS and the 2-D R sweep) of systems for which
+// whole lines in LDS are not the better way (set_line_kernel: lines of more than
+// 1,536 rows, many long ones, neighbours of one colour; the others take
+// k_line_whole or k_line_stream).  Block b takes lines [map[b].y*LPB, +LPB) of colour
 // `param` of system map[b].x, numbered densely by color_line, with five
 // waves: lane l of wave 0 runs DGTSV on line l (the operations and order of
 // solve_line, so the result is bit-identical); waves 1-4 feed it.  Lines along
@@ -802,10 +803,11 @@ __global__ void __launch_bounds__(kFinishBlock) k_finish_sys(const Sys<T> *__res
 // four elements each keep the kernel at two blocks per CU (a loader with eight
 // elements needs 256 registers, one block per CU).  which = 0 preconditions P
 // into Phat, 1 S into Shat.
-template <typename T, int LPB>
+constexpr int kLongLpb = 64;  // lines per block
+template <typename T>
 __global__ void __launch_bounds__(320) k_line_color_sys(const Sys<T> *__restrict__ sys, const int2 *__restrict__ map,
                                                         int param, int which) {
-    static_assert(LPB == 64, "lines per block");
+    constexpr int LPB = kLongLpb;
     constexpr int RL = 1024 / LPB; // rows per run a loader instruction reads of each line
     constexpr int LPI = 64 / RL;   // lines per load instruction
     constexpr int K = 4;           // tile elements per loader lane
@@ -1083,10 +1085,9 @@ __global__ void __launch_bounds__(320) k_line_color_sys(const Sys<T> *__restrict
 
 constexpr int kLineBlock = 320;  // threads of k_line_color_sys: one solving wave, four loaders
 
-constexpr int kLongLpb = 64;     // its lines per block
-
 // Red-black line kernels with one lane per line: k_line_whole (whole lines in
-// LDS) and, for lines that do not fit there, k_line_color_sys.
+// LDS), k_line_color_sys (rows behind tiles) and k_line_stream (whole lines of a
+// system of more than one round of blocks).
 enum LineKernel : int { LINE_WHOLE = 0, LINE_LONG = 1, LINE_STREAM = 2 };
 constexpr int kLineKernels = 3;
 

@@ -361,7 +361,7 @@ static void launch_line_color(int kernel, dim3 gs, int lds, hipStream_t s, const
     if (kernel == LINE_WHOLE)
         launch_timed_lds(ev.first, ev.second, k_line_whole<T>, gs, dim3(kWholeThreads), lds, s, tab, mp, param, which);
     else
-        launch_timed(ev.first, ev.second, k_line_color_sys<T, kLongLpb>, gs, dim3(kLineBlock), s, tab, mp, param,
+        launch_timed(ev.first, ev.second, k_line_color_sys<T>, gs, dim3(kLineBlock), s, tab, mp, param,
                      which);
 }
 static void launch_line_factor(dim3 gs, int lds, hipStream_t s, const Sys<double> *tab, const int2 *mp) {
