@@ -181,7 +181,7 @@ __device__ __forceinline__ double corrected_quotient(double n, double d, double 
 struct WholeLines {
     uint32_t c0[kWholeLines], im[kWholeLines], ip[kWholeLines], km[kWholeLines], kp[kWholeLines];
     int n;
-    int odd;  // (k_line_whole: a right-hand side is out of range)
+    int odd, own;  // (k_line_whole: a right-hand side is out of range; the block's mark is kOwnDgtsv)
 };
 __device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j, int param, WholeLines &w) {
     const int l = threadIdx.x;
@@ -201,7 +201,7 @@ __device__ __forceinline__ void whole_lines(const DGrid &g, uint64_t step, int j
         const uint64_t have = __ballot(ok);
         if (l == 0) {
             w.n = __popcll(have);
-            w.odd = 0;
+            w.odd = w.own = 0;
         }
     }
     __syncthreads();
@@ -874,7 +874,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
         A.d = to_global((const T *)S.ld);
         constexpr int K = 3;  // rows in flight per thread
         T td[kWholeElems];    // the diagonals wait for the multipliers' place
-        int o[kWholeElems], any = 0, out = 0;
+        int o[kWholeElems], any = 0, out = 0, own = 0;
 #pragma unroll
         for (int k0 = 0; k0 < kWholeElems; k0 += K) {
             if (k0 * kWholeThreads >= tot) break;
@@ -894,6 +894,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             for (int k = 0; k < K; ++k) {
                 F[o[k0 + k]] = first[k] ? (T)0 : r[k].f;
                 any |= swapped(r[k].f);
+                own |= own_dgtsv(r[k].f);
                 const T b = r[k].rhs(do_k);
                 out |= !solution_in_range((double)b);
                 B[o[k0 + k]] = b;
@@ -903,6 +904,7 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             }
         }
         if (out) w.odd = 1;
+        if (own) w.own = 1;
         for (int x = threadIdx.x; x < 8 * nl; x += kWholeThreads) {
             const int q = n + (x & 7), at = (x >> 3) * ls + q;
             if (q < held) {  // identity rows
@@ -911,19 +913,16 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
             }
         }
         const bool swaps = __syncthreads_or(any);
-        int own = 0;
         if (swaps) {  // (or the block's mark is kOwnDgtsv, and the planes hold nothing)
             const gptr<const double> lu = to_global((const double *)S.lu), lu2 = to_global((const double *)S.lu2);
-            const double mark = (double)A.f[w.c0[0]];
             for (int x = threadIdx.x; x < tot; x += kWholeThreads) {
                 const int l = line_of(x), q = x - l * n;
                 const uint32_t c = w.c0[l] + (uint32_t)q;
                 U[l * ls + q] = lu[c];
                 D[l * ls + q] = lu2[c];
             }
-            own = __builtin_amdgcn_readfirstlane((int)own_dgtsv(mark));
         }
-        if (!own) {
+        if (!swaps || !w.own) {
             // the solving wave: another one in each of the blocks that share a
             // CU (every 256th), so that they do not share a SIMD
             const int solver = (int)threadIdx.x - 64 * ((blockIdx.x >> 8) & 3);
