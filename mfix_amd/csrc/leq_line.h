@@ -29,7 +29,7 @@
 //
 // Measured (events of the dispatches, LINE solve, colour phase; before, one
 // DGTSV lane per line over 16-row tiles with the finished rows in global
-// scratch): 64^3 28.4 -> 10.2 us, 128^3 56.2 -> 29.0 us, 158^3 70.9 -> 50.5
+// scratch): 64^3 28.4 -> 10.3 us, 128^3 56.2 -> 29.4 us, 158^3 70.9 -> 50.5
 // us, 256^3 409 -> 234 us.
 #pragma once
 #include <cmath>
@@ -990,8 +990,8 @@ __global__ void __launch_bounds__(kWholeThreads, 4) k_line_whole(const Sys<T> *_
 // a block's loads, chain and store came one after the other.  With two solving
 // waves of eight lines the chains fit beside the loads, and a phase moves what
 // it moves (a fifth more than the arrays: the other colour's values twice) at
-// 4.2 of the 5.1 TB/s of a copy: 256^3 233 -> 201 us, 170^3 71 -> 59 us,
-// 150x201x180 76 -> 69 us.  Non-temporal loads of the arrays read once: 195 us
+// 4.2 of the 5.1 TB/s of a copy: 256^3 233 -> 196 us, 170^3 71 -> 59 us,
+// 150x201x180 76 -> 68 us.  Non-temporal loads of the arrays read once: 195 us
 // at 256^3, but 48 for 42 us at 200x100x200, whose arrays the last-level cache
 // holds.  An entry with a pivot or a value of its solution out of range
 // is left for the end; with a right-hand side out of range it divides at once.

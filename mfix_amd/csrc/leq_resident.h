@@ -23,11 +23,13 @@
 // arithmetic gives, until it is stored.  Slots are used in three sets in turn;
 // their owner clears those of the next reduction when a phase begins, by which
 // time they have been read (their readers have taken part in the reduction in
-// between), and the clears are complete before it takes part in this one.  (All blocks reading all partial sums instead took
-// 6.5 us a reduction with 154 blocks against 4.1.)
-// Measured, an iteration with launches -> here: 8^3 17.1 -> 7.0 us, 16^3 28.4
-// -> 11.6, 32^3 28.7 -> 12.3, 40^3 29.9 -> 14.1, 48^3 30.3 -> 15.4 (488 blocks).
-// What is left is three round trips of about 4 us.
+// between), and the clears are complete before it takes part in this one.  (All
+// blocks reading all partial sums instead took 6.5 us a reduction with 154 blocks
+// against 4.1.)
+// Measured, an iteration with launches -> here: 16^3 27.8 -> 9.6 us, 32^3 25.5
+// -> 10.1, 40^3 27.1 -> 11.9, 48^3 27.9 -> 13.1 (488 blocks); with R exchanged
+// through its own array, which the set-up's kernels leave in the L2s, 11.6, 12.1,
+// 14.1 and 15.2.  What is left is three round trips of about 3 us.
 //
 // The arithmetic and the order of every sum are those of the launched kernels
 // (leq_phases.h) and of the one-block finish (finish_sum, fin_apply), so the

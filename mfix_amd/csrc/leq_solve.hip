@@ -1128,7 +1128,7 @@ static Sweep make_sweep(const char *cmethod) {
 // Whether a system can run as one resident launch (k_resident): FP64, DIAG or
 // NONE, 256-cell blocks, at most as many as the device holds at once (two per
 // CU, 131,072 cells).  Up to there an iteration takes half the launches' time
-// (48^3, 488 blocks: 15.4 against 30.3 us); with four blocks of 128 VGPRs per
+// (48^3, 488 blocks: 13.1 against 27.9 us); with four blocks of 128 VGPRs per
 // CU, part of the neighbours' values in scratch, the advantage is gone (50^3
 // 28.4 against 28.9 us, 62^3 35.9 against 34).
 static bool resident_fits(const Sys<double> &S, int bs) {
